@@ -1556,8 +1556,7 @@ int hkv_find_or_insert(hkv_table* t, uint64_t n, const uint64_t* keys,
   if (dg.on) {
     /* the other occurrences of a key get the row its representative ended up with (what it
      * read, or what it inserted; a refused key keeps its own row, like its representative) */
-    hipLaunchKernelGGL(dedup_fix_rows_kernel, dim3((unsigned)n), dim3(64), 0, (hipStream_t)stream,
-                       (const uint32_t*)dg.d.rep, n, (uint8_t*)values, t->view.value_bytes);
+    dedup_fix_rows(dg.d.rep, n, (uint8_t*)values, t->view.value_bytes, (hipStream_t)stream);
     HKV_HIP(hipGetLastError());
   }
   return HKV_SUCCESS;

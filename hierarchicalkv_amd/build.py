@@ -6,6 +6,8 @@ test checker under oracle/ and is built with gcc.  Nothing here runs a GPU.
 import os
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG_DIR)
@@ -21,27 +23,38 @@ HIP_FLAGS = [
     "-O3",
     "-std=c++17",
     "-fPIC",
-    "-shared",
     "-Wall",
     "-Wno-unused-function",
     # packed fp32 VALU forms are kept out of every kernel in this build
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
+# translation units of libhkv.so: (source, its own flags); the upsert family is compiled once per
+# operation, so that its many kernel instances build side by side
+UNITS = ([("hkv_launch_upsert.hip", [f"-DHKV_UPSERT_OP={op}"]) for op in range(5)] +
+         [("hkv_table.hip", []), ("hkv_launch_lookup.hip", []), ("hkv_launch_assign.hip", [])])
 
 
-def build_library(verbose=True):
-    cmd = [HIPCC, *HIP_FLAGS, "-I", INCLUDE, "-I", CSRC,
-           os.path.join(CSRC, "hkv_table.hip"), "-o", LIB_PATH]
+def _run(cmd, verbose):
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)
+
+
+def build_library(verbose=True):
+    with tempfile.TemporaryDirectory() as tmp:
+        objects = [os.path.join(tmp, f"{i}.o") for i in range(len(UNITS))]
+        compiles = [[HIPCC, *HIP_FLAGS, *flags, "-I", INCLUDE, "-I", CSRC, "-c", os.path.join(CSRC, src), "-o", obj]
+                    for (src, flags), obj in zip(UNITS, objects)]
+        with ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 1)) as pool:
+            list(pool.map(lambda cmd: _run(cmd, verbose), compiles))
+        _run([HIPCC, "--offload-arch=gfx950", "-shared", *objects, "-o", LIB_PATH], verbose)
     return LIB_PATH
 
 
 def build_ceilings(verbose=True):
     """The access-pattern ceilings of bench.py --ceilings: a measurement tool in a library of its own."""
     out = os.path.join(PKG_DIR, "libhkv_ceilings.so")
-    cmd = [HIPCC, *HIP_FLAGS, os.path.join(CSRC, "hkv_ceilings.hip"), "-o", out]
+    cmd = [HIPCC, *HIP_FLAGS, "-shared", os.path.join(CSRC, "hkv_ceilings.hip"), "-o", out]
     if verbose:
         print(" ".join(cmd), flush=True)
     subprocess.check_call(cmd)

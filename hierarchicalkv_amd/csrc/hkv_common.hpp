@@ -286,28 +286,105 @@ __device__ __forceinline__ uint64_t now_ns(const Clock& c, uint64_t i) {
 
 /* ---- row copies by an 8-lane tile ------------------------------------------ */
 
-template <int VEC>
-struct VecType;
+/* How wide the units are that rows are moved in.  16, 8, 4, 2, 1: so many bytes, rows and pointers
+ * a multiple of it.  kAny + one of these: rows of at least so many bytes at any address, of any size;
+ * the last unit of a row ends with the row and may overlap the one before it (both carry the same
+ * bytes).  The memory system takes unaligned accesses; what they cost is the extra line that a row
+ * which straddles a line touches anyway. */
+constexpr int kAny = 32;
+constexpr int vec_bytes(int vec) { return vec & 31; }
+
+template <int BYTES>
+struct UnitType;
 template <>
-struct VecType<16> {
+struct UnitType<16> {
   using type = uint4;
 };
 template <>
-struct VecType<8> {
+struct UnitType<8> {
   using type = uint2;
 };
 template <>
-struct VecType<4> {
+struct UnitType<4> {
   using type = uint32_t;
 };
 template <>
-struct VecType<2> {
+struct UnitType<2> {
   using type = uint16_t;
 };
 template <>
-struct VecType<1> {
+struct UnitType<1> {
   using type = uint8_t;
 };
+template <int VEC>
+struct VecType {
+  using type = typename UnitType<vec_bytes(VEC)>::type;
+};
+
+/* units of a row of `bytes` bytes, and where in the row unit u is */
+template <int VEC>
+__device__ __forceinline__ uint32_t row_units(uint32_t bytes) {
+  constexpr uint32_t w = vec_bytes(VEC);
+  return VEC >= kAny ? (bytes + w - 1) / w : bytes / w;
+}
+template <int VEC>
+__device__ __forceinline__ uint32_t unit_offset(uint32_t u, uint32_t bytes) {
+  constexpr uint32_t w = vec_bytes(VEC);
+  if constexpr (VEC >= kAny) return u * w < bytes - w ? u * w : bytes - w;
+  return u * w;
+}
+
+/* One unit of a row that no other wavefront is changing, read once: streaming where it is wide. */
+typedef u32x4_t u32x4_any_t __attribute__((aligned(1)));
+typedef uint32_t u32x2_any_t __attribute__((ext_vector_type(2), aligned(1)));
+typedef uint32_t u32_any_t __attribute__((aligned(1)));
+typedef uint16_t u16_any_t __attribute__((aligned(1)));
+template <int VEC>
+__device__ __forceinline__ typename VecType<VEC>::type load_row_unit(const uint8_t* p) {
+  if constexpr (VEC == 16) {
+    const u32x4_t t = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(p));
+    return make_uint4(t.x, t.y, t.z, t.w);
+  } else if constexpr (VEC == kAny + 16) {
+    const u32x4_t t = __builtin_nontemporal_load(reinterpret_cast<const u32x4_any_t*>(p));
+    return make_uint4(t.x, t.y, t.z, t.w);
+  } else if constexpr (VEC == kAny + 8) {
+    const u32x2_any_t t = *reinterpret_cast<const u32x2_any_t*>(p);
+    return make_uint2(t.x, t.y);
+  } else if constexpr (VEC == kAny + 4) {
+    return *reinterpret_cast<const u32_any_t*>(p);
+  } else if constexpr (VEC == kAny + 2) {
+    return *reinterpret_cast<const u16_any_t*>(p);
+  } else {
+    return *reinterpret_cast<const typename VecType<VEC>::type*>(p);
+  }
+}
+/* The same unit to byte `offset` of a buffer resource; an offset past its end stores nothing. */
+template <int VEC>
+__device__ __forceinline__ void store_row_unit(__amdgpu_buffer_rsrc_t dst, uint32_t offset,
+                                               typename VecType<VEC>::type x) {
+  if constexpr (vec_bytes(VEC) == 16) {
+    const u32x4_t t = {x.x, x.y, x.z, x.w};
+    __builtin_amdgcn_raw_buffer_store_b128(t, dst, offset, 0, 2 /* nt */);
+  } else if constexpr (vec_bytes(VEC) == 8) {
+    typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+    const u32x2_t t = {x.x, x.y};
+    __builtin_amdgcn_raw_buffer_store_b64(t, dst, offset, 0, 0);
+  } else if constexpr (vec_bytes(VEC) == 4) {
+    __builtin_amdgcn_raw_buffer_store_b32(x, dst, offset, 0, 0);
+  } else if constexpr (vec_bytes(VEC) == 2) {
+    __builtin_amdgcn_raw_buffer_store_b16(x, dst, offset, 0, 0);
+  } else {
+    __builtin_amdgcn_raw_buffer_store_b8(x, dst, offset, 0, 0);
+  }
+}
+
+/* What this wavefront has written to LDS is visible to all its lanes, and the compiler moves no
+ * LDS access across.  Staging areas belong to one wavefront each, so nobody waits for anybody. */
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 /* Row copy by the 8 lanes of a tile, VEC bytes per lane and trip (16, 4 or 1).
  * DST_TABLE / SRC_TABLE say which side is a value row of the table and must be

@@ -1,0 +1,59 @@
+/*
+ * Kernel instances of the lookups.
+ */
+#include "hkv_launch.hpp"
+
+namespace hkv {
+namespace {
+
+template <int MODE, int R, bool DUAL = false, int WAVES = 1, bool MISSED = false>
+void launch_lookup_by(int vec, const View& v, const FindArgs& a, hipStream_t s) {
+  constexpr uint64_t kKeys = (uint64_t)kTilesPerWave * R * WAVES;
+  const dim3 grid((unsigned)((a.n + kKeys - 1) / kKeys)), block(kWave * WAVES);
+  if constexpr (MODE == kLookupValues) {
+    switch (vec) {
+      case kAny + 16: launch_main(lookup_kernel<MODE, kAny + 16, DUAL, WAVES, R, MISSED>, grid, block, s, v, a); return;
+      case kAny + 8: launch_main(lookup_kernel<MODE, kAny + 8, DUAL, WAVES, R, MISSED>, grid, block, s, v, a); return;
+      case kAny + 4: launch_main(lookup_kernel<MODE, kAny + 4, DUAL, WAVES, R, MISSED>, grid, block, s, v, a); return;
+      case kAny + 2: launch_main(lookup_kernel<MODE, kAny + 2, DUAL, WAVES, R, MISSED>, grid, block, s, v, a); return;
+      case 1: launch_main(lookup_kernel<MODE, 1, DUAL, WAVES, R, MISSED>, grid, block, s, v, a); return;
+    }
+  }
+  launch_main(lookup_kernel<MODE, 16, DUAL, WAVES, R, MISSED>, grid, block, s, v, a);
+}
+
+/* Keys per tile.  A wavefront of 64 keys (R = 8) holds 114 registers, four of them fit on a SIMD, and
+ * a tile does much of its work on its 8 keys one after the other; with 2 keys per tile it is 48
+ * registers, eight wavefronts, and a quarter of the chain.  us per call (hits 7/8, cold):
+ *   keys     row        R = 8    2      1
+ *   2^20    256 bytes    119    112    115
+ *   2^20     32           73     68     84
+ *   2^18    512           55     51     49.5
+ *   2^15    256           12.2    7.8    7.8
+ *   3001     64           10.1    5.3    4.6
+ *   500     256            9.6    4.6    3.8
+ *   2^20   no rows (contains)  51  46.5  58
+ * One key per tile where that leaves the chip room (a quarter of its 8192 wave slots at 2^14 keys)
+ * or where the rows outweigh the probes. */
+template <int MODE>
+void launch_lookup(int vec, const View& v, const FindArgs& a, hipStream_t s) {
+  if (a.n <= (UINT64_C(1) << 14) || (MODE == kLookupValues && v.value_bytes >= 512))
+    launch_lookup_by<MODE, 1>(vec, v, a, s);
+  else
+    launch_lookup_by<MODE, 2>(vec, v, a, s);
+}
+
+}  // namespace
+
+void launch_find(int vec, const View& v, const FindArgs& a, hipStream_t s) { launch_lookup<kLookupValues>(vec, v, a, s); }
+void launch_find_ptr(const View& v, const FindArgs& a, hipStream_t s) { launch_lookup<kLookupPtr>(16, v, a, s); }
+void launch_contains(const View& v, const FindArgs& a, hipStream_t s) { launch_lookup<kLookupContains>(16, v, a, s); }
+void launch_find_dual(int vec, const View& v, const FindArgs& a, hipStream_t s) {
+  launch_lookup_by<kLookupValues, 2, true>(vec, v, a, s);
+}
+/* 16 wavefronts per workgroup (see lookup_kernel) */
+void launch_find_missed(int vec, const View& v, const FindArgs& a, hipStream_t s) {
+  launch_lookup_by<kLookupValues, kTile, false, 16, true>(vec, v, a, s);
+}
+
+}  // namespace hkv

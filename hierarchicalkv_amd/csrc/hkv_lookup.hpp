@@ -1,7 +1,7 @@
 /*
  * Read-only lookups: find (value copy), find* (row pointer), contains, and
- * the missed-keys variant of find.  One 64-lane wavefront per workgroup,
- * 64 keys per wavefront.
+ * the missed-keys variant of find.  One 64-lane wavefront per workgroup, R keys
+ * per 8-lane tile (8R per wavefront).
  *
  * Replaces lookup_kernel_with_io_pipeline_v1 (lookup.cuh:119-378),
  * lookup_ptr_kernel_with_pipeline / tlp_lookup_ptr_kernel_with_filter
@@ -10,16 +10,18 @@
  * the reference (group_lock.cuh:43-56).
  *
  * Phases of a wavefront
- *   own    lane L loads key L, hashes it and stages (key, bucket, digest) in LDS;
- *   probe  tile t (8 lanes) probes key 8t+r in round r = 0..7: lane j loads
+ *   own    lane 8t + r (r < R) loads its key, hashes it and stages (key, bucket, digest) in LDS;
+ *   probe  tile t (8 lanes) probes the key of lane 8t + r in round r < R: lane j loads
  *          16 of the 128 digest bytes, so a tile reads one whole 128-byte line
- *          per round; the 8 rounds are issued back to back so 8 KB of digests
- *          are in flight per wavefront;
+ *          per round; the rounds are issued back to back, R KB of digests in flight per wavefront;
  *   verify every digest match is checked against the 8-byte key, the first
  *          lane's candidates first and the others only if those were not it;
  *          the hit slot goes to LDS;
- *   copy   the whole wavefront copies the found rows, VEC bytes per lane,
+ *   copy   the whole wavefront copies the found rows, one unit per lane and step,
  *          so the output side is written in fully coalesced 1 KB pieces.
+ * Bound by random 128-byte lines (a digest line, about 1.2 key lines and the row per key): 842 MB
+ * move in 112 us for 2^20 keys with rows of 256 bytes, capacity 2^26.  How many keys a tile takes is
+ * what matters most beside that (launch_lookup in hkv_launch_lookup.hip).
  */
 #ifndef HKV_LOOKUP_HPP_
 #define HKV_LOOKUP_HPP_
@@ -43,7 +45,28 @@ struct FindArgs {
 };
 
 /*
- * Probe the 64 keys staged in s_meta.  On return (after the caller's barrier)
+ * Keys per wavefront.  Tile t owns the keys of its lanes 0 .. R-1, R = 8 being the full 64 keys of
+ * a wavefront: the key of lane 8t + r is number t * R + r of the wavefront, and lanes 8t + R and
+ * above own none.  What is staged in LDS is indexed by lane.  A smaller R spreads a batch over
+ * more wavefronts: a tile handles its R keys one after the other where it cannot overlap them.
+ */
+template <int R>
+__device__ __forceinline__ uint64_t key_of_lane(uint64_t wave, int lane) {
+  if constexpr (R == kTile) return wave * kWave + lane;
+  return wave * (kTilesPerWave * R) + (uint32_t)(lane >> 3) * R + (lane & (kTile - 1));
+}
+template <int R>
+__device__ __forceinline__ bool lane_owns_key(int lane) {
+  return R == kTile || (lane & (kTile - 1)) < R;
+}
+/* the lane that owns key kk of a wavefront */
+template <int R>
+__device__ __forceinline__ uint32_t lane_of_key(uint32_t kk) {
+  return R == kTile ? kk : kk / R * kTile + kk % R;
+}
+
+/*
+ * Probe the keys staged in s_meta.  On return (after the caller's barrier)
  * s_slot[k] is the table slot of key k or -1.  WRITER selects the writers'
  * probe, which runs while other wavefronts change the table:
  *   - s_em[k][j] (when given) receives lane j's 16-bit mask of EMPTY digests of
@@ -53,17 +76,17 @@ struct FindArgs {
  *     another tile's lock, so s_unsure[k] is raised and the writer settles the
  *     question with a second, coherent probe of its own (tile_reprobe).
  */
-template <bool WRITER, bool TWO_STEP>
+template <bool WRITER, bool TWO_STEP, int R = kTile>
 __device__ __forceinline__ void probe_wave(const View& v, const KeyMeta* s_meta,
                                            int64_t* s_slot,
                                            uint16_t (*s_em)[kTile],
                                            uint8_t* s_unsure, int lane) {
   const int tile = lane >> 3, j = lane & 7;
-  uint4 dg[kTile];
-  uint32_t bkt[kTile];
-  uint32_t inf[kTile];
+  uint4 dg[R];
+  uint32_t bkt[R];
+  uint32_t inf[R];
 #pragma unroll
-  for (int r = 0; r < kTile; r++) {
+  for (int r = 0; r < R; r++) {
     const KeyMeta m = s_meta[tile * kTile + r];
     bkt[r] = m.bkt;
     inf[r] = m.info;
@@ -80,11 +103,11 @@ __device__ __forceinline__ void probe_wave(const View& v, const KeyMeta* s_meta,
    * (keys that went into a free slot / into a victim's slot) instead of 1.44.  The lookups
    * and the kernels that move rows use it; erase and lock_keys, which move little besides
    * the probe and are bound by their dependent round trips, take all candidates at once. */
-  uint32_t cm[kTile];    /* this lane's digest matches, bw order */
-  uint32_t later[kTile]; /* lanes of the tile whose candidates wait for step 2 */
-  uint64_t k0[kTile], k1[kTile];
+  uint32_t cm[R];       /* this lane's digest matches, bw order */
+  uint32_t later[R];     /* lanes of the tile whose candidates wait for step 2 */
+  uint64_t k0[R], k1[R];
 #pragma unroll
-  for (int r = 0; r < kTile; r++) {
+  for (int r = 0; r < R; r++) {
     const bool valid = inf[r] & 0x100u;
     const uint32_t d = inf[r] & 0xFFu;
     cm[r] = valid ? match16(dg[r], d * 0x01010101u) : 0u;
@@ -137,7 +160,7 @@ __device__ __forceinline__ void probe_wave(const View& v, const KeyMeta* s_meta,
   };
   bool more = false;
 #pragma unroll
-  for (int r = 0; r < kTile; r++) {
+  for (int r = 0; r < R; r++) {
     const bool mine = cm[r] && !((later[r] >> j) & 1u);
     const bool hit = mine && check(r);
     if (TWO_STEP) {
@@ -147,7 +170,7 @@ __device__ __forceinline__ void probe_wave(const View& v, const KeyMeta* s_meta,
   }
   if (TWO_STEP && __ballot(more)) {
 #pragma unroll
-    for (int r = 0; r < kTile; r++) {
+    for (int r = 0; r < R; r++) {
       if ((later[r] >> j) & 1u) {
         const uint64_t* kb = v.keys + (uint64_t)bkt[r] * kBucketSize + j * 16;
         k0[r] = kb[bw_to_pos(__ffs(cm[r]) - 1)];
@@ -156,7 +179,7 @@ __device__ __forceinline__ void probe_wave(const View& v, const KeyMeta* s_meta,
       }
     }
 #pragma unroll
-    for (int r = 0; r < kTile; r++)
+    for (int r = 0; r < R; r++)
       if ((later[r] >> j) & 1u) check(r);
   }
 }
@@ -211,7 +234,7 @@ __device__ __forceinline__ int64_t tile_reprobe(const View& v, uint64_t key,
   return locks ? -2 : -1;
 }
 
-/* Lane-owned part shared by all wave-per-64-keys kernels: load, hash, stage. */
+/* Lane-owned part shared by all probing kernels: load, hash, stage.  Lanes without a key pass i >= n. */
 __device__ __forceinline__ uint64_t stage_keys(const View& v,
                                                const uint64_t* keys, uint64_t n,
                                                uint64_t i, KeyMeta* s_meta,
@@ -260,12 +283,56 @@ __device__ __forceinline__ void restage_second_bucket(const View& v, KeyMeta* s_
 
 enum LookupMode { kLookupValues = 0, kLookupPtr = 1, kLookupContains = 2 };
 
-/* WAVES wavefronts per workgroup, each with its own 64 keys and its own staging area.  One
+/* rows s_slot[lane_of_key(kk)] of the table -> rows base + kk of `out`, for the keys that were found.
+ * PLAIN: all rows are in HBM and slot numbers fit 32 bits (an address is one multiply-add). */
+template <int VEC, int R, bool PLAIN>
+__device__ __forceinline__ void copy_found_rows(const View& v, const int64_t* s_slot, uint8_t* out,
+                                                uint64_t base, uint64_t n, int lane) {
+  using T = typename VecType<VEC>::type;
+  constexpr uint32_t kKeys = kTilesPerWave * R;
+  constexpr uint32_t kPast = 0x80000000u; /* an offset that is past the end of any wavefront's rows */
+  const uint32_t units = row_units<VEC>(v.value_bytes);
+  const uint32_t total = units * kKeys;
+  /* Units a lane has in flight: all of a wavefront's for rows of up to 256 bytes (twice as many
+   * cost registers: rows of 32 bytes 72 instead of 68 us per 2^20 keys).  A row of less than 16
+   * bytes is one or two units. */
+  constexpr int kB = vec_bytes(VEC) == 16 ? 2 * R : (R + 3) / 4;
+  const uint64_t rows_here = n - base < kKeys ? n - base : kKeys;
+  const __amdgpu_buffer_rsrc_t dst = __builtin_amdgcn_make_buffer_rsrc(
+      out + base * v.value_bytes, 0, (uint32_t)(rows_here * v.value_bytes), 0x00020000);
+  /* (key, unit) of this lane's next step; a step moves 64 units on */
+  uint32_t kk = (uint32_t)lane / units, c = (uint32_t)lane % units;
+  const uint32_t kk_step = kWave / units, c_step = kWave % units;
+  for (uint32_t idx0 = lane; idx0 < total; idx0 += kWave * kB) {
+    T buf[kB];
+    uint32_t at[kB];
+#pragma unroll
+    for (int b = 0; b < kB; b++) {
+      const bool inside = kk < kKeys;
+      const int64_t slot = s_slot[lane_of_key<R>(inside ? kk : 0)];
+      const bool found = inside && slot >= 0;
+      const uint64_t from = found ? (uint64_t)slot : 0;
+      const uint32_t off = unit_offset<VEC>(c, v.value_bytes);
+      at[b] = found ? kk * v.value_bytes + off : kPast;
+      buf[b] = load_row_unit<VEC>((PLAIN ? v.values + (uint64_t)(uint32_t)from * v.value_bytes : value_row(v, from)) + off);
+      kk += kk_step;
+      c += c_step;
+      if (c >= units) {
+        c -= units;
+        kk++;
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < kB; b++) store_row_unit<VEC>(dst, at[b], buf[b]);
+  }
+}
+
+/* WAVES wavefronts per workgroup, each with its own keys and its own staging area.  One
  * wavefront per workgroup everywhere except the missed-keys variant, whose workgroups are
  * large so that the list of misses is claimed with one atomic per 1024 keys (updates of one
  * word are served one at a time, about 15 ns each: one per wavefront would take longer than
  * the lookup itself). */
-template <int MODE, int VEC, bool DUAL = false, int WAVES = 1>
+template <int MODE, int VEC, bool DUAL = false, int WAVES = 1, int R = kTile, bool MISSED = false>
 __global__ void __launch_bounds__(kWave * WAVES)
 lookup_kernel(View v, FindArgs a) {
   __shared__ KeyMeta s_meta_all[WAVES][kWave];
@@ -275,19 +342,19 @@ lookup_kernel(View v, FindArgs a) {
   const int wave = threadIdx.x / kWave;
   KeyMeta* const s_meta = s_meta_all[wave];
   int64_t* const s_slot = s_slot_all[wave];
-  const uint64_t base = ((uint64_t)blockIdx.x * WAVES + wave) * kWave;
-  const uint64_t i = base + lane;
+  const uint64_t base = ((uint64_t)blockIdx.x * WAVES + wave) * (kTilesPerWave * R);
+  const uint64_t i = lane_owns_key<R>(lane) ? key_of_lane<R>((uint64_t)blockIdx.x * WAVES + wave, lane) : a.n;
   const uint64_t key = stage_keys(v, a.keys, a.n, i, s_meta, s_slot, lane);
   if (DUAL) restage_first_bucket(v, s_meta, lane);
-  if (WAVES > 1 && threadIdx.x == 0) s_missed[0] = 0;
-  __syncthreads();
-  probe_wave<false, true>(v, s_meta, s_slot, nullptr, nullptr, lane);
-  __syncthreads();
+  if (MISSED && threadIdx.x == 0) s_missed[0] = 0;
+  wave_sync();
+  probe_wave<false, true, R>(v, s_meta, s_slot, nullptr, nullptr, lane);
+  wave_sync();
   if (DUAL) {
     restage_second_bucket(v, s_meta, s_slot, lane);
-    __syncthreads();
-    probe_wave<false, true>(v, s_meta, s_slot, nullptr, nullptr, lane);
-    __syncthreads();
+    wave_sync();
+    probe_wave<false, true, R>(v, s_meta, s_slot, nullptr, nullptr, lane);
+    wave_sync();
   }
 
   const int64_t my_slot = s_slot[lane];
@@ -300,22 +367,18 @@ lookup_kernel(View v, FindArgs a) {
       if (MODE == kLookupPtr) a.out_ptrs[i] = nullptr;
     }
   }
-  if (a.missed_size) {
+  if constexpr (MISSED) {
     /* missed-keys variant (lookup.cuh:36-60): compact list of misses, in no particular
      * order; reserved keys are not probed and count as missed. */
     const bool miss = i < a.n && my_slot < 0;
     const unsigned long long mm = __ballot(miss);
     int32_t at = 0;
-    if (WAVES > 1) {
-      if (lane == 0 && mm) at = atomicAdd(&s_missed[0], (int32_t)__popcll(mm));
-      __syncthreads();
-      if (threadIdx.x == 0 && s_missed[0]) s_missed[1] = atomicAdd(a.missed_size, s_missed[0]);
-      __syncthreads();
-      at = __shfl(at, 0) + s_missed[1];
-    } else {
-      if (lane == 0 && mm) at = atomicAdd(a.missed_size, (int32_t)__popcll(mm));
-      at = __shfl(at, 0);
-    }
+    __syncthreads(); /* s_missed has been cleared */
+    if (lane == 0 && mm) at = atomicAdd(&s_missed[0], (int32_t)__popcll(mm));
+    __syncthreads();
+    if (threadIdx.x == 0 && s_missed[0]) s_missed[1] = atomicAdd(a.missed_size, s_missed[0]);
+    __syncthreads();
+    at = __shfl(at, 0) + s_missed[1];
     if (miss) {
       at += (int32_t)__popcll(mm & ((1ull << lane) - 1));
       a.missed_keys[at] = key;
@@ -324,117 +387,16 @@ lookup_kernel(View v, FindArgs a) {
   }
   if (MODE != kLookupValues) return;
 
-  /* copy stage: 64 rows x units-per-row spread over the 64 lanes.  All loads
-   * of a batch are issued before the first store, so a wavefront keeps up to
-   * kBatch KB of value rows in flight (the whole 16 KB for 256-byte rows). */
-  using T = typename VecType<VEC>::type;
-  const uint32_t units = v.value_bytes / VEC;
-  const uint32_t total = units * kWave;
-  const bool pow2 = (units & (units - 1)) == 0;
-  const uint32_t sh = 31 - __clz(units);
-  if constexpr (VEC == 16) {
-    /* Rows of 16 to 1024 bytes whose size is a power of two, all in HBM, slot numbers below
-     * 2^32 (every decision here is the same for the whole wavefront): lane L then always
-     * moves unit L mod units of a row, and in pass b the row of key (L / units) + b * (64 /
-     * units), so the slot numbers are read from LDS in one go and an address costs one
-     * multiply-add.  The general form below spends more instructions on addresses than
-     * the memory system needs time for the rows. */
-    if (pow2 && units <= kWave && v.hbm_slots >= v.capacity && v.capacity <= 0xFFFFFFFFull) {
-      constexpr int kB = 16;
-      const uint32_t c = lane & (units - 1);
-      const uint32_t kk0 = lane >> sh;
-      const uint32_t kstep = kWave >> sh;
-      const uint8_t* const src0 = v.values + c * 16;
-      uint8_t* const dst0 = a.out_values + (base + kk0) * v.value_bytes + c * 16;
-      const uint64_t dstep = (uint64_t)kstep * v.value_bytes;
-      /* with all 64 keys found nothing below is conditional, and the stores start as the
-       * first rows arrive instead of after the last one */
-      const bool all = __ballot(my_slot >= 0) == ~0ull;
-      auto move = [&](auto all_found) {
-        constexpr bool ALL = decltype(all_found)::value;
-        for (uint32_t b0 = 0; b0 < units; b0 += kB) {
-          int64_t sl[kB];
-          u32x4_t buf[kB];
-          if (ALL && units >= kB) {
-#pragma unroll
-            for (int b = 0; b < kB; b++) sl[b] = s_slot[kk0 + (b0 + b) * kstep];
-#pragma unroll
-            for (int b = 0; b < kB; b++)
-              buf[b] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(
-                  src0 + (uint64_t)(uint32_t)sl[b] * v.value_bytes));
-#pragma unroll
-            for (int b = 0; b < kB; b++)
-              __builtin_nontemporal_store(buf[b],
-                                          reinterpret_cast<u32x4_t*>(dst0 + (b0 + b) * dstep));
-          } else {
-#pragma unroll
-            for (int b = 0; b < kB; b++)
-              sl[b] = b0 + b < units ? s_slot[kk0 + (b0 + b) * kstep] : -1;
-#pragma unroll
-            for (int b = 0; b < kB; b++)
-              if (sl[b] >= 0)
-                buf[b] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(
-                    src0 + (uint64_t)(uint32_t)sl[b] * v.value_bytes));
-#pragma unroll
-            for (int b = 0; b < kB; b++)
-              if (sl[b] >= 0)
-                __builtin_nontemporal_store(buf[b],
-                                            reinterpret_cast<u32x4_t*>(dst0 + (b0 + b) * dstep));
-          }
-        }
-      };
-      if (all)
-        move(std::true_type{});
-      else
-        move(std::false_type{});
-      return;
-    }
-  }
-  constexpr int kBatch = VEC == 16 ? 16 : 4;
-  for (uint32_t idx0 = lane; idx0 < total; idx0 += kWave * kBatch) {
-    T buf[kBatch];
-#pragma unroll
-    for (int b = 0; b < kBatch; b++) {
-      const uint32_t idx = idx0 + b * kWave;
-      buf[b] = T{};
-      if (idx < total) {
-        const uint32_t kk = pow2 ? (idx >> sh) : (idx / units);
-        const uint32_t c = idx - kk * units;
-        const int64_t slot = s_slot[kk];
-        if (slot >= 0) {
-          const T* src = reinterpret_cast<const T*>(value_row(v, (uint64_t)slot)) + c;
-          if constexpr (VEC == 16) {
-            /* a row is read once: streaming (non-temporal) loads, measured ~6 %
-             * faster here than plain ones */
-            const u32x4_t t = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(src));
-            buf[b] = make_uint4(t.x, t.y, t.z, t.w);
-          } else {
-            buf[b] = *src;
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int b = 0; b < kBatch; b++) {
-      const uint32_t idx = idx0 + b * kWave;
-      if (idx < total) {
-        const uint32_t kk = pow2 ? (idx >> sh) : (idx / units);
-        const uint32_t c = idx - kk * units;
-        if (s_slot[kk] >= 0) {
-          T* dst = reinterpret_cast<T*>(a.out_values + (base + kk) * v.value_bytes) + c;
-          if constexpr (VEC == 16) {
-            /* streaming store: the output is not read again here, and rows left dirty
-             * in the caches would be written back at the expense of the next call
-             * (measured: find itself 2 % slower, a following upsert 6 % faster) */
-            const u32x4_t t = {buf[b].x, buf[b].y, buf[b].z, buf[b].w};
-            __builtin_nontemporal_store(t, reinterpret_cast<u32x4_t*>(dst));
-          } else {
-            *dst = buf[b];
-          }
-        }
-      }
-    }
-  }
+  /* Copy stage: the rows of the wavefront's keys, spread over its 64 lanes.  All loads of a batch
+   * are issued before the first store, and none of them is conditional: a key that was not found
+   * reads slot 0's row, which stays in the caches, and its store goes past the end of the buffer
+   * resource, where the hardware drops it.  Behind a condition every load and store is a block of
+   * its own, and the compiler waits for more loads than a store needs. */
+  if (base >= a.n) return;
+  if (v.hbm_slots >= v.capacity && v.capacity <= 0xFFFFFFFFull)
+    copy_found_rows<VEC, R, true>(v, s_slot, a.out_values, base, a.n, lane);
+  else
+    copy_found_rows<VEC, R, false>(v, s_slot, a.out_values, base, a.n, lane);
 }
 
 }  // namespace hkv

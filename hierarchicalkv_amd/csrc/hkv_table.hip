@@ -4,10 +4,11 @@
  * What lives here: argument checks with the reference's messages
  * (merlin_hashtable.cuh:1016-1048, 3832-3861), table memory (flat arenas; HBM
  * first, pinned mapped host memory for value rows past max_hbm_for_vectors),
- * the stream-ordered group lock, and the choice of kernel instance per call.
+ * the stream-ordered group lock, and what a call asks of its kernel.  The kernel
+ * instances of the lookups, the upserts and the assigns are chosen and compiled
+ * in translation units of their own (hkv_launch.hpp).
  */
 #include <hip/hip_runtime.h>
-#include <hip/hip_ext.h>
 
 #include <algorithm>
 #include <atomic>
@@ -25,14 +26,16 @@
 #include <vector>
 
 #include "hkv_c_api.h"
+#include "hkv_launch.hpp"
 #include "hkv_misc.hpp"
-#include "hkv_upsert.hpp"
 #include "hkv_dedup.hpp"
 #include "hkv_dual.hpp"
 #include "hkv_grouped.hpp"
 #include "hkv_keylocks.hpp"
 
 using namespace hkv;
+
+thread_local hipEvent_t hkv::g_time_start = nullptr, hkv::g_time_stop = nullptr;
 
 namespace {
 
@@ -295,19 +298,6 @@ int pick_vec(uint32_t value_bytes, std::initializer_list<const void*> ptrs) {
   return 1;
 }
 
-inline unsigned grid_for(uint64_t n) { return (unsigned)((n + kWave - 1) / kWave); }
-
-/* units per lane that the bulk copy keeps in registers: rows of up to 8 * UPL
- * units go through in one pass (16-byte units: 128, 256, 512, 1024 bytes) */
-int pick_upl(uint32_t value_bytes, int vec) {
-  if (vec != 16) return 8;
-  const uint32_t units = value_bytes / 16;
-  if (units <= 8) return 1;
-  if (units <= 16) return 2;
-  if (units <= 32) return 4;
-  return 8;
-}
-
 /* accum_or_assign adds element by element, so its unit must hold whole elements: the widest of
  * 16, 8, 4, 2 and 1 bytes that the row size and the pointer allow, or 0 when that is less than
  * one element (an odd address for 16-bit elements, and the like). */
@@ -321,78 +311,6 @@ int accum_unit(uint32_t value_bytes, const void* p, int kind) {
       break;
     }
   return unit >= (int)elem[kind] ? unit : 0;
-}
-
-/* hkv_time_next_kernel: the pair of events that the calling thread's next main kernel (the one
- * kernel of a find or of an upsert-family call) is launched with.  The runtime stamps them with
- * the start and the end of that kernel's execution, so the time between them is the kernel's own,
- * without the gaps between the launches of a stream that events recorded around a call include. */
-thread_local hipEvent_t g_time_start = nullptr, g_time_stop = nullptr;
-
-template <class... KArgs, class... Args>
-void launch_main(void (*kernel)(KArgs...), dim3 grid, dim3 block, hipStream_t s, Args... args) {
-  if (g_time_start) {
-    hipExtLaunchKernelGGL(kernel, grid, block, 0, s, g_time_start, g_time_stop, 0, args...);
-    g_time_start = g_time_stop = nullptr;
-  } else {
-    hipLaunchKernelGGL(kernel, grid, block, 0, s, args...);
-  }
-}
-
-/* BOUNDS: the victim search reads the bucket's score bounds and one or two of its score lines
- * instead of all eight (hkv_upsert.hpp); for 16-byte units, which is what tables with rows of a
- * multiple of 16 bytes use. */
-template <int OP, bool LOCKED_RULE, bool BOUNDS = false, int WAVES = 1, bool HOLD = false>
-void launch_upsert(int vec, const View& v, const UpsertArgs& a, hipStream_t s) {
-  const dim3 grid(grid_for((a.n + WAVES - 1) / WAVES)), block(kWave * WAVES);
-  if constexpr (OP == kOpAccumOrAssign && !BOUNDS) {
-    /* the two units that only the element-wise add needs */
-    if (vec == 8) {
-      launch_main(upsert_kernel<OP, 8, 8, LOCKED_RULE, false, WAVES, HOLD>, grid, block, s, v, a);
-      return;
-    }
-    if (vec == 2) {
-      launch_main(upsert_kernel<OP, 2, 8, LOCKED_RULE, false, WAVES, HOLD>, grid, block, s, v, a);
-      return;
-    }
-  }
-  if (OP == kOpFindOrInsertPtr) {
-    launch_main(upsert_kernel<OP, 16, 1, LOCKED_RULE, BOUNDS, WAVES, HOLD>, grid, block, s, v, a);
-    return;
-  }
-  if (vec == 16) {
-    switch (pick_upl(v.value_bytes, 16)) {
-      case 1: launch_main(upsert_kernel<OP, 16, 1, LOCKED_RULE, BOUNDS, WAVES, HOLD>, grid, block, s, v, a); break;
-      case 2: launch_main(upsert_kernel<OP, 16, 2, LOCKED_RULE, BOUNDS, WAVES, HOLD>, grid, block, s, v, a); break;
-      case 4: launch_main(upsert_kernel<OP, 16, 4, LOCKED_RULE, BOUNDS, WAVES, HOLD>, grid, block, s, v, a); break;
-      default: launch_main(upsert_kernel<OP, 16, 8, LOCKED_RULE, BOUNDS, WAVES, HOLD>, grid, block, s, v, a); break;
-    }
-  } else if constexpr (!BOUNDS) {
-    if (vec == 4)
-      launch_main(upsert_kernel<OP, 4, 8, LOCKED_RULE, false, WAVES, HOLD>, grid, block, s, v, a);
-    else
-      launch_main(upsert_kernel<OP, 1, 8, LOCKED_RULE, false, WAVES, HOLD>, grid, block, s, v, a);
-  }
-}
-
-/* insert_and_evict with `pair`: two wavefronts per workgroup share the claims on the
- * evicted-keys output (hkv_upsert.hpp) */
-template <int OP, bool LOCKED_RULE, bool BOUNDS = false>
-void launch_upsert_for(bool pair, int vec, const View& v, const UpsertArgs& a, hipStream_t s) {
-  if constexpr (OP == kOpInsertOrAssign || OP == kOpFindOrInsert) {
-    /* hybrid mode: the list of slots that stay LOCKED to the end of the launch */
-    if (a.held_scores) {
-      launch_upsert<OP, LOCKED_RULE, BOUNDS, 1, true>(vec, v, a, s);
-      return;
-    }
-  }
-  if constexpr (OP == kOpInsertAndEvict) {
-    if (pair) {
-      launch_upsert<OP, LOCKED_RULE, BOUNDS, 2>(vec, v, a, s);
-      return;
-    }
-  }
-  launch_upsert<OP, LOCKED_RULE, BOUNDS, 1>(vec, v, a, s);
 }
 
 /* The two kernels of the two-phase insert_or_assign (hkv_grouped.hpp) for a row size. */
@@ -855,12 +773,12 @@ int run_upsert(hkv_table* t, UpsertArgs a, int vec, bool hybrid_rule, hipStream_
        * no such slot the plain scan finds the same victims (a slot locked by another key of
        * the batch is retried instead of skipped) */
       writes_scores_outside_bounds(t, s, own_rule);
-      launch_upsert_for<OP, true>(pair, vec, t->view, a, s);
+      launch_upsert<OP>({true, false, pair}, vec, t->view, a, s);
     } else if (prepare_bounds<OP>(t, a, vec, s)) {
-      launch_upsert_for<OP, false, true>(pair, vec, t->view, a, s);
+      launch_upsert<OP>({false, true, pair}, vec, t->view, a, s);
     } else {
       writes_scores_outside_bounds(t, s, own_rule);
-      launch_upsert_for<OP, false>(pair, vec, t->view, a, s);
+      launch_upsert<OP>({false, false, pair}, vec, t->view, a, s);
     }
     hipError_t e = hipGetLastError();
     if (hold) {
@@ -980,7 +898,7 @@ int cpu_io_upsert(hkv_table* t, UpsertArgs a, void* values, bool reads, hipStrea
     if (e == hipSuccess) e = hipMemsetAsync(d_tmp, 0, n * 9, s); /* reserved / refused keys: no address */
     if (e == hipSuccess) {
       writes_scores_outside_bounds(t, s, a.strategy == t->opts.evict_strategy);
-      launch_upsert<kOpFindOrInsertPtr, true>(16, t->view, a, s);
+      launch_upsert<kOpFindOrInsertPtr>({true, false, false}, 16, t->view, a, s);
       hipLaunchKernelGGL(cpu_io_owner_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
                          t->view, a.keys, (uint8_t**)d_tmp,
                          reads ? (const uint8_t*)d_tmp + n * 8 : nullptr, n);
@@ -1067,54 +985,13 @@ void launch_dual_upsert(int vec, const View& v, const UpsertArgs& whole, hipStre
   }
 }
 
-void launch_dual_lookup(int vec, const View& v, const FindArgs& a, hipStream_t s) {
-  const dim3 grid(grid_for(a.n)), block(kWave);
-  if (vec == 16)
-    hipLaunchKernelGGL((lookup_kernel<kLookupValues, 16, true>), grid, block, 0, s, v, a);
-  else if (vec == 4)
-    hipLaunchKernelGGL((lookup_kernel<kLookupValues, 4, true>), grid, block, 0, s, v, a);
-  else
-    hipLaunchKernelGGL((lookup_kernel<kLookupValues, 1, true>), grid, block, 0, s, v, a);
-}
-
-template <int MODE>
-void launch_lookup(int vec, const View& v, const FindArgs& a, hipStream_t s) {
-  const dim3 grid(grid_for(a.n)), block(kWave);
-  if (vec == 16)
-    launch_main(lookup_kernel<MODE, 16>, grid, block, s, v, a);
-  else if (vec == 4)
-    launch_main(lookup_kernel<MODE, 4>, grid, block, s, v, a);
-  else
-    launch_main(lookup_kernel<MODE, 1>, grid, block, s, v, a);
-}
-
-/* the missed-keys find: 16 wavefronts per workgroup (see lookup_kernel) */
-void launch_lookup_missed(int vec, const View& v, const FindArgs& a, hipStream_t s) {
-  constexpr int kWaves = 16;
-  const dim3 grid((unsigned)((a.n + kWave * kWaves - 1) / (kWave * kWaves))), block(kWave * kWaves);
-  if (vec == 16)
-    hipLaunchKernelGGL((lookup_kernel<kLookupValues, 16, false, kWaves>), grid, block, 0, s, v, a);
-  else if (vec == 4)
-    hipLaunchKernelGGL((lookup_kernel<kLookupValues, 4, false, kWaves>), grid, block, 0, s, v, a);
-  else
-    hipLaunchKernelGGL((lookup_kernel<kLookupValues, 1, false, kWaves>), grid, block, 0, s, v, a);
-}
-
-template <bool LOCKFREE>
-void launch_assign(int vec, const View& v, const AssignArgs& a, hipStream_t s) {
-  const dim3 grid(grid_for(a.n)), block(kWave);
-  if (vec == 16) {
-    switch (pick_upl(v.value_bytes, 16)) {
-      case 1: hipLaunchKernelGGL((assign_kernel<16, 1, LOCKFREE>), grid, block, 0, s, v, a); break;
-      case 2: hipLaunchKernelGGL((assign_kernel<16, 2, LOCKFREE>), grid, block, 0, s, v, a); break;
-      case 4: hipLaunchKernelGGL((assign_kernel<16, 4, LOCKFREE>), grid, block, 0, s, v, a); break;
-      default: hipLaunchKernelGGL((assign_kernel<16, 8, LOCKFREE>), grid, block, 0, s, v, a); break;
-    }
-  } else if (vec == 4) {
-    hipLaunchKernelGGL((assign_kernel<4, 8, LOCKFREE>), grid, block, 0, s, v, a);
-  } else {
-    hipLaunchKernelGGL((assign_kernel<1, 8, LOCKFREE>), grid, block, 0, s, v, a);
-  }
+/* unit of the row copies of a lookup: 16 bytes where rows and pointer allow it, else the widest unit
+ * that fits into a row, at any address */
+int lookup_unit(uint32_t value_bytes, const void* out) {
+  if (((value_bytes | (uintptr_t)out) & 15) == 0) return 16;
+  for (int w : {16, 8, 4, 2})
+    if (value_bytes >= (uint32_t)w) return kAny + w;
+  return 1;
 }
 
 template <class Pred>
@@ -1640,7 +1517,7 @@ static int assign_common(hkv_table* t, uint64_t n, const uint64_t* keys,
       if (e == hipSuccess && touch_scores) {
         a.values = nullptr;
         writes_scores_outside_bounds(t, s, true);
-        launch_assign<false>(16, t->view, a, s);
+        launch_assign(false, 16, t->view, a, s);
         e = hipGetLastError();
       }
       if (e == hipSuccess) e = hipMemsetAsync(d_tmp, 0, n * 9, s); /* reserved keys: no address */
@@ -1650,7 +1527,7 @@ static int assign_common(hkv_table* t, uint64_t n, const uint64_t* keys,
         f.out_ptrs = (void**)d_tmp;
         f.founds = (uint8_t*)d_tmp + n * 8;
         f.n = n;
-        launch_lookup<kLookupPtr>(16, t->view, f, s);
+        launch_find_ptr(t->view, f, s);
         e = hipGetLastError();
       }
       if (e == hipSuccess) e = hipMemcpyAsync(st.ptrs, d_tmp, n * 8, hipMemcpyDeviceToHost, s);
@@ -1676,9 +1553,9 @@ static int assign_common(hkv_table* t, uint64_t n, const uint64_t* keys,
         a.bound_ceil = t->d_bound_ceil;
     }
     if (lockfree)
-      launch_assign<true>(vec, t->view, a, s);
+      launch_assign(true, vec, t->view, a, s);
     else
-      launch_assign<false>(vec, t->view, a, s);
+      launch_assign(false, vec, t->view, a, s);
     HKV_HIP(hipGetLastError());
   }
   if (t->clock.mode == 1) t->clock.base += UINT64_C(1) << 40;
@@ -1718,13 +1595,13 @@ int hkv_find(const hkv_table* t, uint64_t n, const uint64_t* keys, void* values,
   a.founds = founds;
   a.out_scores = scores;
   a.n = n;
-  const int vec = pick_vec(t->view.value_bytes, {values});
+  const int vec = lookup_unit(t->view.value_bytes, values);
   LockGuard g(t, StreamGroupLock::kReader, s);
   HKV_HIP(g.acquire());
   if (t->dual)
-    launch_dual_lookup(vec, t->view, a, s);
+    launch_find_dual(vec, t->view, a, s);
   else
-    launch_lookup<kLookupValues>(vec, t->view, a, s);
+    launch_find(vec, t->view, a, s);
   HKV_HIP(hipGetLastError());
   return HKV_SUCCESS;
 }
@@ -1743,11 +1620,11 @@ int hkv_find_missed(const hkv_table* t, uint64_t n, const uint64_t* keys,
   a.missed_indices = missed_indices;
   a.missed_size = missed_size;
   a.n = n;
-  const int vec = pick_vec(t->view.value_bytes, {values});
+  const int vec = lookup_unit(t->view.value_bytes, values);
   hipLaunchKernelGGL(zero_i32_kernel, dim3(1), dim3(1), 0, s, missed_size);
   LockGuard g(t, StreamGroupLock::kReader, s);
   HKV_HIP(g.acquire());
-  launch_lookup_missed(vec, t->view, a, s);
+  launch_find_missed(vec, t->view, a, s);
   HKV_HIP(hipGetLastError());
   return HKV_SUCCESS;
 }
@@ -1767,7 +1644,7 @@ int hkv_find_ptr(const hkv_table* t, uint64_t n, const uint64_t* keys,
   a.n = n;
   LockGuard g(t, StreamGroupLock::kReader, s);
   HKV_HIP(g.acquire());
-  launch_lookup<kLookupPtr>(16, t->view, a, s);
+  launch_find_ptr(t->view, a, s);
   HKV_HIP(hipGetLastError());
   return HKV_SUCCESS;
 }
@@ -1783,7 +1660,7 @@ int hkv_contains(const hkv_table* t, uint64_t n, const uint64_t* keys,
   a.n = n;
   LockGuard g(t, StreamGroupLock::kReader, s);
   HKV_HIP(g.acquire());
-  launch_lookup<kLookupContains>(16, t->view, a, s);
+  launch_contains(t->view, a, s);
   HKV_HIP(hipGetLastError());
   return HKV_SUCCESS;
 }

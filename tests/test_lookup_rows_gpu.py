@@ -1,0 +1,49 @@
+"""find over row sizes, output addresses and batch sizes: the rows of keys that are present come back
+byte for byte, everything else in the output buffer stays as it was."""
+import numpy as np
+import pytest
+import torch
+
+import workloads as w
+from gpu_util import DEV, dev
+from hierarchicalkv_amd import HashTable, default_options
+
+pytestmark = pytest.mark.gpu
+PAD = 64
+
+
+# rows below 16 bytes (units of 1, 2, 4, 8), at and around 16, with a last unit that overlaps, of 512
+# bytes and more (one key per tile); addresses off by nothing, by 4, by 1; batches at the edges of a
+# tile's and a wavefront's keys and where the keys per tile change (2^14)
+@pytest.mark.parametrize("row_bytes,shift", [
+    (1, 0), (2, 0), (3, 1), (5, 0), (7, 1), (8, 0), (12, 4), (15, 0), (16, 0), (16, 4), (17, 0), (31, 1), (32, 1), (66, 0),
+    (200, 4), (256, 0), (512, 0), (516, 0), (1028, 1), (4100, 0)])
+def test_rows_of_every_size(row_bytes, shift):
+    cap, resident = 1 << 15, 20000
+    t = HashTable()
+    t.init(default_options(init_capacity=cap, max_capacity=cap, max_hbm_for_vectors=1 << 34, dim=row_bytes,
+                           value_kind=0, value_size=1))
+    keys = w.unique_keys(61, 0, resident)
+    rng = np.random.Generator(np.random.PCG64(row_bytes))
+    rows = rng.integers(0, 256, (resident, row_bytes), dtype=np.uint8)
+    t.insert_or_assign(resident, dev(keys), dev(rows))
+    assert t.size() == resident
+    absent = w.unique_keys(62, 0, 3000)
+    for n in (1, 2, 7, 8, 9, 15, 16, 17, 63, 65, 1000, 16384, 16385, 16400):
+        if n > 1000 and row_bytes > 2000:
+            continue
+        pick = rng.integers(0, resident, n)
+        miss = rng.random(n) < 0.2
+        q = np.where(miss, absent[np.arange(n) % len(absent)], keys[pick])
+        buf = torch.full((PAD + shift + n * row_bytes + PAD,), 0xA5, dtype=torch.uint8, device=DEV)
+        founds = torch.zeros(n, dtype=torch.bool, device=DEV)
+        d_q = dev(q)
+        t.find(n, d_q, buf[PAD + shift:], founds)
+        torch.cuda.synchronize()
+        assert (founds.cpu().numpy() == ~miss).all()
+        got = buf.cpu().numpy()
+        body = got[PAD + shift:PAD + shift + n * row_bytes].reshape(n, row_bytes)
+        assert (body[~miss] == rows[pick[~miss]]).all()
+        assert (body[miss] == 0xA5).all()
+        assert (got[:PAD + shift] == 0xA5).all() and (got[PAD + shift + n * row_bytes:] == 0xA5).all()
+    t.close()

@@ -8,58 +8,85 @@ namespace {
 
 /* BOUNDS: the victim search reads the bucket's score bounds and one or two of its score lines
  * instead of all eight (hkv_upsert.hpp); for 16-byte units, which is what tables with rows of a
- * multiple of 16 bytes use. */
-template <int OP, bool LOCKED_RULE, bool BOUNDS = false, int WAVES = 1, bool HOLD = false>
+ * multiple of 16 bytes use.
+ * R: keys per tile (hkv_lookup.hpp). */
+template <int OP, int R, bool LOCKED_RULE, bool BOUNDS = false, int WAVES = 1, bool HOLD = false>
 void launch_form(int vec, const View& v, const UpsertArgs& a, hipStream_t s) {
-  const dim3 grid(grid_for((a.n + WAVES - 1) / WAVES)), block(kWave * WAVES);
+  constexpr uint64_t kKeys = (uint64_t)kTilesPerWave * R * WAVES;
+  const dim3 grid((unsigned)((a.n + kKeys - 1) / kKeys)), block(kWave * WAVES);
   if constexpr (OP == kOpAccumOrAssign && !BOUNDS) {
     /* the two units that only the element-wise add needs */
     if (vec == 8) {
-      launch_main(upsert_kernel<OP, 8, 8, LOCKED_RULE, false, WAVES, HOLD>, grid, block, s, v, a);
+      launch_main(upsert_kernel<OP, 8, 8, LOCKED_RULE, false, WAVES, HOLD, R>, grid, block, s, v, a);
       return;
     }
     if (vec == 2) {
-      launch_main(upsert_kernel<OP, 2, 8, LOCKED_RULE, false, WAVES, HOLD>, grid, block, s, v, a);
+      launch_main(upsert_kernel<OP, 2, 8, LOCKED_RULE, false, WAVES, HOLD, R>, grid, block, s, v, a);
       return;
     }
   }
   if (OP == kOpFindOrInsertPtr) {
-    launch_main(upsert_kernel<OP, 16, 1, LOCKED_RULE, BOUNDS, WAVES, HOLD>, grid, block, s, v, a);
+    launch_main(upsert_kernel<OP, 16, 1, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a);
     return;
   }
   if (vec == 16) {
     switch (pick_upl(v.value_bytes, 16)) {
-      case 1: launch_main(upsert_kernel<OP, 16, 1, LOCKED_RULE, BOUNDS, WAVES, HOLD>, grid, block, s, v, a); break;
-      case 2: launch_main(upsert_kernel<OP, 16, 2, LOCKED_RULE, BOUNDS, WAVES, HOLD>, grid, block, s, v, a); break;
-      case 4: launch_main(upsert_kernel<OP, 16, 4, LOCKED_RULE, BOUNDS, WAVES, HOLD>, grid, block, s, v, a); break;
-      default: launch_main(upsert_kernel<OP, 16, 8, LOCKED_RULE, BOUNDS, WAVES, HOLD>, grid, block, s, v, a); break;
+      case 1: launch_main(upsert_kernel<OP, 16, 1, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+      case 2: launch_main(upsert_kernel<OP, 16, 2, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+      case 4: launch_main(upsert_kernel<OP, 16, 4, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+      default: launch_main(upsert_kernel<OP, 16, 8, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
     }
   } else if constexpr (!BOUNDS) {
     if (vec == 4)
-      launch_main(upsert_kernel<OP, 4, 8, LOCKED_RULE, false, WAVES, HOLD>, grid, block, s, v, a);
+      launch_main(upsert_kernel<OP, 4, 8, LOCKED_RULE, false, WAVES, HOLD, R>, grid, block, s, v, a);
     else
-      launch_main(upsert_kernel<OP, 1, 8, LOCKED_RULE, false, WAVES, HOLD>, grid, block, s, v, a);
+      launch_main(upsert_kernel<OP, 1, 8, LOCKED_RULE, false, WAVES, HOLD, R>, grid, block, s, v, a);
   }
 }
 
-/* insert_and_evict with `pair`: two wavefronts per workgroup share the claims on the
+/* insert_and_evict with `pair`: the wavefronts of 128 keys share the claims on the
  * evicted-keys output (hkv_upsert.hpp) */
-template <int OP, bool LOCKED_RULE, bool BOUNDS = false>
+template <int OP, bool LOCKED_RULE, bool BOUNDS, int R>
 void launch_upsert_for(bool pair, int vec, const View& v, const UpsertArgs& a, hipStream_t s) {
   if constexpr (OP == kOpInsertOrAssign || OP == kOpFindOrInsert) {
     /* hybrid mode: the list of slots that stay LOCKED to the end of the launch */
     if (a.held_scores) {
-      launch_form<OP, LOCKED_RULE, BOUNDS, 1, true>(vec, v, a, s);
+      launch_form<OP, R, LOCKED_RULE, BOUNDS, 1, true>(vec, v, a, s);
       return;
     }
   }
   if constexpr (OP == kOpInsertAndEvict) {
     if (pair) {
-      launch_form<OP, LOCKED_RULE, BOUNDS, 2>(vec, v, a, s);
+      launch_form<OP, R, LOCKED_RULE, BOUNDS, 2 * kTile / R>(vec, v, a, s);
       return;
     }
   }
-  launch_form<OP, LOCKED_RULE, BOUNDS, 1>(vec, v, a, s);
+  launch_form<OP, R, LOCKED_RULE, BOUNDS, 1>(vec, v, a, s);
+}
+
+/* Keys per tile.  With 8 a wavefront holds 64 keys in 110 to 128 registers and takes them through the
+ * victim search and the row copies one or two at a time, so that a batch of a few ten thousand keys
+ * is a long chain on part of the chip; with fewer keys per tile the chain is shorter, more wavefronts
+ * fit on a SIMD, and every step is issued for fewer keys at once, which is what costs once the chip is
+ * full anyway.  us for the whole step, R = 8 / 2 / 1:
+ *   full table (bounds), insert_or_assign with half of the keys new, and find, rows of 256 bytes
+ *     2^12 keys   68 /  36 /  31      2^16   84 /  54 /  51      2^18  127 / 116 / 120
+ *     2^14        71 /  41 /  36      2^17   97 /  74 /  73      2^20  393 / 397 / 438
+ *   the same with nearly all keys found, 2^19 keys of 64 bytes: 123 / 132 / 151
+ *   full table, insert_and_evict, rows of 64 bytes
+ *     2^15 keys  128 /  92 /  88      2^17  151 / 122 / 139      2^18  186 / 167 / 207
+ *   table with free slots, find_or_insert and insert_or_assign of repeated ids, 512 (2^18: 128) bytes
+ *     2^15 keys   88 /  81 /  81      2^17  145 / 136 / 143      2^18  133 / 147 / 156
+ * The last line is what `repeats` is for: there is no search for a victim to shorten, and a good part
+ * of the keys has been crossed off beforehand. */
+template <int OP, bool BOUNDS>
+void launch_by_size(bool pair, bool repeats, int vec, const View& v, const UpsertArgs& a, hipStream_t s) {
+  if (a.n <= (UINT64_C(1) << (BOUNDS ? 15 : 14)))
+    launch_upsert_for<OP, false, BOUNDS, 1>(pair, vec, v, a, s);
+  else if (a.n <= (UINT64_C(1) << (BOUNDS && !repeats ? 18 : 17)))
+    launch_upsert_for<OP, false, BOUNDS, 2>(pair, vec, v, a, s);
+  else
+    launch_upsert_for<OP, false, BOUNDS, kTile>(pair, vec, v, a, s);
 }
 
 }  // namespace
@@ -67,11 +94,11 @@ void launch_upsert_for(bool pair, int vec, const View& v, const UpsertArgs& a, h
 template <int OP>
 void launch_upsert(const UpsertForm& form, int vec, const View& v, const UpsertArgs& a, hipStream_t s) {
   if (form.locked_rule)
-    launch_upsert_for<OP, true>(form.pair, vec, v, a, s);
+    launch_upsert_for<OP, true, false, kTile>(form.pair, vec, v, a, s);
   else if (form.bounds)
-    launch_upsert_for<OP, false, true>(form.pair, vec, v, a, s);
+    launch_by_size<OP, true>(form.pair, form.repeats, vec, v, a, s);
   else
-    launch_upsert_for<OP, false>(form.pair, vec, v, a, s);
+    launch_by_size<OP, false>(form.pair, form.repeats, vec, v, a, s);
 }
 template void launch_upsert<HKV_UPSERT_OP>(const UpsertForm&, int, const View&, const UpsertArgs&, hipStream_t);
 

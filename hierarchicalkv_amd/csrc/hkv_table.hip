@@ -728,7 +728,7 @@ bool prepare_bounds(hkv_table* t, UpsertArgs& a, int vec, hipStream_t s) {
  * the table is not pure HBM (insert_or_assign, find_or_insert); the pointer
  * overload always does. */
 template <int OP>
-int run_upsert(hkv_table* t, UpsertArgs a, int vec, bool hybrid_rule, hipStream_t s) {
+int run_upsert(hkv_table* t, UpsertArgs a, int vec, bool hybrid_rule, hipStream_t s, bool repeats = false) {
   HKV_TRY(grow_for(t, a.n, s));
   a.epoch = t->epoch;
   a.clock = t->clock;
@@ -773,12 +773,12 @@ int run_upsert(hkv_table* t, UpsertArgs a, int vec, bool hybrid_rule, hipStream_
        * no such slot the plain scan finds the same victims (a slot locked by another key of
        * the batch is retried instead of skipped) */
       writes_scores_outside_bounds(t, s, own_rule);
-      launch_upsert<OP>({true, false, pair}, vec, t->view, a, s);
+      launch_upsert<OP>({true, false, pair, repeats}, vec, t->view, a, s);
     } else if (prepare_bounds<OP>(t, a, vec, s)) {
-      launch_upsert<OP>({false, true, pair}, vec, t->view, a, s);
+      launch_upsert<OP>({false, true, pair, repeats}, vec, t->view, a, s);
     } else {
       writes_scores_outside_bounds(t, s, own_rule);
-      launch_upsert<OP>({false, false, pair}, vec, t->view, a, s);
+      launch_upsert<OP>({false, false, pair, repeats}, vec, t->view, a, s);
     }
     hipError_t e = hipGetLastError();
     if (hold) {
@@ -1276,7 +1276,7 @@ int hkv_insert_or_assign(hkv_table* t, uint64_t n, const uint64_t* keys,
   if (t->io_by_cpu) return cpu_io_upsert(t, a, const_cast<void*>(values), false, (hipStream_t)stream);
   /* with unique_key == false the reference leaves its lock-key kernels for the plain one
    * (merlin_hashtable.cuh:1235-1258), whose rule is "refuse when score < min" */
-  return run_upsert<kOpInsertOrAssign>(t, a, vec, unique_key != 0, (hipStream_t)stream);
+  return run_upsert<kOpInsertOrAssign>(t, a, vec, unique_key != 0, (hipStream_t)stream, !unique_key);
 }
 
 int hkv_insert_or_assign_noalloc(hkv_table* t, uint64_t n, const uint64_t* keys,
@@ -1367,7 +1367,7 @@ int hkv_insert_and_evict(hkv_table* t, uint64_t n, const uint64_t* keys,
   a.n = n;
   a.strategy = strategy;
   const int vec = pick_vec(t->view.value_bytes, {values, evicted_values});
-  return run_upsert<kOpInsertAndEvict>(t, a, vec, false, (hipStream_t)stream);
+  return run_upsert<kOpInsertAndEvict>(t, a, vec, false, (hipStream_t)stream, !unique_key);
 }
 
 int hkv_insert_and_evict_count(hkv_table* t, uint64_t n, const uint64_t* keys,
@@ -1429,7 +1429,7 @@ int hkv_find_or_insert(hkv_table* t, uint64_t n, const uint64_t* keys,
   if (t->io_by_cpu)
     HKV_TRY(cpu_io_upsert(t, a, values, true, (hipStream_t)stream));
   else /* merlin_hashtable.cuh:1779-1803: lock-key kernels only with unique keys */
-    HKV_TRY(run_upsert<kOpFindOrInsert>(t, a, vec, unique_key != 0, (hipStream_t)stream));
+    HKV_TRY(run_upsert<kOpFindOrInsert>(t, a, vec, unique_key != 0, (hipStream_t)stream, !unique_key));
   if (dg.on) {
     /* the other occurrences of a key get the row its representative ended up with (what it
      * read, or what it inserted; a refused key keeps its own row, like its representative) */

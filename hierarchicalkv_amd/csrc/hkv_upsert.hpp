@@ -2,7 +2,8 @@
  * The upsert family: insert_or_assign, insert_and_evict, find_or_insert
  * (values and pointers), accum_or_assign, and the assign family.  One kernel
  * template for every load factor; one 64-lane wavefront per workgroup,
- * 64 keys per wavefront.
+ * 8 to 64 keys per wavefront (R keys per 8-lane tile, chosen by the size of the batch in
+ * hkv_launch_upsert.hip; below for R = 8).
  *
  * Replaces tlp_v1/tlp_v2/pipeline_upsert_kernel_with_io (upsert.cuh:27-986),
  * the *_upsert_and_evict_kernel_unique kernels (upsert_and_evict.cuh:27-1099),
@@ -13,8 +14,9 @@
  * upsert.cuh:52-233.
  *
  * Division of labour inside a wavefront
- *   control  lane L owns key L: it decides what to lock, issues the 64-bit CAS
- *            on the key word, writes digest / score, and unlocks.  All 64 keys
+ *   control  lane L owns key L (with R < 8 the first R lanes of a tile own one each, the
+ *            others none): it decides what to lock, issues the 64-bit CAS
+ *            on the key word, writes digest / score, and unlocks.  All keys of a wavefront
  *            take each of these steps in one instruction, so a wavefront pays
  *            one memory round trip per step, not one per key.
  *   bulk     tile t (lanes 8t..8t+7) serves the keys 8t..8t+7 of its own
@@ -436,18 +438,18 @@ constexpr int kRowUnits = 8;
  * UPL = units per lane and row held in registers (1, 2, 4 or 8).
  * Every lane of the wavefront must call this.
  */
-template <int VEC, int UPL, bool CAN_READ_TABLE, bool CAN_ACCUM>
+template <int VEC, int UPL, bool CAN_READ_TABLE, bool CAN_ACCUM, int R = kTile>
 __device__ __forceinline__ void bulk_rows(int move, uint8_t* tab, uint8_t* usr,
                                           uint32_t units, int value_kind, int lane) {
   using T = typename VecType<VEC>::type;
   /* accumulating holds two rows per key (the table's and the caller's): half as many keys at a time */
   constexpr int kUnits = CAN_ACCUM ? kRowUnits / 2 : kRowUnits;
-  constexpr int kGroup = kUnits / UPL < 1 ? 1 : (kUnits / UPL < kTile ? kUnits / UPL : kTile);
+  constexpr int kGroup = kUnits / UPL < 1 ? 1 : (kUnits / UPL < R ? kUnits / UPL : R);
   const int j = lane & (kTile - 1);
   const int lane_base = lane & ~(kTile - 1);
   for (uint32_t u0 = 0; u0 < units; u0 += kTile * UPL) {
 #pragma unroll
-    for (int g = 0; g < kTile; g += kGroup) {
+    for (int g = 0; g < R; g += kGroup) {
       T x[kGroup][UPL];
       T y[CAN_ACCUM ? kGroup : 1][CAN_ACCUM ? UPL : 1];
 #pragma unroll
@@ -496,16 +498,16 @@ __device__ __forceinline__ void bulk_rows(int move, uint8_t* tab, uint8_t* usr,
 
 /* Copies towards the evicted-values output: kind 2 = the victim's table row
  * (coherent read), kind 1 = the refused key's input row, 0 = nothing. */
-template <int VEC, int UPL>
+template <int VEC, int UPL, int R>
 __device__ __forceinline__ void bulk_evicted(int kind, const uint8_t* src, uint8_t* dst,
                                              uint32_t units, int lane) {
   using T = typename VecType<VEC>::type;
-  constexpr int kGroup = kRowUnits / UPL < 1 ? 1 : (kRowUnits / UPL < kTile ? kRowUnits / UPL : kTile);
+  constexpr int kGroup = kRowUnits / UPL < 1 ? 1 : (kRowUnits / UPL < R ? kRowUnits / UPL : R);
   const int j = lane & (kTile - 1);
   const int lane_base = lane & ~(kTile - 1);
   for (uint32_t u0 = 0; u0 < units; u0 += kTile * UPL) {
 #pragma unroll
-    for (int g = 0; g < kTile; g += kGroup) {
+    for (int g = 0; g < R; g += kGroup) {
       T x[kGroup][UPL];
 #pragma unroll
       for (int q = 0; q < kGroup; q++) {
@@ -545,6 +547,7 @@ __device__ __forceinline__ void bulk_evicted(int kind, const uint8_t* src, uint8
  * 128-bit mask of EMPTY digests.  Every lane of the wavefront must call this.
  */
 constexpr int kMaxLockedWaits = 64;
+template <int R = kTile>
 __device__ __forceinline__ void settle_reprobes(const View& v, uint64_t key, uint32_t bkt,
                                                 uint32_t digest, bool pending, bool& reprobe,
                                                 int64_t& hit, uint64_t& em_lo, uint64_t& em_hi,
@@ -552,7 +555,7 @@ __device__ __forceinline__ void settle_reprobes(const View& v, uint64_t key, uin
   const int tile = lane >> 3, j = lane & 7;
   const int lane_base = lane & ~(kTile - 1);
 #pragma unroll 1
-  for (int r = 0; r < kTile; r++) {
+  for (int r = 0; r < R; r++) {
     const int src = lane_base + r;
     if (!__shfl((int)(pending && reprobe), src)) continue; /* tile-uniform */
     const uint64_t k2 = __shfl((unsigned long long)key, src);
@@ -593,15 +596,15 @@ __device__ __forceinline__ void settle_reprobes(const View& v, uint64_t key, uin
  * the plain scan would pick and wait for without end.  Whether a key is
  * refused at score == min is a separate switch (UpsertArgs::refuse_equal).
  */
-/* WAVES wavefronts per workgroup, each with its own 64 keys and its own staging area.  One
- * everywhere except insert_and_evict on a table that is about full, whose wavefronts claim their
- * part of the evicted-keys output together: updates of one word are served one at a time, about
+/* WAVES wavefronts per workgroup, each with its own 8 R keys and its own staging area.  One
+ * everywhere except insert_and_evict on a table that is about full, where the wavefronts of 128 keys
+ * claim their part of the evicted-keys output together: updates of one word are served one at a time, about
  * 15 ns each, and one per wavefront and trip (some 24 thousand for 2^20 keys into full buckets)
  * took 0.07 ms of the call's 0.46.  (While buckets have free slots there is nothing to claim,
  * and two wavefronts that wait for each other in every trip are 4 % slower than one.) */
-template <int OP, int VEC, int UPL, bool LOCKED_RULE, bool BOUNDS = false, int WAVES = 1, bool HOLD = false>
+template <int OP, int VEC, int UPL, bool LOCKED_RULE, bool BOUNDS = false, int WAVES = 1, bool HOLD = false, int R = kTile>
 __global__ void __launch_bounds__(kWave * WAVES)
-    __attribute__((amdgpu_waves_per_eu(BOUNDS ? 4 : 1)))
+    __attribute__((amdgpu_waves_per_eu(BOUNDS && R == kTile ? 4 : 1)))
 upsert_kernel(View v, UpsertArgs a) {
   static_assert(!(BOUNDS && LOCKED_RULE), "the bounded search does not look at key words");
   static_assert(WAVES == 1 || OP == kOpInsertAndEvict, "only insert_and_evict has anything to share");
@@ -623,7 +626,7 @@ upsert_kernel(View v, UpsertArgs a) {
   uint16_t (*const s_em)[kTile] = s_em_all[wave];
   uint8_t* const s_unsure = s_unsure_all[wave];
   const int tile = lane >> 3, j = lane & 7;
-  const uint64_t i = ((uint64_t)blockIdx.x * WAVES + wave) * kWave + lane;
+  const uint64_t i = lane_owns_key<R>(lane) ? key_of_lane<R>((uint64_t)blockIdx.x * WAVES + wave, lane) : a.n;
   const uint32_t units = v.value_bytes / VEC;
 
   uint64_t bound_cap = 0, bound_ceil = 0;
@@ -645,7 +648,7 @@ upsert_kernel(View v, UpsertArgs a) {
   const uint64_t in_score = (a.scores && i < a.n) ? a.scores[i] : 0;
   s_unsure[lane] = 0;
   __syncthreads();
-  probe_wave<true, kTwoStepWriters>(v, s_meta, s_slot, s_em, s_unsure, lane);
+  probe_wave<true, kTwoStepWriters, R>(v, s_meta, s_slot, s_em, s_unsure, lane);
   __syncthreads();
 
   /* ---- state of the key this lane owns ---------------------------------------------- */
@@ -683,7 +686,7 @@ upsert_kernel(View v, UpsertArgs a) {
   if (HOLD || (OP == kOpFindOrInsertPtr && a.locked_key_ptrs != nullptr)) waited = kMaxLockedWaits;
   for (int trip = 0; more; trip++) {
     if (__ballot(pending && reprobe))
-      settle_reprobes(v, key, me.bkt, digest, pending, reprobe, hit, em_lo, em_hi, waited, lane);
+      settle_reprobes<R>(v, key, me.bkt, digest, pending, reprobe, hit, em_lo, em_hi, waited, lane);
 
     bool active = pending && !reprobe;
     if constexpr (OP == kOpAccumOrAssign) {
@@ -719,20 +722,21 @@ upsert_kernel(View v, UpsertArgs a) {
       /* the bounds of four buckets, then the most promising score line of each, in flight */
       const uint32_t need = tile_ballot(want_scan, tile);
       const int lane_base = lane & ~(kTile - 1);
+      constexpr int kQ = R < 4 ? R : 4;
 #pragma unroll
-      for (int h = 0; h < kTile; h += 4) {
-        if (!__ballot(((need >> h) & 0xFu) != 0)) continue;
-        uint64_t bs[4], bd[4];
-        uint32_t g[4];
-        uint4 x[4];
+      for (int h = 0; h < R; h += kQ) {
+        if (!__ballot(((need >> h) & ((1u << kQ) - 1)) != 0)) continue;
+        uint64_t bs[kQ], bd[kQ];
+        uint32_t g[kQ];
+        uint4 x[kQ];
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
+        for (int q = 0; q < kQ; q++) {
           bs[q] = __shfl((unsigned long long)bslot, lane_base + h + q);
           bd[q] = kMaxScore;
           if ((need >> (h + q)) & 1u) bd[q] = ld_u64(v.bounds + (bs[q] >> 4) + j);
         }
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
+        for (int q = 0; q < kQ; q++) {
           uint64_t b = bd[q];
           uint32_t gi = (uint32_t)j;
           tile_min_pair(b, gi);
@@ -741,7 +745,7 @@ upsert_kernel(View v, UpsertArgs a) {
           if ((need >> (h + q)) & 1u) x[q] = line_load(v, bs[q], g[q], j);
         }
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
+        for (int q = 0; q < kQ; q++) {
           if ((need >> (h + q)) & 1u) {
             uint64_t b0, nb0;
             uint32_t p0;
@@ -936,7 +940,7 @@ upsert_kernel(View v, UpsertArgs a) {
           a.evicted_keys[idx] = refused_now ? key : victim;
           if (a.evicted_scores) a.evicted_scores[idx] = refused_now ? desired : best;
         }
-        bulk_evicted<VEC, UPL>(emit ? (refused_now ? 1 : 2) : 0,
+        bulk_evicted<VEC, UPL, R>(emit ? (refused_now ? 1 : 2) : 0,
                                refused_now ? a.values_in + i * v.value_bytes : row,
                                a.evicted_values + idx * v.value_bytes, units, lane);
       }
@@ -957,7 +961,7 @@ upsert_kernel(View v, UpsertArgs a) {
         }
       }
       if (__ballot(move != kMoveNone))
-        bulk_rows<VEC, UPL, OP == kOpFindOrInsert, OP == kOpAccumOrAssign>(
+        bulk_rows<VEC, UPL, OP == kOpFindOrInsert, OP == kOpAccumOrAssign, R>(
             move, row, usr, units, a.value_kind, lane);
     }
 

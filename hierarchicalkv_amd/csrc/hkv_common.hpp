@@ -358,6 +358,26 @@ __device__ __forceinline__ typename VecType<VEC>::type load_row_unit(const uint8
     return *reinterpret_cast<const typename VecType<VEC>::type*>(p);
   }
 }
+/* The same unit to an address. */
+template <int VEC>
+__device__ __forceinline__ void store_row_unit(uint8_t* p, typename VecType<VEC>::type x) {
+  if constexpr (vec_bytes(VEC) == 16) {
+    const u32x4_t t = {x.x, x.y, x.z, x.w};
+    if constexpr (VEC >= kAny)
+      __builtin_nontemporal_store(t, reinterpret_cast<u32x4_any_t*>(p));
+    else
+      __builtin_nontemporal_store(t, reinterpret_cast<u32x4_t*>(p));
+  } else if constexpr (VEC == kAny + 8) {
+    const u32x2_any_t t = {x.x, x.y};
+    *reinterpret_cast<u32x2_any_t*>(p) = t;
+  } else if constexpr (VEC == kAny + 4) {
+    *reinterpret_cast<u32_any_t*>(p) = x;
+  } else if constexpr (VEC == kAny + 2) {
+    *reinterpret_cast<u16_any_t*>(p) = x;
+  } else {
+    *reinterpret_cast<typename VecType<VEC>::type*>(p) = x;
+  }
+}
 /* The same unit to byte `offset` of a buffer resource; an offset past its end stores nothing. */
 template <int VEC>
 __device__ __forceinline__ void store_row_unit(__amdgpu_buffer_rsrc_t dst, uint32_t offset,

@@ -151,7 +151,7 @@ upsert_hits_kernel(View v, UpsertArgs a, ChainArgs h) {
       if (idx < total) {
         const uint32_t kk = pow2 ? (idx >> sh) : (idx / units);
         const uint32_t c = idx - kk * units;
-        if (s_slot[kk] >= 0) buf[b] = ld_unit<VEC, false>(usr_base + (uint64_t)kk * v.value_bytes, c);
+        if (s_slot[kk] >= 0) buf[b] = ld_unit<VEC, false>(usr_base + (uint64_t)kk * v.value_bytes + c * VEC);
       }
     }
 #pragma unroll
@@ -161,7 +161,7 @@ upsert_hits_kernel(View v, UpsertArgs a, ChainArgs h) {
         const uint32_t kk = pow2 ? (idx >> sh) : (idx / units);
         const uint32_t c = idx - kk * units;
         const int64_t sl = s_slot[kk];
-        if (sl >= 0) st_unit<VEC, true>(value_row(v, (uint64_t)sl), c, buf[b]);
+        if (sl >= 0) st_unit<VEC, true>(value_row(v, (uint64_t)sl) + c * VEC, buf[b]);
       }
     }
   }
@@ -314,7 +314,7 @@ __device__ __forceinline__ void group_bucket(const View& v, const UpsertArgs& a,
         for (int w = 0; w < UPL; w++) {
           const uint32_t u = j + w * kTile;
           xin[q][w] = T{};
-          if (q < mg && u < units) xin[q][w] = ld_unit<VEC, false>(us, u);
+          if (q < mg && u < units) xin[q][w] = ld_unit<VEC, false>(us + u * VEC);
         }
       }
     }
@@ -464,7 +464,7 @@ __device__ __forceinline__ void group_bucket(const View& v, const UpsertArgs& a,
 #pragma unroll
         for (int w = 0; w < UPL; w++) {
           const uint32_t u = j + w * kTile;
-          if (u < units) st_unit<VEC, true>(tb, u, xin[q][w]);
+          if (u < units) st_unit<VEC, true>(tb + u * VEC, xin[q][w]);
         }
       } else {
         const uint8_t* us = rows_in + (uint64_t)s_idx[q0 + q] * v.value_bytes;
@@ -474,12 +474,12 @@ __device__ __forceinline__ void group_bucket(const View& v, const UpsertArgs& a,
           for (int w = 0; w < UPL; w++) {
             const uint32_t u = u0 + j + w * kTile;
             x[w] = T{};
-            if (u < units) x[w] = ld_unit<VEC, false>(us, u);
+            if (u < units) x[w] = ld_unit<VEC, false>(us + u * VEC);
           }
 #pragma unroll
           for (int w = 0; w < UPL; w++) {
             const uint32_t u = u0 + j + w * kTile;
-            if (u < units) st_unit<VEC, true>(tb, u, x[w]);
+            if (u < units) st_unit<VEC, true>(tb + u * VEC, x[w]);
           }
         }
       }

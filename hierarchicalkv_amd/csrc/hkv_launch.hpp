@@ -33,14 +33,12 @@ void launch_main(void (*kernel)(KArgs...), dim3 grid, dim3 block, hipStream_t s,
 
 inline unsigned grid_for(uint64_t n) { return (unsigned)((n + kWave - 1) / kWave); }
 
-/* units per lane that the bulk copy keeps in registers: rows of up to 8 * UPL
- * units go through in one pass (16-byte units: 128, 256, 512, 1024 bytes) */
-inline int pick_upl(uint32_t value_bytes, int vec) {
-  if (vec != 16) return 8;
-  const uint32_t units = value_bytes / 16;
-  if (units <= 8) return 1;
-  if (units <= 16) return 2;
-  if (units <= 32) return 4;
+/* 16-byte units per lane that the bulk copy keeps in registers: rows of up to 8 * UPL units (128, 256,
+ * 512, 1024 bytes) go through in one pass */
+inline int pick_upl(uint32_t value_bytes) {
+  if (value_bytes <= 128) return 1;
+  if (value_bytes <= 256) return 2;
+  if (value_bytes <= 512) return 4;
   return 8;
 }
 

@@ -10,7 +10,7 @@ template <bool LOCKFREE>
 void launch_assign_by(int vec, const View& v, const AssignArgs& a, hipStream_t s) {
   const dim3 grid(grid_for(a.n)), block(kWave);
   if (vec == 16) {
-    switch (pick_upl(v.value_bytes, 16)) {
+    switch (pick_upl(v.value_bytes)) {
       case 1: hipLaunchKernelGGL((assign_kernel<16, 1, LOCKFREE>), grid, block, 0, s, v, a); break;
       case 2: hipLaunchKernelGGL((assign_kernel<16, 2, LOCKFREE>), grid, block, 0, s, v, a); break;
       case 4: hipLaunchKernelGGL((assign_kernel<16, 4, LOCKFREE>), grid, block, 0, s, v, a); break;

@@ -7,40 +7,37 @@ namespace hkv {
 namespace {
 
 /* BOUNDS: the victim search reads the bucket's score bounds and one or two of its score lines
- * instead of all eight (hkv_upsert.hpp); for 16-byte units, which is what tables with rows of a
- * multiple of 16 bytes use.
- * R: keys per tile (hkv_lookup.hpp). */
+ * instead of all eight (hkv_upsert.hpp).
+ * R: keys per tile (hkv_lookup.hpp).
+ * vec: accum_or_assign adds in units of whole elements (accum_unit); the others move rows of 16 bytes
+ * and more in 16-byte units at any address, shorter ones in one or two units of the widest power of
+ * two that fits (lookup_unit). */
 template <int OP, int R, bool LOCKED_RULE, bool BOUNDS = false, int WAVES = 1, bool HOLD = false>
 void launch_form(int vec, const View& v, const UpsertArgs& a, hipStream_t s) {
   constexpr uint64_t kKeys = (uint64_t)kTilesPerWave * R * WAVES;
   const dim3 grid((unsigned)((a.n + kKeys - 1) / kKeys)), block(kWave * WAVES);
-  if constexpr (OP == kOpAccumOrAssign && !BOUNDS) {
-    /* the two units that only the element-wise add needs */
-    if (vec == 8) {
-      launch_main(upsert_kernel<OP, 8, 8, LOCKED_RULE, false, WAVES, HOLD, R>, grid, block, s, v, a);
-      return;
-    }
-    if (vec == 2) {
-      launch_main(upsert_kernel<OP, 2, 8, LOCKED_RULE, false, WAVES, HOLD, R>, grid, block, s, v, a);
-      return;
-    }
-  }
-  if (OP == kOpFindOrInsertPtr) {
+  if constexpr (OP == kOpFindOrInsertPtr) {
     launch_main(upsert_kernel<OP, 16, 1, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a);
     return;
   }
-  if (vec == 16) {
-    switch (pick_upl(v.value_bytes, 16)) {
-      case 1: launch_main(upsert_kernel<OP, 16, 1, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
-      case 2: launch_main(upsert_kernel<OP, 16, 2, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
-      case 4: launch_main(upsert_kernel<OP, 16, 4, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
-      default: launch_main(upsert_kernel<OP, 16, 8, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+  constexpr bool kAdds = OP == kOpAccumOrAssign;
+  constexpr int kWide = kAdds ? 16 : kAny + 16;
+  constexpr int kNarrowUpl = kAdds ? 8 : 1; /* the others' rows have no more than two units of less than 16 bytes */
+  if (vec_bytes(vec) == 16) {
+    switch (pick_upl(v.value_bytes)) {
+      case 1: launch_main(upsert_kernel<OP, kWide, 1, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+      case 2: launch_main(upsert_kernel<OP, kWide, 2, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+      case 4: launch_main(upsert_kernel<OP, kWide, 4, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+      default: launch_main(upsert_kernel<OP, kWide, 8, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
     }
-  } else if constexpr (!BOUNDS) {
-    if (vec == 4)
-      launch_main(upsert_kernel<OP, 4, 8, LOCKED_RULE, false, WAVES, HOLD, R>, grid, block, s, v, a);
-    else
-      launch_main(upsert_kernel<OP, 1, 8, LOCKED_RULE, false, WAVES, HOLD, R>, grid, block, s, v, a);
+    return;
+  }
+  constexpr int kNarrow = kAdds ? 0 : kAny;
+  switch (vec_bytes(vec)) {
+    case 8: launch_main(upsert_kernel<OP, kNarrow + 8, kNarrowUpl, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+    case 4: launch_main(upsert_kernel<OP, kNarrow + 4, kNarrowUpl, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+    case 2: launch_main(upsert_kernel<OP, kNarrow + 2, kNarrowUpl, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+    default: launch_main(upsert_kernel<OP, 1, kNarrowUpl, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
   }
 }
 

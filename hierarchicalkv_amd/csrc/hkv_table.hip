@@ -317,7 +317,7 @@ int accum_unit(uint32_t value_bytes, const void* p, int kind) {
 template <template <int, int> class Launcher, class... Args>
 void dispatch_vec_upl(int vec, uint32_t value_bytes, Args&&... args) {
   if (vec == 16) {
-    switch (pick_upl(value_bytes, 16)) {
+    switch (pick_upl(value_bytes)) {
       case 1: Launcher<16, 1>::go(args...); break;
       case 2: Launcher<16, 2>::go(args...); break;
       case 4: Launcher<16, 4>::go(args...); break;
@@ -658,10 +658,9 @@ uint64_t host_realtime_ns() {
 /* Whether this upsert searches victims through the score bounds, and with which limits (the
  * fields of `a`); launches what has to run first (the batch's lowest score, the rebuild).  The
  * caller holds the inserter role on `s`. */
-template <int OP>
-bool prepare_bounds(hkv_table* t, UpsertArgs& a, int vec, hipStream_t s) {
+bool prepare_bounds(hkv_table* t, UpsertArgs& a, hipStream_t s) {
   const int st = t->opts.evict_strategy;
-  if (!t->score_bounds || a.strategy != st || !(vec == 16 || OP == kOpFindOrInsertPtr)) return false;
+  if (!t->score_bounds || a.strategy != st) return false;
   /* The bounded search pays once buckets are full; a table that cannot be nine tenths full yet (it
    * has not been offered that many keys since it was created or cleared) takes the plain kernel. */
   if (t->keys_offered * 10 < t->view.capacity * 9) return false;
@@ -774,7 +773,7 @@ int run_upsert(hkv_table* t, UpsertArgs a, int vec, bool hybrid_rule, hipStream_
        * the batch is retried instead of skipped) */
       writes_scores_outside_bounds(t, s, own_rule);
       launch_upsert<OP>({true, false, pair, repeats}, vec, t->view, a, s);
-    } else if (prepare_bounds<OP>(t, a, vec, s)) {
+    } else if (prepare_bounds(t, a, s)) {
       launch_upsert<OP>({false, true, pair, repeats}, vec, t->view, a, s);
     } else {
       writes_scores_outside_bounds(t, s, own_rule);
@@ -985,7 +984,7 @@ void launch_dual_upsert(int vec, const View& v, const UpsertArgs& whole, hipStre
   }
 }
 
-/* unit of the row copies of a lookup: 16 bytes where rows and pointer allow it, else the widest unit
+/* unit of the row copies of a lookup or an upsert: 16 bytes where rows and pointer allow it, else the widest unit
  * that fits into a row, at any address */
 int lookup_unit(uint32_t value_bytes, const void* out) {
   if (((value_bytes | (uintptr_t)out) & 15) == 0) return 16;
@@ -1254,7 +1253,6 @@ int hkv_insert_or_assign(hkv_table* t, uint64_t n, const uint64_t* keys,
   a.scores = scores;
   a.n = n;
   a.strategy = strategy;
-  const int vec = pick_vec(t->view.value_bytes, {values});
   if (t->dual) {
     /* merlin_hashtable.cuh:1166-1190 */
     if (!unique_key)
@@ -1267,7 +1265,7 @@ int hkv_insert_or_assign(hkv_table* t, uint64_t n, const uint64_t* keys,
     {
       LockGuard g(t, StreamGroupLock::kInserter, s);
       HKV_HIP(g.acquire());
-      launch_dual_upsert(vec, t->view, a, s);
+      launch_dual_upsert(pick_vec(t->view.value_bytes, {values}), t->view, a, s);
       HKV_HIP(hipGetLastError());
     }
     if (t->clock.mode == 1) t->clock.base += UINT64_C(1) << 40;
@@ -1276,6 +1274,7 @@ int hkv_insert_or_assign(hkv_table* t, uint64_t n, const uint64_t* keys,
   if (t->io_by_cpu) return cpu_io_upsert(t, a, const_cast<void*>(values), false, (hipStream_t)stream);
   /* with unique_key == false the reference leaves its lock-key kernels for the plain one
    * (merlin_hashtable.cuh:1235-1258), whose rule is "refuse when score < min" */
+  const int vec = lookup_unit(t->view.value_bytes, values);
   return run_upsert<kOpInsertOrAssign>(t, a, vec, unique_key != 0, (hipStream_t)stream, !unique_key);
 }
 
@@ -1366,7 +1365,7 @@ int hkv_insert_and_evict(hkv_table* t, uint64_t n, const uint64_t* keys,
   a.evicted_counter = (unsigned long long*)d_evicted_counter;
   a.n = n;
   a.strategy = strategy;
-  const int vec = pick_vec(t->view.value_bytes, {values, evicted_values});
+  const int vec = lookup_unit(t->view.value_bytes, values);
   return run_upsert<kOpInsertAndEvict>(t, a, vec, false, (hipStream_t)stream, !unique_key);
 }
 
@@ -1425,7 +1424,7 @@ int hkv_find_or_insert(hkv_table* t, uint64_t n, const uint64_t* keys,
   a.scores = scores;
   a.n = n;
   a.strategy = strategy;
-  const int vec = pick_vec(t->view.value_bytes, {values});
+  const int vec = lookup_unit(t->view.value_bytes, values);
   if (t->io_by_cpu)
     HKV_TRY(cpu_io_upsert(t, a, values, true, (hipStream_t)stream));
   else /* merlin_hashtable.cuh:1779-1803: lock-key kernels only with unique keys */

@@ -203,59 +203,46 @@ __device__ __forceinline__ uint8_t add_unit(uint8_t x, uint8_t y, int) {
   return (uint8_t)(x + y); /* i8 */
 }
 
-/* One VEC-byte unit of a row.  Table rows are read and written coherently
- * (agent-scope accesses: 2 x 8 bytes per 16-byte unit on the load side, one
- * 16-byte write-through store on the store side), caller buffers plainly. */
-template <int VEC, bool TABLE>
-__device__ __forceinline__ typename VecType<VEC>::type ld_unit(const uint8_t* row, uint32_t u) {
-  using T = typename VecType<VEC>::type;
-  if constexpr (!TABLE) {
-    if constexpr (VEC == 16) {
-      /* a caller's row is read once: streaming load, so that it does not push table
-       * lines out of the caches */
-      const u32x4_t t = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(row) + u);
-      return make_uint4(t.x, t.y, t.z, t.w);
-    } else {
-      return reinterpret_cast<const T*>(row)[u];
-    }
-  } else if constexpr (VEC == 16) {
-    const uint64_t* p = reinterpret_cast<const uint64_t*>(row) + 2 * u;
-    const uint64_t lo = ld_u64(p), hi = ld_u64(p + 1);
+/* One unit of a row at p.  Table rows are written coherently (agent scope: one 16-byte write-through
+ * store), and read so where another wavefront of the launch may have written them (COHERENT: 2 x 8
+ * bytes per 16-byte unit); caller buffers are accessed plainly, and streaming where the unit is wide:
+ * a caller's row is touched once and should not push table lines out of the caches. */
+template <int VEC, bool COHERENT>
+__device__ __forceinline__ typename VecType<VEC>::type ld_unit(const uint8_t* p) {
+  constexpr int w = vec_bytes(VEC);
+  if constexpr (!COHERENT) {
+    return load_row_unit<VEC>(p);
+  } else if constexpr (w == 16) {
+    const uint64_t* q = reinterpret_cast<const uint64_t*>(p);
+    const uint64_t lo = ld_u64(q), hi = ld_u64(q + 1);
     return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
-  } else if constexpr (VEC == 8) {
-    const uint64_t x = ld_u64(reinterpret_cast<const uint64_t*>(row) + u);
+  } else if constexpr (w == 8) {
+    const uint64_t x = ld_u64(reinterpret_cast<const uint64_t*>(p));
     return make_uint2((uint32_t)x, (uint32_t)(x >> 32));
-  } else if constexpr (VEC == 4) {
-    return ld_u32(reinterpret_cast<const uint32_t*>(row) + u);
-  } else if constexpr (VEC == 2) {
-    return __hip_atomic_load(reinterpret_cast<const uint16_t*>(row) + u, __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
+  } else if constexpr (w == 4) {
+    return ld_u32(reinterpret_cast<const uint32_t*>(p));
+  } else if constexpr (w == 2) {
+    return __hip_atomic_load(reinterpret_cast<const uint16_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   } else {
-    return ld_u8(row + u);
+    return ld_u8(p);
   }
 }
+/* to a table row (TABLE) or a caller's */
 template <int VEC, bool TABLE>
-__device__ __forceinline__ void st_unit(uint8_t* row, uint32_t u, typename VecType<VEC>::type x) {
-  using T = typename VecType<VEC>::type;
+__device__ __forceinline__ void st_unit(uint8_t* p, typename VecType<VEC>::type x) {
+  constexpr int w = vec_bytes(VEC);
   if constexpr (!TABLE) {
-    if constexpr (VEC == 16) {
-      /* written once, not read again by this kernel: streaming store */
-      const u32x4_t t = {x.x, x.y, x.z, x.w};
-      __builtin_nontemporal_store(t, reinterpret_cast<u32x4_t*>(row) + u);
-    } else {
-      reinterpret_cast<T*>(row)[u] = x;
-    }
-  } else if constexpr (VEC == 16) {
-    st_u128(row + 16 * (size_t)u, x);
-  } else if constexpr (VEC == 8) {
-    st_u64(reinterpret_cast<uint64_t*>(row) + u, x.x | ((uint64_t)x.y << 32));
-  } else if constexpr (VEC == 4) {
-    st_u32(reinterpret_cast<uint32_t*>(row) + u, x);
-  } else if constexpr (VEC == 2) {
-    __hip_atomic_store(reinterpret_cast<uint16_t*>(row) + u, x, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+    store_row_unit<VEC>(p, x);
+  } else if constexpr (w == 16) {
+    st_u128(p, x);
+  } else if constexpr (w == 8) {
+    st_u64(reinterpret_cast<uint64_t*>(p), x.x | ((uint64_t)x.y << 32));
+  } else if constexpr (w == 4) {
+    st_u32(reinterpret_cast<uint32_t*>(p), x);
+  } else if constexpr (w == 2) {
+    __hip_atomic_store(reinterpret_cast<uint16_t*>(p), x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   } else {
-    st_u8(row + u, x);
+    st_u8(p, x);
   }
 }
 
@@ -436,12 +423,14 @@ constexpr int kRowUnits = 8;
  * first store; a group holds 16 units per lane (64 VGPRs at 16-byte units),
  * i.e. the whole trip for rows up to 256 bytes.
  * UPL = units per lane and row held in registers (1, 2, 4 or 8).
+ * Units may overlap within a row (kAny) where rows are moved as they are, not where they are added to.
  * Every lane of the wavefront must call this.
  */
 template <int VEC, int UPL, bool CAN_READ_TABLE, bool CAN_ACCUM, int R = kTile>
 __device__ __forceinline__ void bulk_rows(int move, uint8_t* tab, uint8_t* usr,
-                                          uint32_t units, int value_kind, int lane) {
+                                          uint32_t bytes, int value_kind, int lane) {
   using T = typename VecType<VEC>::type;
+  const uint32_t units = row_units<VEC>(bytes);
   /* accumulating holds two rows per key (the table's and the caller's): half as many keys at a time */
   constexpr int kUnits = CAN_ACCUM ? kRowUnits / 2 : kRowUnits;
   constexpr int kGroup = kUnits / UPL < 1 ? 1 : (kUnits / UPL < R ? kUnits / UPL : R);
@@ -461,16 +450,17 @@ __device__ __forceinline__ void bulk_rows(int move, uint8_t* tab, uint8_t* usr,
 #pragma unroll
         for (int w = 0; w < UPL; w++) {
           const uint32_t u = u0 + j + w * kTile;
+          const uint32_t at = unit_offset<VEC>(u, bytes);
           x[q][w] = T{};
           if (u < units) {
-            if (mv == kMoveInToTable) x[q][w] = ld_unit<VEC, false>(us, u);
+            if (mv == kMoveInToTable) x[q][w] = ld_unit<VEC, false>(us + at);
             /* the row of a key that was found was last written before this launch (keys are
              * unique, so no other key of the batch has touched it): an ordinary streaming
              * load, one 16-byte access instead of the two 8-byte coherent ones */
-            if (CAN_READ_TABLE && mv == kMoveTableToIo) x[q][w] = ld_unit<VEC, false>(tb, u);
+            if (CAN_READ_TABLE && mv == kMoveTableToIo) x[q][w] = ld_unit<VEC, false>(tb + at);
             if (CAN_ACCUM && mv == kMoveAccum) {
-              x[q][w] = ld_unit<VEC, false>(tb, u);
-              y[q][w] = ld_unit<VEC, false>(us, u);
+              x[q][w] = ld_unit<VEC, false>(tb + at);
+              y[q][w] = ld_unit<VEC, false>(us + at);
             }
           }
         }
@@ -484,11 +474,12 @@ __device__ __forceinline__ void bulk_rows(int move, uint8_t* tab, uint8_t* usr,
 #pragma unroll
         for (int w = 0; w < UPL; w++) {
           const uint32_t u = u0 + j + w * kTile;
+          const uint32_t at = unit_offset<VEC>(u, bytes);
           if (u < units) {
-            if (mv == kMoveInToTable) st_unit<VEC, true>(tb, u, x[q][w]);
-            if (CAN_READ_TABLE && mv == kMoveTableToIo) st_unit<VEC, false>(us, u, x[q][w]);
+            if (mv == kMoveInToTable) st_unit<VEC, true>(tb + at, x[q][w]);
+            if (CAN_READ_TABLE && mv == kMoveTableToIo) st_unit<VEC, false>(us + at, x[q][w]);
             if (CAN_ACCUM && mv == kMoveAccum)
-              st_unit<VEC, true>(tb, u, add_unit(x[q][w], y[q][w], value_kind));
+              st_unit<VEC, true>(tb + at, add_unit(x[q][w], y[q][w], value_kind));
           }
         }
       }
@@ -500,8 +491,9 @@ __device__ __forceinline__ void bulk_rows(int move, uint8_t* tab, uint8_t* usr,
  * (coherent read), kind 1 = the refused key's input row, 0 = nothing. */
 template <int VEC, int UPL, int R>
 __device__ __forceinline__ void bulk_evicted(int kind, const uint8_t* src, uint8_t* dst,
-                                             uint32_t units, int lane) {
+                                             uint32_t bytes, int lane) {
   using T = typename VecType<VEC>::type;
+  const uint32_t units = row_units<VEC>(bytes);
   constexpr int kGroup = kRowUnits / UPL < 1 ? 1 : (kRowUnits / UPL < R ? kRowUnits / UPL : R);
   const int j = lane & (kTile - 1);
   const int lane_base = lane & ~(kTile - 1);
@@ -517,10 +509,11 @@ __device__ __forceinline__ void bulk_evicted(int kind, const uint8_t* src, uint8
 #pragma unroll
         for (int w = 0; w < UPL; w++) {
           const uint32_t u = u0 + j + w * kTile;
+          const uint32_t at = unit_offset<VEC>(u, bytes);
           x[q][w] = T{};
           if (u < units) {
-            if (kd == 2) x[q][w] = ld_unit<VEC, true>(sp, u);
-            if (kd == 1) x[q][w] = ld_unit<VEC, false>(sp, u);
+            if (kd == 2) x[q][w] = ld_unit<VEC, true>(sp + at);
+            if (kd == 1) x[q][w] = ld_unit<VEC, false>(sp + at);
           }
         }
       }
@@ -532,7 +525,8 @@ __device__ __forceinline__ void bulk_evicted(int kind, const uint8_t* src, uint8
 #pragma unroll
         for (int w = 0; w < UPL; w++) {
           const uint32_t u = u0 + j + w * kTile;
-          if (u < units && kd) st_unit<VEC, false>(dp, u, x[q][w]);
+          const uint32_t at = unit_offset<VEC>(u, bytes);
+          if (u < units && kd) st_unit<VEC, false>(dp + at, x[q][w]);
         }
       }
     }
@@ -627,7 +621,6 @@ upsert_kernel(View v, UpsertArgs a) {
   uint8_t* const s_unsure = s_unsure_all[wave];
   const int tile = lane >> 3, j = lane & 7;
   const uint64_t i = lane_owns_key<R>(lane) ? key_of_lane<R>((uint64_t)blockIdx.x * WAVES + wave, lane) : a.n;
-  const uint32_t units = v.value_bytes / VEC;
 
   uint64_t bound_cap = 0, bound_ceil = 0;
   if constexpr (BOUNDS) {
@@ -942,7 +935,7 @@ upsert_kernel(View v, UpsertArgs a) {
         }
         bulk_evicted<VEC, UPL, R>(emit ? (refused_now ? 1 : 2) : 0,
                                refused_now ? a.values_in + i * v.value_bytes : row,
-                               a.evicted_values + idx * v.value_bytes, units, lane);
+                               a.evicted_values + idx * v.value_bytes, v.value_bytes, lane);
       }
     }
     if (OP != kOpFindOrInsertPtr) {
@@ -962,7 +955,7 @@ upsert_kernel(View v, UpsertArgs a) {
       }
       if (__ballot(move != kMoveNone))
         bulk_rows<VEC, UPL, OP == kOpFindOrInsert, OP == kOpAccumOrAssign, R>(
-            move, row, usr, units, a.value_kind, lane);
+            move, row, usr, v.value_bytes, a.value_kind, lane);
     }
 
     /* ---- step 5: everything written under the locks is out; release them --------------------------- */
@@ -1045,7 +1038,6 @@ assign_kernel(View v, AssignArgs a) {
   __shared__ uint8_t s_unsure[kWave];
   const int lane = threadIdx.x;
   const uint64_t i = (uint64_t)blockIdx.x * kWave + lane;
-  const uint32_t units = v.value_bytes / VEC;
   const uint64_t bound_ceil = a.bound_ceil ? *a.bound_ceil : 0;
   const uint64_t key = stage_keys(v, a.keys, a.n, i, s_meta, s_slot, lane);
   s_unsure[lane] = 0;
@@ -1089,7 +1081,7 @@ assign_kernel(View v, AssignArgs a) {
       const int move = locked ? kMoveInToTable : kMoveNone;
       uint8_t* usr = const_cast<uint8_t*>(a.values) + i * v.value_bytes;
       if (__ballot(move != kMoveNone))
-        bulk_rows<VEC, UPL, false, false>(move, row, usr, units, 0, lane);
+        bulk_rows<VEC, UPL, false, false>(move, row, usr, v.value_bytes, 0, lane);
     }
     if (!LOCKFREE) {
       wait_stores();

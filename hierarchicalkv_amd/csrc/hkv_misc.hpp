@@ -165,21 +165,42 @@ rehash_kernel(View src, View dst) {
   }
 }
 
-/* keys in the first n buckets (fast_load_factor, merlin_hashtable.cuh:3796-3830); one workgroup,
- * which stores its whole result in one write */
-__global__ void __launch_bounds__(256)
+/* keys in the first n buckets (fast_load_factor, merlin_hashtable.cuh:3796-3830), n at most 1024; one
+ * workgroup, all of whose loads are in flight together, and which stores its whole result in one
+ * write to a word of host memory.  Bound by the latency of one load and of the launch: 256 threads
+ * that went through the sample in 32 dependent steps took 11 to 14 us. */
+constexpr int kSampleThreads = 1024;
+constexpr int kSampleLoads = 1024 * (kBucketSize / 16) / kSampleThreads; /* per thread */
+__global__ void __launch_bounds__(kSampleThreads)
 load_sample_kernel(View v, uint32_t n, unsigned long long* out) {
-  __shared__ unsigned long long s_part[4];
-  unsigned long long local = 0;
+  __shared__ uint32_t s_part[kSampleThreads / kWave];
   const uint32_t e4 = v.empty_digest * 0x01010101u;
   const uint4* d = reinterpret_cast<const uint4*>(v.digests);
-  for (uint32_t g = threadIdx.x; g < n * (kBucketSize / 16); g += 256) local += 16 - __popc(match16(d[g], e4));
+  const uint32_t groups = n * (kBucketSize / 16);
+  uint4 x[kSampleLoads];
+#pragma unroll
+  for (int k = 0; k < kSampleLoads; k++) {
+    const uint32_t g = k * kSampleThreads + threadIdx.x;
+    x[k] = g < groups ? d[g] : make_uint4(e4, e4, e4, e4);
+  }
+  uint32_t local = 0;
+#pragma unroll
+  for (int k = 0; k < kSampleLoads; k++) local += 16 - __popc(match16(x[k], e4));
   for (int off = 32; off > 0; off >>= 1) local += __shfl_xor(local, off);
-  if ((threadIdx.x & 63) == 0) s_part[threadIdx.x >> 6] = local;
+  if ((threadIdx.x & (kWave - 1)) == 0) s_part[threadIdx.x / kWave] = local;
   __syncthreads();
-  if (threadIdx.x == 0) *out = s_part[0] + s_part[1] + s_part[2] + s_part[3];
+  if (threadIdx.x == 0) {
+    unsigned long long total = 0;
+    for (int w = 0; w < kSampleThreads / kWave; w++) total += s_part[w];
+    __hip_atomic_store(out, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  }
 }
 
+/* the value of a device word goes to a word of host memory and the device word back to 0 */
+__global__ void report_word_kernel(unsigned long long* word, unsigned long long* host) {
+  __hip_atomic_store(host, *word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+  *word = 0;
+}
 __global__ void zero_u64_kernel(unsigned long long* p) { *p = 0; }
 /* the table's count of LOCKED slots, all its words (one thread each) */
 __global__ void zero_locked_kernel(unsigned long long* count) { count[threadIdx.x * kLockedStride] = 0; }

@@ -43,23 +43,24 @@ __global__ void clock_sample_kernel(unsigned long long* out) { *out = wall_clock
  * wavefronts may count it twice).  Otherwise the slot changes hands with a compare-and-swap.
  * A key that an 8-lane tile holds twice is erased once.  No counter is kept per bucket (the
  * number of keys of a table is the number of digests that are not the EMPTY marker, counted
- * when somebody asks), so an erase is two stores. */
-template <bool EXCLUSIVE>
+ * when somebody asks), so an erase is two stores.
+ * R: keys per tile (hkv_lookup.hpp). */
+template <bool EXCLUSIVE, int R>
 __global__ void __launch_bounds__(kWave)
 erase_kernel(View v, const uint64_t* keys, uint64_t n) {
   __shared__ KeyMeta s_meta[kWave];
   __shared__ int64_t s_slot[kWave];
   const int lane = threadIdx.x;
-  const uint64_t i = (uint64_t)blockIdx.x * kWave + lane;
+  const uint64_t i = lane_owns_key<R>(lane) ? key_of_lane<R>(blockIdx.x, lane) : n;
   const uint64_t key = stage_keys(v, keys, n, i, s_meta, s_slot, lane);
   __syncthreads();
-  probe_wave<false, false>(v, s_meta, s_slot, nullptr, nullptr, lane);
+  probe_wave<false, false, R>(v, s_meta, s_slot, nullptr, nullptr, lane);
   __syncthreads();
   const int64_t slot = s_slot[lane];
   const int tile_base = lane & ~(kTile - 1), j = lane & (kTile - 1);
   bool mine = slot >= 0;
 #pragma unroll
-  for (int q = 0; q < kTile; q++) {
+  for (int q = 0; q < R; q++) {
     const int64_t other = __shfl((long long)slot, tile_base + q);
     if (q < j && other == slot) mine = false; /* the same key earlier in the tile */
   }

@@ -366,10 +366,18 @@ __device__ __forceinline__ uint4 line_load(const View& v, uint64_t bs, uint32_t 
   const uint64_t a = ld_u64(v.scores + at), b = ld_u64(v.scores + at + 1);
   return make_uint4((uint32_t)a, (uint32_t)(a >> 32), (uint32_t)b, (uint32_t)(b >> 32));
 }
+/* slots of a bucket that a search passes over */
+struct SlotSet {
+  uint64_t lo, hi;
+  __device__ __forceinline__ bool has(uint32_t p) const { return ((p < 64 ? lo : hi) >> (p & 63)) & 1u; }
+  __device__ __forceinline__ void add(uint32_t p) { (p < 64 ? lo : hi) |= UINT64_C(1) << (p & 63); }
+};
 /* minimum of line g over the tile: score and slot position in the bucket */
-__device__ __forceinline__ void line_min(const uint4& x, uint32_t g, int j, uint64_t& m, uint32_t& pos) {
-  const uint64_t s0 = x.x | ((uint64_t)x.y << 32), s1 = x.z | ((uint64_t)x.w << 32);
+__device__ __forceinline__ void line_min(const uint4& x, uint32_t g, int j, const SlotSet& skip, uint64_t& m,
+                                         uint32_t& pos) {
   const uint32_t p0 = g * 16 + j * 2;
+  const uint64_t s0 = skip.has(p0) ? kMaxScore : x.x | ((uint64_t)x.y << 32);
+  const uint64_t s1 = skip.has(p0 + 1) ? kMaxScore : x.z | ((uint64_t)x.w << 32);
   m = s1 < s0 ? s1 : s0;
   pos = s1 < s0 ? p0 + 1 : p0;
   tile_min_pair(m, pos);
@@ -378,10 +386,10 @@ __device__ __forceinline__ void line_min(const uint4& x, uint32_t g, int j, uint
  * part of it.  All 8 lanes of the tile call this together.  `nb`: what line bpos / 16 is bounded
  * by once slot bpos has been given a score that is above everything else in it. */
 __device__ __forceinline__ void bounded_min(const View& v, uint64_t bs, int tile, int j, uint64_t bd,
-                                            uint32_t g, uint4 x, uint64_t cap, uint64_t& best,
-                                            uint32_t& bpos, uint64_t& nb) {
+                                            uint32_t g, uint4 x, uint64_t cap, const SlotSet& skip,
+                                            uint64_t& best, uint32_t& bpos, uint64_t& nb) {
   uint64_t* const bounds = v.bounds + (bs >> 4);
-  line_min(x, g, j, best, bpos);
+  line_min(x, g, j, skip, best, bpos);
   uint32_t opened = 1u << g;
   for (;;) {
     const bool lower = !((opened >> j) & 1u) && (bd < best || (bd == best && (uint32_t)j < (bpos >> 4)));
@@ -392,7 +400,7 @@ __device__ __forceinline__ void bounded_min(const View& v, uint64_t bs, int tile
     const uint4 y = line_load(v, bs, c, j);
     uint64_t m;
     uint32_t pos;
-    line_min(y, c, j, m, pos);
+    line_min(y, c, j, skip, m, pos);
     if (m < best || (m == best && pos < bpos)) {
       /* the line that held the best so far is bounded by exactly that */
       if ((uint32_t)j == (bpos >> 4)) st_u64(bounds + j, best < cap ? best : cap);
@@ -406,7 +414,8 @@ __device__ __forceinline__ void bounded_min(const View& v, uint64_t bs, int tile
   /* the smallest score of the chosen line apart from the chosen slot */
   const uint64_t s0 = x.x | ((uint64_t)x.y << 32), s1 = x.z | ((uint64_t)x.w << 32);
   const uint32_t p0 = (bpos & ~15u) + j * 2;
-  const uint64_t r0 = p0 == bpos ? kMaxScore : s0, r1 = p0 + 1 == bpos ? kMaxScore : s1;
+  const uint64_t r0 = p0 == bpos || skip.has(p0) ? kMaxScore : s0;
+  const uint64_t r1 = p0 + 1 == bpos || skip.has(p0 + 1) ? kMaxScore : s1;
   nb = tile_min(r1 < r0 ? r1 : r0);
 }
 
@@ -541,6 +550,8 @@ __device__ __forceinline__ void bulk_evicted(int kind, const uint8_t* src, uint8
  * 128-bit mask of EMPTY digests.  Every lane of the wavefront must call this.
  */
 constexpr int kMaxLockedWaits = 64;
+/* slots a new key of a full bucket tries in one trip (searches through the score bounds) */
+constexpr int kVictimAttempts = 4;
 template <int R = kTile>
 __device__ __forceinline__ void settle_reprobes(const View& v, uint64_t key, uint32_t bkt,
                                                 uint32_t digest, bool pending, bool& reprobe,
@@ -742,7 +753,7 @@ upsert_kernel(View v, UpsertArgs a) {
           if ((need >> (h + q)) & 1u) {
             uint64_t b0, nb0;
             uint32_t p0;
-            bounded_min(v, bs[q], tile, j, bd[q], g[q], x[q], bound_cap, b0, p0, nb0);
+            bounded_min(v, bs[q], tile, j, bd[q], g[q], x[q], bound_cap, SlotSet{0, 0}, b0, p0, nb0);
             if (j == h + q) {
               best = b0;
               bpos = p0;
@@ -802,9 +813,8 @@ upsert_kernel(View v, UpsertArgs a) {
     bool cas_ok = false;
     if (has_hit || has_free)
       cas_ok = cas_lock(has_hit ? v.keys + hit : v.keys + bslot + p_free, seen, v.locked_key);
-    uint64_t* const kp = v.keys + bslot + bpos;
     uint64_t vk = v.locked_key;
-    if (try_victim) vk = swap_lock(kp, v.locked_key);
+    if (try_victim) vk = swap_lock(v.keys + bslot + bpos, v.locked_key);
 
     /* ---- step 3: what came back ------------------------------------------------------------------------ */
     if (has_hit) {
@@ -844,7 +854,8 @@ upsert_kernel(View v, UpsertArgs a) {
         }
       }
     }
-    if (try_victim) {
+    /* the slot at bpos after the exchange has brought back vk */
+    auto claim_victim = [&]() {
       const bool mine = vk != v.locked_key && vk != v.empty_key;
       if (vk == v.empty_key) {
         /* The slot has become free since the probe (an erase that runs beside this call) and
@@ -861,9 +872,56 @@ upsert_kernel(View v, UpsertArgs a) {
           got = (vk == v.reclaim_key) ? kStReclaimed : kStEvict;
           pos = bpos;
         } else {
-          st_unlock(kp, vk); /* nothing was written under this lock */
+          st_unlock(v.keys + bslot + bpos, vk); /* nothing was written under this lock */
         }
-      } /* else: the victim is locked or was taken by somebody else; next trip */
+      } /* else: the victim is locked or was taken by somebody else */
+    };
+    if (try_victim) claim_victim();
+    if constexpr (BOUNDS) {
+      /* Several new keys of a bucket find the same lowest score, and one of them gets the slot.  Whoever
+       * holds it, or has raised its score since the search, is a key of this launch, which leaves a
+       * score there that is not below bound_cap.  So as long as the lowest score of the other slots is
+       * below bound_cap, that is where the next victim is, whatever becomes of the slot that was
+       * lost: it is tried right away, instead of in another trip behind this one's rows and locks.
+       * insert_and_evict, 2^17 keys of 128 bytes, two new ones per bucket: 82 -> 68 us; insert_or_assign
+       * and find, one new key per bucket: 2^16 keys of 512 bytes 65 -> 59, 2^20 of 256 376 -> 363. */
+      SlotSet lost{0, 0};
+      bool again = try_victim && got == kStNone;
+#pragma unroll 1
+      for (int attempt = 1; attempt < kVictimAttempts && __ballot(again); attempt++) {
+        if (again) lost.add(bpos);
+        uint32_t need = tile_ballot(again, tile);
+        const int lane_base = lane & ~(kTile - 1);
+        for (unsigned long long rest = __ballot(need != 0); rest; rest = __ballot(need != 0)) {
+          if (need) {
+            const int r0 = __ffs(need) - 1, src = lane_base + r0;
+            need &= need - 1;
+            const uint64_t bs0 = __shfl((unsigned long long)bslot, src);
+            const SlotSet skip{__shfl((unsigned long long)lost.lo, src), __shfl((unsigned long long)lost.hi, src)};
+            /* what bounds the line of the slot that was lost, apart from that slot */
+            const uint32_t line = (uint32_t)__shfl((int)bpos, src) >> 4;
+            const uint64_t others = __shfl((unsigned long long)new_bound, src);
+            uint64_t bd = ld_u64(v.bounds + (bs0 >> 4) + j);
+            if ((uint32_t)j == line && others > bd) bd = others;
+            uint64_t b = bd;
+            uint32_t g = (uint32_t)j;
+            tile_min_pair(b, g);
+            uint64_t b0, nb0;
+            uint32_t p0;
+            bounded_min(v, bs0, tile, j, bd, g, line_load(v, bs0, g, j), bound_cap, skip, b0, p0, nb0);
+            if (j == r0) {
+              best = b0;
+              bpos = p0;
+              new_bound = nb0;
+            }
+          }
+        }
+        again = again && best < bound_cap;
+        vk = v.locked_key;
+        if (again) vk = swap_lock(v.keys + bslot + bpos, v.locked_key);
+        if (again) claim_victim();
+        again = again && got == kStNone;
+      }
     }
 
     /* ---- step 4: critical sections of every lock taken in this trip ------------------------------ */

@@ -41,8 +41,11 @@ void launch_form(int vec, const View& v, const UpsertArgs& a, hipStream_t s) {
   }
 }
 
-/* insert_and_evict with `pair`: the wavefronts of 128 keys share the claims on the
- * evicted-keys output (hkv_upsert.hpp) */
+/* insert_and_evict with `pair`: the wavefronts of a workgroup share the claims on the
+ * evicted-keys output (hkv_upsert.hpp), two of 64 keys or four of 8 or 16.  Fewer keys per claim
+ * queue up at the counter, more wait for each other at every trip.  2^12 keys of 64 bytes, workgroups
+ * of 4 / 8 / 16 wavefronts with a key per tile: 60.5 / 63.5 / 67.4 us for the call; 2^17 of 128 bytes, two
+ * keys per tile: 101.5 / 102.4 / 108.3. */
 template <int OP, bool LOCKED_RULE, bool BOUNDS, int R>
 void launch_upsert_for(bool pair, int vec, const View& v, const UpsertArgs& a, hipStream_t s) {
   if constexpr (OP == kOpInsertOrAssign || OP == kOpFindOrInsert) {
@@ -54,7 +57,7 @@ void launch_upsert_for(bool pair, int vec, const View& v, const UpsertArgs& a, h
   }
   if constexpr (OP == kOpInsertAndEvict) {
     if (pair) {
-      launch_form<OP, R, LOCKED_RULE, BOUNDS, 2 * kTile / R>(vec, v, a, s);
+      launch_form<OP, R, LOCKED_RULE, BOUNDS, R == kTile ? 2 : 4>(vec, v, a, s);
       return;
     }
   }

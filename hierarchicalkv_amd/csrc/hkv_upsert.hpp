@@ -602,7 +602,7 @@ __device__ __forceinline__ void settle_reprobes(const View& v, uint64_t key, uin
  * refused at score == min is a separate switch (UpsertArgs::refuse_equal).
  */
 /* WAVES wavefronts per workgroup, each with its own 8 R keys and its own staging area.  One
- * everywhere except insert_and_evict on a table that is about full, where the wavefronts of 128 keys
+ * everywhere except insert_and_evict on a table that is about full, where two or four wavefronts
  * claim their part of the evicted-keys output together: updates of one word are served one at a time, about
  * 15 ns each, and one per wavefront and trip (some 24 thousand for 2^20 keys into full buckets)
  * took 0.07 ms of the call's 0.46.  (While buckets have free slots there is nothing to claim,

@@ -765,13 +765,8 @@ int run_upsert(hkv_table* t, UpsertArgs a, int vec, bool hybrid_rule, hipStream_
                       (OP == kOpInsertOrAssign || OP == kOpFindOrInsert);
     uint64_t** held = nullptr;
     if (hold) {
-      /* n slot addresses, then n scores */
+      /* n slot addresses, then n scores; the kernel writes an address or null for every key */
       HKV_HIP(hipMallocAsync((void**)&held, a.n * 16, s));
-      const hipError_t e = hipMemsetAsync(held, 0, a.n * 8, s);
-      if (e != hipSuccess) {
-        (void)hipFreeAsync(held, s);
-        HKV_HIP(e);
-      }
       a.locked_key_ptrs = held;
       a.held_scores = reinterpret_cast<uint64_t*>(held) + a.n;
       a.locked_count = nullptr; /* nothing stays LOCKED beyond this call */

@@ -683,6 +683,7 @@ upsert_kernel(View v, UpsertArgs a) {
    * the end of the launch (an instantiation of its own: as a run-time switch it cost the kernels
    * of tables without host rows 3 %) */
   constexpr bool hold = HOLD;
+  bool held = false; /* this lane's key has its slot */
   /* Where every slot that is taken stays LOCKED to the end of the launch, a LOCKED word is never
    * this key's slot about to be given back: it is another key of the batch, or this key on its
    * way out.  The second probe does not wait for it.  (With the waits, a key whose digest
@@ -966,10 +967,10 @@ upsert_kernel(View v, UpsertArgs a) {
         st_u64(v.bounds + (slot >> 4), new_bound < bound_cap ? new_bound : bound_cap);
       const uint64_t stored = write_meta(v, a, slot, digest, desired, in_score, i, got != kStDuplicate, hold);
       if (hold) {
-        /* hybrid mode: the slots of a batch stay LOCKED until all its keys are settled; the
-         * list starts out as all null */
+        /* hybrid mode: the slots of a batch stay LOCKED until all its keys are settled */
         a.locked_key_ptrs[i] = v.keys + slot;
         a.held_scores[i] = stored;
+        held = true;
       }
       /* Scores from the caller may be below what the line's bound says: a key that goes into a
        * free slot, and a key that was found, under Customized (its score becomes the caller's)
@@ -1034,6 +1035,8 @@ upsert_kernel(View v, UpsertArgs a) {
     pend_mask = __ballot(pending);
     if constexpr (WAVES == 1) more = pend_mask != 0;
   }
+  /* (a clear of the list beforehand is a launch of its own, 4.8 us) */
+  if (HOLD && !held && i < a.n) a.locked_key_ptrs[i] = nullptr;
 }
 
 /* ---- assign family: update keys that are present, never insert -----------------

@@ -68,7 +68,8 @@ void launch_upsert_for(bool pair, int vec, const View& v, const UpsertArgs& a, h
  * victim search and the row copies one or two at a time, so that a batch of a few ten thousand keys
  * is a long chain on part of the chip; with fewer keys per tile the chain is shorter, more wavefronts
  * fit on a SIMD, and every step is issued for fewer keys at once, which is what costs once the chip is
- * full anyway.  us for the whole step, R = 8 / 2 / 1:
+ * full anyway.  us for the whole step, R = 8 / 2 / 1 (with one try for a victim per trip; the tries that
+ * follow in the same trip now take 3 to 15 % off each):
  *   full table (bounds), insert_or_assign with half of the keys new, and find, rows of 256 bytes
  *     2^12 keys   68 /  36 /  31      2^16   84 /  54 /  51      2^18  127 / 116 / 120
  *     2^14        71 /  41 /  36      2^17   97 /  74 /  73      2^20  393 / 397 / 438

@@ -10,7 +10,6 @@ from gpu_util import DEV, assert_same_table, dev, host_bytes, host_u64
 from hierarchicalkv_amd import HashTable, default_options
 
 pytestmark = pytest.mark.gpu
-DIM = 8
 
 
 def bytes_of(a):
@@ -18,16 +17,18 @@ def bytes_of(a):
 
 
 # full tables (victims through the score bounds; one key per tile up to 2^15 keys, two up to 2^18) and
-# tables with free slots (2^14, 2^17)
-@pytest.mark.parametrize("full,cap_bits,sizes", [
-    (True, 18, (1, 7, 8, 9, 16, 17, 65, 1 << 15, (1 << 15) + 1)),
-    (True, 21, (1 << 18, (1 << 18) + 1)),
-    (False, 18, (1, 8, 9, 17, 1 << 14, (1 << 14) + 1)),
-    (False, 21, (1 << 17, (1 << 17) + 1)),
+# tables with free slots (2^14, 2^17); rows of 36 and 40 bytes: accum_or_assign adds them in units of 4 and 8
+@pytest.mark.parametrize("full,cap_bits,dim,sizes", [
+    (True, 14, 9, (1, 9, 65, 1000)),
+    (True, 14, 10, (1, 9, 65, 1000)),
+    (True, 18, 8, (1, 7, 8, 9, 16, 17, 65, 1 << 15, (1 << 15) + 1)),
+    (True, 21, 8, (1 << 18, (1 << 18) + 1)),
+    (False, 18, 8, (1, 8, 9, 17, 1 << 14, (1 << 14) + 1)),
+    (False, 21, 8, (1 << 17, (1 << 17) + 1)),
 ])
-def test_every_upsert_at_the_edges(oracle, full, cap_bits, sizes):
+def test_every_upsert_at_the_edges(oracle, full, cap_bits, dim, sizes):
     cap = 1 << cap_bits
-    o = default_options(init_capacity=cap, max_capacity=cap, max_hbm_for_vectors=1 << 30, dim=DIM)
+    o = default_options(init_capacity=cap, max_capacity=cap, max_hbm_for_vectors=1 << 30, dim=dim)
     t = HashTable()
     t.init(o)
     ot = oracle.OracleTable(o)
@@ -44,10 +45,10 @@ def test_every_upsert_at_the_edges(oracle, full, cap_bits, sizes):
     fill = cap + cap // 4 if full else cap // 4
     while at < fill:
         keys = new_keys(cap // 8)
-        rows = rng.random((len(keys), DIM), dtype=np.float32)
+        rows = rng.random((len(keys), dim), dtype=np.float32)
         t.insert_or_assign(len(keys), dev(keys), dev(rows))
         ot.insert_or_assign_mt(keys, bytes_of(rows), None)
-    assert_same_table(t, ot, DIM * 4)
+    assert_same_table(t, ot, dim * 4)
     recent = keys
     for n in sizes:
         for op in ("insert_or_assign", "find_or_insert", "accum_or_assign", "insert_and_evict"):
@@ -56,7 +57,7 @@ def test_every_upsert_at_the_edges(oracle, full, cap_bits, sizes):
             is_hit = np.arange(n) < n // 2
             order = rng.permutation(n)
             keys, is_hit = keys[order], is_hit[order]
-            rows = rng.random((n, DIM), dtype=np.float32)
+            rows = rng.random((n, dim), dtype=np.float32)
             dk, dv = dev(keys), dev(rows)
             if op == "insert_or_assign":
                 t.insert_or_assign(n, dk, dv)
@@ -65,21 +66,21 @@ def test_every_upsert_at_the_edges(oracle, full, cap_bits, sizes):
                 t.find_or_insert(n, dk, dv)
                 want = bytes_of(rows).copy()
                 ot.find_or_insert(keys, want, None)
-                assert (host_bytes(dv, n, DIM * 4) == want).all(), (n, op)
+                assert (host_bytes(dv, n, dim * 4) == want).all(), (n, op)
             elif op == "accum_or_assign":
                 t.accum_or_assign(n, dk, dv, dev(is_hit))
                 ot.accum_or_assign(keys, bytes_of(rows), is_hit.astype(np.uint8), None)
             else:
                 ek = torch.zeros(n, dtype=torch.int64, device=DEV)
-                ev = torch.zeros(n, DIM, dtype=torch.float32, device=DEV)
+                ev = torch.zeros(n, dim, dtype=torch.float32, device=DEV)
                 es = torch.zeros(n, dtype=torch.int64, device=DEV)
                 gone = t.insert_and_evict(n, dk, dv, None, ek, ev, es)
                 wk, wv, ws = ot.insert_and_evict(keys, bytes_of(rows), None)[:3]
                 assert gone == len(wk), (n, op)
                 a, b = np.argsort(host_u64(ek)[:gone]), np.argsort(wk)
                 assert (host_u64(ek)[:gone][a] == wk[b]).all(), (n, op)
-                assert (host_bytes(ev, n, DIM * 4)[:gone][a] == wv[b]).all(), (n, op)
+                assert (host_bytes(ev, n, dim * 4)[:gone][a] == wv[b]).all(), (n, op)
                 assert (host_u64(es)[:gone][a] == ws[b]).all(), (n, op)
             assert t.size() == ot.size(), (n, op)
-        assert_same_table(t, ot, DIM * 4)
+        assert_same_table(t, ot, dim * 4)
     t.close()

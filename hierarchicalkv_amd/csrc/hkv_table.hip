@@ -675,6 +675,9 @@ bool prepare_bounds(hkv_table* t, UpsertArgs& a, hipStream_t s) {
   if (t->keys_offered * 10 < t->view.capacity * 9) return false;
   if (capturing(s)) return false; /* writes_scores_outside_bounds() then switches the bounds off */
   const bool from_clock = st == HKV_LRU || st == HKV_EPOCH_LRU;
+  /* Customized with ignore_evict_strategy may come without scores, which then count as 0: there is
+   * nothing to take the lowest of (writes_scores_outside_bounds() has the bounds made again) */
+  if (!from_clock && !a.scores) return false;
   if (st == HKV_EPOCH_LRU) {
     /* (epoch << 32) | (clock >> 20 & 0xFFFFFFFF) grows while the epoch does not go back and the low
      * half does not wrap (every 2^52 ns); a call that may see the wrap happen, or a clock that

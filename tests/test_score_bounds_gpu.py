@@ -322,6 +322,72 @@ def test_customized_scores_that_go_down(oracle):
     t.close()
 
 
+@pytest.mark.parametrize("row_bytes", [16, 36, 40])
+def test_customized_calls_without_scores(oracle, row_bytes):
+    """A full Customized table, ignore_evict_strategy and no scores: every key of the call counts as 0.
+    New keys are refused where every score is above 0 and take the place of a key with score 0
+    otherwise; a key that is found keeps its place with score 0 and is the next one to go."""
+    cap, bs, dim = 1 << 13, 2048, row_bytes // 4
+    buckets = cap // 128
+    t, o = make(cap, dim, EvictStrategy.kCustomized)
+    ot = oracle.OracleTable(o)
+    pos, batch = 0, 10
+    while pos < cap + 4 * bs:
+        k = w.unique_keys(660, pos, bs)
+        upsert(t, ot, k, w.values_from_keys(k, dim), w.monotone_scores(batch, bs, seed=66))
+        pos += bs
+        batch += 1
+    assert_same_table(t, ot, row_bytes)
+    assert bounds_hold(t)[0]
+    at = 0
+    for step in range(12):
+        # one key of the call per bucket: two would evict each other in an order that nothing fixes
+        fresh = one_per_bucket(oracle, w.unique_keys(661, at, 400), buckets)
+        at += 400
+        if step % 3 == 0:
+            k = fresh  # refused at first (no score is 0 yet)
+        else:
+            # (a key with score 0 before any other of its bucket, so that no bucket gets two of them: which
+            # of two goes first depends on where they are)
+            resident, _, score = ot.export_all()
+            order = np.random.default_rng(step).permutation(len(resident))
+            found = one_per_bucket(oracle, resident[order][np.argsort(score[order] > 0, kind="stable")], buckets)
+            k = found if step % 3 == 1 else one_per_bucket(oracle, np.concatenate([found[:20], fresh]), buckets)
+        v = w.values_from_keys(k, dim) + step
+        n, zeros = len(k), np.zeros(len(k), np.uint64)
+        op = ("insert_or_assign", "accum_or_assign", "find_or_insert", "insert_and_evict")[(step // 3 + step % 3) % 4]
+        if op == "insert_or_assign":
+            t.insert_or_assign(n, dev(k), dev(v), None, ignore_evict_strategy=True)
+            ot.insert_or_assign(k, bytes_of(v), zeros, ignore=True)
+        elif op == "accum_or_assign":
+            there = ot.contains(k)
+            t.accum_or_assign(n, dev(k), dev(v), dev(there), None, ignore_evict_strategy=True)
+            ot.accum_or_assign(k, bytes_of(v), there.astype(np.uint8), zeros, ignore=True)
+        elif op == "find_or_insert":
+            dv, ov = dev(v), bytes_of(v).copy()
+            t.find_or_insert(n, dev(k), dv, None, ignore_evict_strategy=True)
+            ot.find_or_insert(k, ov, zeros, ignore=True)
+            assert (dv.cpu().numpy().view(np.uint8).reshape(n, -1) == ov).all(), step
+        else:
+            ek = torch.zeros(n, dtype=torch.int64, device=DEV)
+            ev = torch.zeros(n, dim, dtype=torch.float32, device=DEV)
+            es = torch.zeros(n, dtype=torch.int64, device=DEV)
+            gone = t.insert_and_evict(n, dev(k), dev(v), None, ek, ev, es, ignore_evict_strategy=True)
+            oek, _, oes = ot.insert_and_evict(k, bytes_of(v), zeros, ignore=True)
+            got = zip(ek[:gone].cpu().numpy().view(np.uint64).tolist(), es[:gone].cpu().numpy().view(np.uint64).tolist())
+            assert sorted(got) == sorted(zip(oek.tolist(), oes.tolist())), step
+        assert_same_table(t, ot, row_bytes)
+    # keys with scores again: the ones with score 0 go first, and the bounds are right
+    assert (ot.export_all()[2] == 0).sum() > buckets // 2
+    for rep in range(2):
+        k = w.unique_keys(662, rep * 900, 900)
+        upsert(t, ot, k, w.values_from_keys(k, dim), w.monotone_scores(batch + rep, len(k), seed=66))
+        ok, bad, n_tight = bounds_hold(t)
+        assert ok and n_tight > 0, (rep, bad)
+        assert_same_table(t, ot, row_bytes)
+    t.close()
+
+
 @pytest.mark.parametrize("strategy", [EvictStrategy.kLfu, EvictStrategy.kEpochLfu])
 def test_frequency_scores_and_bounds(oracle, strategy):
     """LFU / EpochLFU: a new key comes in with the caller's count, which under LFU may be below

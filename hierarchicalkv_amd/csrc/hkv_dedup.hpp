@@ -118,28 +118,36 @@ __global__ void dedup_fix_ptrs_kernel(const uint32_t* rep, uint64_t n, void** ou
   if (out_ptrs) out_ptrs[i] = out_ptrs[r];
   if (founds) founds[i] = founds[r];
 }
-/* ... or its row, one T per thread.  The rows that are read belong to representatives, which nobody
- * writes.  2^18 rows of 128 bytes, Zipf(1.05): 6 us; 59 us with a workgroup per key, 18 us with four
- * copies in flight per thread or with a list of the duplicates per wavefront. */
+/* ... or its row, one T per thread: keys first .. first + n - 1.  The rows that are read belong to
+ * representatives, which nobody writes.  2^18 rows of 128 bytes, Zipf(1.05): 6 us; 59 us with a workgroup per
+ * key, 18 us with four copies in flight per thread or with a list of the duplicates per wavefront. */
 template <class T>
 __global__ void __launch_bounds__(256)
-dedup_fix_rows_kernel(const uint32_t* rep, uint64_t n, uint8_t* rows, uint32_t row_bytes) {
+dedup_fix_rows_kernel(const uint32_t* rep, uint64_t first, uint32_t n, uint8_t* rows, uint32_t row_bytes) {
   const uint32_t units = row_bytes / sizeof(T);
-  const uint64_t total = n * units;
-  const uint64_t u = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (u >= total) return;
-  const uint64_t i = total <= 0xFFFFFFFFull ? (uint32_t)u / units : u / units;
+  const uint32_t u = blockIdx.x * 256u + threadIdx.x;
+  if (u >= n * units) return;
+  const uint64_t i = first + u / units;
   const uint32_t r = rep[i];
   if (r == (uint32_t)i) return;
-  const uint32_t c = (uint32_t)(u - i * units);
+  const uint32_t c = u % units;
   reinterpret_cast<T*>(rows + i * row_bytes)[c] = reinterpret_cast<const T*>(rows + r * (uint64_t)row_bytes)[c];
 }
 
+/* A launch may not have 2^32 threads (the runtime was seen to run a part of them and to report nothing), and
+ * 4 GiB of rows are a possible batch on this card: so many keys go into one launch that it has 2^31
+ * threads at most (a row is at most 2^20 bytes). */
+constexpr uint64_t kDedupLaunchThreads = UINT64_C(1) << 31;
+constexpr uint64_t dedup_keys_per_launch(uint64_t units) { return kDedupLaunchThreads / units; }
+
 template <class T>
 inline void dedup_fix_rows_by(const uint32_t* rep, uint64_t n, uint8_t* rows, uint32_t row_bytes, hipStream_t s) {
-  const uint64_t units = n * (row_bytes / sizeof(T));
-  hipLaunchKernelGGL(dedup_fix_rows_kernel<T>, dim3((unsigned)((units + 255) / 256)), dim3(256), 0, s, rep, n, rows,
-                     row_bytes);
+  const uint64_t units = row_bytes / sizeof(T), step = dedup_keys_per_launch(units);
+  for (uint64_t first = 0; first < n; first += step) {
+    const uint64_t m = n - first < step ? n - first : step;
+    hipLaunchKernelGGL(dedup_fix_rows_kernel<T>, dim3((unsigned)((m * units + 255) / 256)), dim3(256), 0, s, rep, first,
+                       (uint32_t)m, rows, row_bytes);
+  }
 }
 inline void dedup_fix_rows(const uint32_t* rep, uint64_t n, uint8_t* rows, uint32_t row_bytes, hipStream_t s) {
   const uintptr_t mis = row_bytes | (uintptr_t)rows;

@@ -26,6 +26,11 @@ constexpr uint64_t kLow32 = UINT64_C(0xFFFFFFFF);
 constexpr int kTile = 8;
 constexpr int kTilesPerWave = kWave / kTile;
 
+/* A launch may not have 2^32 threads (the runtime was seen to run a part of them and to report nothing).
+ * Kernels with several threads per key or one per unit of a row stay at this many and go over a
+ * longer batch in several launches. */
+constexpr uint64_t kLaunchThreads = UINT64_C(1) << 31;
+
 /* Everything the probe needs to know about one key of the batch; staged in
  * LDS by the lane that owns the key, read back by the tile that probes it. */
 struct KeyMeta {

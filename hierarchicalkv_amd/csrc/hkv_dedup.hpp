@@ -134,15 +134,10 @@ dedup_fix_rows_kernel(const uint32_t* rep, uint64_t first, uint32_t n, uint8_t* 
   reinterpret_cast<T*>(rows + i * row_bytes)[c] = reinterpret_cast<const T*>(rows + r * (uint64_t)row_bytes)[c];
 }
 
-/* A launch may not have 2^32 threads (the runtime was seen to run a part of them and to report nothing), and
- * 4 GiB of rows are a possible batch on this card: so many keys go into one launch that it has 2^31
- * threads at most (a row is at most 2^20 bytes). */
-constexpr uint64_t kDedupLaunchThreads = UINT64_C(1) << 31;
-constexpr uint64_t dedup_keys_per_launch(uint64_t units) { return kDedupLaunchThreads / units; }
-
+/* (4 GiB of rows are a possible batch on this card; a row is at most 2^20 bytes) */
 template <class T>
 inline void dedup_fix_rows_by(const uint32_t* rep, uint64_t n, uint8_t* rows, uint32_t row_bytes, hipStream_t s) {
-  const uint64_t units = row_bytes / sizeof(T), step = dedup_keys_per_launch(units);
+  const uint64_t units = row_bytes / sizeof(T), step = kLaunchThreads / units;
   for (uint64_t first = 0; first < n; first += step) {
     const uint64_t m = n - first < step ? n - first : step;
     hipLaunchKernelGGL(dedup_fix_rows_kernel<T>, dim3((unsigned)((m * units + 255) / 256)), dim3(256), 0, s, rep, first,

@@ -6,8 +6,20 @@
 namespace hkv {
 namespace {
 
-template <int MODE, int R, bool DUAL = false, int WAVES = 1, bool MISSED = false>
-void launch_lookup_by(int vec, const View& v, const FindArgs& a, hipStream_t s) {
+/* the part of a call from key `first` on, at most `most` keys of it */
+FindArgs part_of(const View& v, const FindArgs& a, uint64_t first, uint64_t most) {
+  FindArgs p = a;
+  p.keys += first;
+  if (p.out_values) p.out_values += first * v.value_bytes;
+  if (p.out_ptrs) p.out_ptrs += first;
+  if (p.founds) p.founds += first;
+  if (p.out_scores) p.out_scores += first;
+  p.n = a.n - first < most ? a.n - first : most;
+  return p;
+}
+
+template <int MODE, int R, bool DUAL, int WAVES, bool MISSED>
+void launch_one(int vec, const View& v, const FindArgs& a, hipStream_t s) {
   constexpr uint64_t kKeys = (uint64_t)kTilesPerWave * R * WAVES;
   const dim3 grid((unsigned)((a.n + kKeys - 1) / kKeys)), block(kWave * WAVES);
   if constexpr (MODE == kLookupValues) {
@@ -20,6 +32,19 @@ void launch_lookup_by(int vec, const View& v, const FindArgs& a, hipStream_t s) 
     }
   }
   launch_main(lookup_kernel<MODE, 16, DUAL, WAVES, R, MISSED>, grid, block, s, v, a);
+}
+
+/* One launch for all but the longest batches: two keys per tile are four threads per key, 2^31 of them at
+ * 2^29 keys.  (The missed-keys form has one thread per key, and its 32-bit indices end before that matters.) */
+template <int MODE, int R, bool DUAL = false, int WAVES = 1, bool MISSED = false>
+void launch_lookup_by(int vec, const View& v, const FindArgs& a, hipStream_t s) {
+  if constexpr (MISSED) {
+    launch_one<MODE, R, DUAL, WAVES, MISSED>(vec, v, a, s);
+  } else {
+    constexpr uint64_t kMost = kLaunchThreads / (kTile / R);
+    for (uint64_t first = 0; first < a.n; first += kMost)
+      launch_one<MODE, R, DUAL, WAVES, MISSED>(vec, v, part_of(v, a, first, kMost), s);
+  }
 }
 
 /* Keys per tile.  A wavefront of 64 keys (R = 8) holds 114 registers, four of them fit on a SIMD, and

@@ -47,3 +47,34 @@ def test_rows_of_every_size(row_bytes, shift):
         assert (body[miss] == 0xA5).all()
         assert (got[:PAD + shift] == 0xA5).all() and (got[PAD + shift + n * row_bytes:] == 0xA5).all()
     t.close()
+
+
+# more keys than one launch takes at two keys per tile (2^29); at 2^30 a single one would have 2^32 threads
+@pytest.mark.parametrize("call", ["contains", "find_ptr", "find"])
+def test_more_than_2_30_keys(call):
+    part, n = 1 << 20, (1 << 30) + 4097
+    t = HashTable()
+    t.init(default_options(init_capacity=1 << 20, max_capacity=1 << 20, max_hbm_for_vectors=1 << 30, dim=1))
+    universe = dev(w.unique_keys(63, 0, part))
+    rows = torch.arange(part, dtype=torch.float32, device=DEV)
+    t.insert_or_assign(part // 4, universe, rows)
+    there = torch.arange(part, device=DEV) < part // 4
+    keys = universe.repeat(n // part + 1)[:n]
+    founds = torch.zeros(n, dtype=torch.bool, device=DEV)
+    out = torch.full((n,), -1, dtype=torch.int64 if call == "find_ptr" else torch.int32, device=DEV)
+    if call == "contains":
+        t.contains(n, keys, founds)
+        want = out[:part]
+    elif call == "find":
+        t.find(n, keys, out, founds)
+        want = torch.where(there, rows.view(torch.int32), -1)
+    else:
+        t.find_ptr(n, keys, out, founds)
+        want = torch.zeros(part, dtype=torch.int64, device=DEV)
+        t.find_ptr(part, universe, want, torch.zeros(part, dtype=torch.bool, device=DEV))
+        assert torch.equal(want != 0, there)
+    for lo in range(0, n, part):
+        m = min(part, n - lo)
+        if not (torch.equal(founds[lo:lo + m], there[:m]) and torch.equal(out[lo:lo + m], want[:m])):
+            raise AssertionError(f"keys {lo} to {lo + m}")
+    t.close()

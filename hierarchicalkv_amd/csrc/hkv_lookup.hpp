@@ -311,10 +311,14 @@ __device__ __forceinline__ void copy_found_rows(const View& v, const int64_t* s_
       const bool inside = kk < kKeys;
       const int64_t slot = s_slot[lane_of_key<R>(inside ? kk : 0)];
       const bool found = inside && slot >= 0;
-      const uint64_t from = found ? (uint64_t)slot : 0;
       const uint32_t off = unit_offset<VEC>(c, v.value_bytes);
       at[b] = found ? kk * v.value_bytes + off : kPast;
-      buf[b] = load_row_unit<VEC>((PLAIN ? v.values + (uint64_t)(uint32_t)from * v.value_bytes : value_row(v, from)) + off);
+      const uint8_t* src;
+      if constexpr (PLAIN)
+        src = v.values + (uint64_t)(uint32_t)(found ? slot : 0) * v.value_bytes + off;
+      else
+        src = found ? value_row(v, (uint64_t)slot) + off : v.digests;
+      buf[b] = load_row_unit<VEC>(src);
       kk += kk_step;
       c += c_step;
       if (c >= units) {
@@ -389,8 +393,9 @@ lookup_kernel(View v, FindArgs a) {
 
   /* Copy stage: the rows of the wavefront's keys, spread over its 64 lanes.  All loads of a batch
    * are issued before the first store, and none of them is conditional: a key that was not found
-   * reads slot 0's row, which stays in the caches, and its store goes past the end of the buffer
-   * resource, where the hardware drops it.  Behind a condition every load and store is a block of
+   * reads slot 0's row, which stays in the caches (a table with rows in host memory, where that row
+   * may be behind the host link: the first digests; 2^17 misses, rows of 1024 bytes, none in HBM: 22.9 ->
+   * 16.2 us), and its store goes past the end of the buffer resource, where the hardware drops it.  Behind a condition every load and store is a block of
    * its own, and the compiler waits for more loads than a store needs. */
   if (base >= a.n) return;
   if (v.hbm_slots >= v.capacity && v.capacity <= 0xFFFFFFFFull)

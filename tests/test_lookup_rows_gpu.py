@@ -19,17 +19,31 @@ PAD = 64
     (1, 0), (2, 0), (3, 1), (5, 0), (7, 1), (8, 0), (12, 4), (15, 0), (16, 0), (16, 4), (17, 0), (31, 1), (32, 1), (66, 0),
     (200, 4), (256, 0), (512, 0), (516, 0), (1028, 1), (4100, 0)])
 def test_rows_of_every_size(row_bytes, shift):
+    check(row_bytes, shift, 1 << 34, (1, 2, 7, 8, 9, 15, 16, 17, 63, 65, 1000, 16384, 16385, 16400))
+
+
+# the other form of the row copy: no row in HBM (where a miss must not reach over the host link), and half of them;
+# 2^14 and 2^14 + 1 keys are one and two per tile
+@pytest.mark.parametrize("hbm_share", [0, 0.5])
+@pytest.mark.parametrize("row_bytes,shift", [
+    (1, 0), (2, 1), (3, 0), (6, 0), (12, 1), (15, 0), (16, 0), (17, 4), (40, 0), (66, 1), (256, 4), (516, 0), (1030, 1)])
+def test_rows_in_host_memory(row_bytes, shift, hbm_share):
+    check(row_bytes, shift, int((1 << 15) * row_bytes * hbm_share), (1, 9, 65, 1000, 16384, 16385))
+
+
+def check(row_bytes, shift, hbm, sizes):
     cap, resident = 1 << 15, 20000
     t = HashTable()
-    t.init(default_options(init_capacity=cap, max_capacity=cap, max_hbm_for_vectors=1 << 34, dim=row_bytes,
+    t.init(default_options(init_capacity=cap, max_capacity=cap, max_hbm_for_vectors=hbm, dim=row_bytes,
                            value_kind=0, value_size=1))
+    assert t.is_pure_hbm() == (hbm >= cap * row_bytes)
     keys = w.unique_keys(61, 0, resident)
     rng = np.random.Generator(np.random.PCG64(row_bytes))
     rows = rng.integers(0, 256, (resident, row_bytes), dtype=np.uint8)
     t.insert_or_assign(resident, dev(keys), dev(rows))
     assert t.size() == resident
     absent = w.unique_keys(62, 0, 3000)
-    for n in (1, 2, 7, 8, 9, 15, 16, 17, 63, 65, 1000, 16384, 16385, 16400):
+    for n in sizes:
         if n > 1000 and row_bytes > 2000:
             continue
         pick = rng.integers(0, resident, n)

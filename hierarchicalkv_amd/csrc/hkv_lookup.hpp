@@ -395,8 +395,9 @@ lookup_kernel(View v, FindArgs a) {
    * are issued before the first store, and none of them is conditional: a key that was not found
    * reads slot 0's row, which stays in the caches (a table with rows in host memory, where that row
    * may be behind the host link: the first digests; 2^17 misses, rows of 1024 bytes, none in HBM: 22.9 ->
-   * 16.2 us), and its store goes past the end of the buffer resource, where the hardware drops it.  Behind a condition every load and store is a block of
-   * its own, and the compiler waits for more loads than a store needs. */
+   * 16.2 us), and its store goes past the end of the buffer resource, where the hardware drops it.
+   * Behind a condition every load and store is a block of its own, and the compiler waits for more
+   * loads than a store needs. */
   if (base >= a.n) return;
   if (v.hbm_slots >= v.capacity && v.capacity <= 0xFFFFFFFFull)
     copy_found_rows<VEC, R, true>(v, s_slot, a.out_values, base, a.n, lane);

@@ -188,6 +188,7 @@ struct hkv_table {
   mutable std::mutex counter_mu;
   mutable std::condition_variable counter_cv;
   mutable std::vector<unsigned> counter_free;
+  mutable std::vector<uint8_t> counter_dirty; /* per word: the last call that had it did not leave 0 */
   uint64_t epoch;
   Clock clock;
   mutable StreamGroupLock lock;
@@ -381,29 +382,34 @@ constexpr unsigned kCounterWords = 128;
 constexpr unsigned kExtraWords = 8 + kLockedShards * kLockedStride;
 
 /* A device word for a call that returns a count.  The word belongs to the call from the
- * lease to its end (it is 0 when it is leased out, a kernel adds to it, another hands the sum to the
+ * lease to its end (it is 0 for the call's kernels, one adds to it, another hands the sum to the
  * host and leaves 0), so host threads inside such calls never share one;
  * when all words are out, the next caller waits for one to come back.
  * The sum goes to the host through a word of pinned memory that the kernel stores to: a copy of 8 bytes
  * to pageable memory is a kernel of the runtime too (4.2 us), and a copy on the host behind it.  With
  * the word left at 0 the call needs no launch to clear it.  An insert_and_evict of 2^17 keys that
- * returns a count, with what a write-back cache does around it: 124 -> 112 us. */
+ * returns a count, with what a write-back cache does around it: 124 -> 112 us.
+ * A call that came to no sum (it was refused, or a launch failed) marks the word, and the next one
+ * that gets it clears it, on the stream it counts on. */
 class CounterLease {
  public:
   CounterLease(const hkv_table* t, hipStream_t s) : t_(t), s_(s) {
-    std::unique_lock<std::mutex> g(t->counter_mu);
-    t->counter_cv.wait(g, [&] { return !t->counter_free.empty(); });
-    idx_ = t->counter_free.back();
-    t->counter_free.pop_back();
+    bool dirty;
+    {
+      std::unique_lock<std::mutex> g(t->counter_mu);
+      t->counter_cv.wait(g, [&] { return !t->counter_free.empty(); });
+      idx_ = t->counter_free.back();
+      t->counter_free.pop_back();
+      dirty = t->counter_dirty[idx_];
+    }
+    if (dirty) hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(1), 0, s, word());
   }
   ~CounterLease() {
     /* an early return may have left work on the stream that still writes the word */
-    if (!read_) {
-      (void)hipStreamSynchronize(s_);
-      (void)hipMemset(word(), 0, sizeof(unsigned long long));
-    }
+    if (!read_) (void)hipStreamSynchronize(s_);
     {
       std::lock_guard<std::mutex> g(t_->counter_mu);
+      t_->counter_dirty[idx_] = !read_;
       t_->counter_free.push_back(idx_);
     }
     t_->counter_cv.notify_one();
@@ -1197,6 +1203,7 @@ int create_impl(const hkv_options* o, const hkv_allocator* al, hkv_table** out) 
     if (e != hipSuccess) return bail(fail(HKV_ERROR_HIP, "hipHostMalloc: %s", hipGetErrorString(e)));
   }
   for (unsigned w = 0; w < kCounterWords; w++) t->counter_free.push_back(w);
+  t->counter_dirty.assign(kCounterWords, 0);
   t->d_bound_caps = t->d_counters + kCounterWords;
   t->d_score_floor = t->d_counters + kCounterWords + 2;
   t->d_bound_ceil = t->d_counters + kCounterWords + 4;
@@ -1207,6 +1214,8 @@ int create_impl(const hkv_options* o, const hkv_allocator* al, hkv_table** out) 
     /* score_floor_kernel takes the minimum into a word that holds the highest score */
     if (hipMemset(t->d_score_floor, 0xFF, 2 * sizeof(unsigned long long)) != hipSuccess)
       return bail(fail(HKV_ERROR_HIP, "hipMemset of the score floor words failed"));
+    /* the words are set before a call on any stream uses them */
+    if (hipDeviceSynchronize() != hipSuccess) return bail(fail(HKV_ERROR_HIP, "device synchronisation failed"));
   }
   t->reach_max_capacity = t->dual || o->init_capacity * 2 > o->max_capacity; /* merlin_hashtable.cuh:1064-1069 */
   *out = t;

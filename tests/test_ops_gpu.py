@@ -1282,3 +1282,30 @@ def test_accum_flags_that_disagree_in_nearly_full_buckets(oracle, monkeypatch, b
         assert t.size() == o.size()
         assert_same_table(t, o, vb)
     t.close()
+
+
+def test_counts_after_calls_that_came_to_none():
+    """A count-returning insert_and_evict that is refused (rows in host memory; scores missing) hands back
+    its device word like any other; whoever gets it next, on whichever stream, counts from 0."""
+    cap, dim = 1 << 12, 4
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    tables = []
+    for hbm, strategy in ((0, EvictStrategy.kLru), (1 << 30, EvictStrategy.kCustomized)):
+        t = HashTable()
+        t.init(default_options(init_capacity=cap, max_capacity=cap, max_hbm_for_vectors=hbm, dim=dim,
+                               evict_strategy=strategy))
+        tables.append((t, strategy))
+    keys = w.unique_keys(990, 0, 1500)
+    dk, dv = dev(keys), dev(w.values_from_keys(keys, dim))
+    sc = torch.arange(1, len(keys) + 1, dtype=torch.int64, device=DEV)
+    ek, ev = torch.zeros_like(dk), torch.zeros_like(dv)
+    torch.cuda.synchronize()
+    for t, strategy in tables:
+        t.insert_or_assign(len(keys), dk, dv, sc if strategy == EvictStrategy.kCustomized else None)
+        torch.cuda.synchronize()
+        for rep in range(30):
+            with pytest.raises(RuntimeError):
+                t.insert_and_evict(len(keys), dk, dv, None, ek, ev, None, stream=streams[rep % 3])
+            assert t.size(stream=streams[(rep + 1) % 3]) == len(keys)
+            assert t.size(stream=streams[(rep + 2) % 3]) == len(keys)
+        t.close()

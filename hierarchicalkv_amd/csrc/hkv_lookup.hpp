@@ -17,8 +17,8 @@
  *   verify every digest match is checked against the 8-byte key, the first
  *          lane's candidates first and the others only if those were not it;
  *          the hit slot goes to LDS;
- *   copy   the whole wavefront copies the found rows, one unit per lane and step,
- *          so the output side is written in fully coalesced 1 KB pieces.
+ *   copy   the found keys are listed in LDS, and the whole wavefront copies their rows, one unit per
+ *          lane and step, so the output side is written in coalesced pieces of up to 1 KB.
  * Bound by random 128-byte lines (a digest line, about 1.2 key lines and the row per key): 842 MB
  * move in 112 us for 2^20 keys with rows of 256 bytes, capacity 2^26.  How many keys a tile takes is
  * what matters most beside that (launch_lookup in hkv_launch_lookup.hip).
@@ -59,12 +59,6 @@ template <int R>
 __device__ __forceinline__ bool lane_owns_key(int lane) {
   return R == kTile || (lane & (kTile - 1)) < R;
 }
-/* the lane that owns key kk of a wavefront */
-template <int R>
-__device__ __forceinline__ uint32_t lane_of_key(uint32_t kk) {
-  return R == kTile ? kk : kk / R * kTile + kk % R;
-}
-
 /*
  * Probe the keys staged in s_meta.  On return (after the caller's barrier)
  * s_slot[k] is the table slot of key k or -1.  WRITER selects the writers'
@@ -283,24 +277,30 @@ __device__ __forceinline__ void restage_second_bucket(const View& v, KeyMeta* s_
 
 enum LookupMode { kLookupValues = 0, kLookupPtr = 1, kLookupContains = 2 };
 
-/* rows s_slot[lane_of_key(kk)] of the table -> rows base + kk of `out`, for the keys that were found.
- * PLAIN: all rows are in HBM and slot numbers fit 32 bits (an address is one multiply-add). */
-template <int VEC, int R, bool PLAIN>
-__device__ __forceinline__ void copy_found_rows(const View& v, const int64_t* s_slot, uint8_t* out,
-                                                uint64_t base, uint64_t n, int lane) {
+/* Where a found key's row is and where it goes, in one word: the slot (buckets_num < 2^31, so below
+ * 2^38) and the key's number in its wavefront. */
+constexpr int kFoundShift = 56;
+constexpr uint64_t kFoundSlot = (UINT64_C(1) << kFoundShift) - 1;
+
+/* Where the rows of the table are; an address is one multiply-add in the first case (slot numbers fit 32 bits
+ * there).  A lane past the end of the list reads a row that the caches have: the first key's; slot 0's, in
+ * HBM; or, so that it does not go over the host link, the first digests (as an address beside the two others
+ * these cost 3 of 84 us on a table with rows in both places). */
+enum RowsIn { kRowsHbm, kRowsBoth, kRowsHost };
+
+/* The rows of the `count` found keys listed in `found` -> their places in `out`, where key `base` is the first of
+ * the wavefront. */
+template <int VEC, int R, int WHERE, int kB>
+__device__ __forceinline__ void copy_units(const View& v, const uint64_t* found, uint32_t count, uint32_t units,
+                                           uint8_t* out, uint64_t base, uint64_t n, int lane) {
   using T = typename VecType<VEC>::type;
   constexpr uint32_t kKeys = kTilesPerWave * R;
   constexpr uint32_t kPast = 0x80000000u; /* an offset that is past the end of any wavefront's rows */
-  const uint32_t units = row_units<VEC>(v.value_bytes);
-  const uint32_t total = units * kKeys;
-  /* Units a lane has in flight: all of a wavefront's for rows of up to 256 bytes (twice as many
-   * cost registers: rows of 32 bytes 72 instead of 68 us per 2^20 keys).  A row of less than 16
-   * bytes is one or two units. */
-  constexpr int kB = vec_bytes(VEC) == 16 ? 2 * R : (R + 3) / 4;
+  const uint32_t total = units * count;
   const uint64_t rows_here = n - base < kKeys ? n - base : kKeys;
   const __amdgpu_buffer_rsrc_t dst = __builtin_amdgcn_make_buffer_rsrc(
       out + base * v.value_bytes, 0, (uint32_t)(rows_here * v.value_bytes), 0x00020000);
-  /* (key, unit) of this lane's next step; a step moves 64 units on */
+  /* (found key, unit) of this lane's next step; a step moves 64 units on */
   uint32_t kk = (uint32_t)lane / units, c = (uint32_t)lane % units;
   const uint32_t kk_step = kWave / units, c_step = kWave % units;
   for (uint32_t idx0 = lane; idx0 < total; idx0 += kWave * kB) {
@@ -308,16 +308,17 @@ __device__ __forceinline__ void copy_found_rows(const View& v, const int64_t* s_
     uint32_t at[kB];
 #pragma unroll
     for (int b = 0; b < kB; b++) {
-      const bool inside = kk < kKeys;
-      const int64_t slot = s_slot[lane_of_key<R>(inside ? kk : 0)];
-      const bool found = inside && slot >= 0;
+      const bool inside = kk < count;
+      const uint64_t f = found[inside ? kk : 0];
       const uint32_t off = unit_offset<VEC>(c, v.value_bytes);
-      at[b] = found ? kk * v.value_bytes + off : kPast;
+      at[b] = inside ? (uint32_t)(f >> kFoundShift) * v.value_bytes + off : kPast;
       const uint8_t* src;
-      if constexpr (PLAIN)
-        src = v.values + (uint64_t)(uint32_t)(found ? slot : 0) * v.value_bytes + off;
+      if constexpr (WHERE == kRowsHbm)
+        src = v.values + (uint64_t)(uint32_t)f * v.value_bytes + off;
+      else if constexpr (WHERE == kRowsBoth)
+        src = value_row(v, inside ? f & kFoundSlot : 0) + off;
       else
-        src = found ? value_row(v, (uint64_t)slot) + off : v.digests;
+        src = inside ? v.host_values + (f & kFoundSlot) * v.value_bytes + off : v.digests;
       buf[b] = load_row_unit<VEC>(src);
       kk += kk_step;
       c += c_step;
@@ -329,6 +330,22 @@ __device__ __forceinline__ void copy_found_rows(const View& v, const int64_t* s_
 #pragma unroll
     for (int b = 0; b < kB; b++) store_row_unit<VEC>(dst, at[b], buf[b]);
   }
+}
+
+/* Units a lane has in flight: all of a wavefront's for rows of up to 256 bytes (twice as many
+ * cost registers: rows of 32 bytes 72 instead of 68 us per 2^20 keys), or a quarter of them where the rows
+ * that were found are no more than that: a step past their end costs a load and a store all the same.
+ * A row of less than 16 bytes is one or two units. */
+template <int VEC, int R, int WHERE>
+__device__ __forceinline__ void copy_found_rows(const View& v, const uint64_t* found, uint32_t count,
+                                                uint8_t* out, uint64_t base, uint64_t n, int lane) {
+  constexpr int kMany = vec_bytes(VEC) == 16 ? 2 * R : (R + 3) / 4;
+  constexpr int kFew = kMany / 4 > 1 ? kMany / 4 : 1;
+  const uint32_t units = row_units<VEC>(v.value_bytes);
+  if (kFew < kMany && units * count <= kWave * kFew)
+    copy_units<VEC, R, WHERE, kFew>(v, found, count, units, out, base, n, lane);
+  else
+    copy_units<VEC, R, WHERE, kMany>(v, found, count, units, out, base, n, lane);
 }
 
 /* WAVES wavefronts per workgroup, each with its own keys and its own staging area.  One
@@ -391,18 +408,29 @@ lookup_kernel(View v, FindArgs a) {
   }
   if (MODE != kLookupValues) return;
 
-  /* Copy stage: the rows of the wavefront's keys, spread over its 64 lanes.  All loads of a batch
-   * are issued before the first store, and none of them is conditional: a key that was not found
-   * reads slot 0's row, which stays in the caches (a table with rows in host memory, where that row
-   * may be behind the host link: the first digests; 2^17 misses, rows of 1024 bytes, none in HBM: 22.9 ->
-   * 16.2 us), and its store goes past the end of the buffer resource, where the hardware drops it.
-   * Behind a condition every load and store is a block of its own, and the compiler waits for more
-   * loads than a store needs. */
-  if (base >= a.n) return;
+  /* Copy stage: the rows of the keys that were found, spread over the wavefront's 64 lanes.  The keys
+   * are listed first, so that a miss costs neither a load nor a store.  All loads of a batch are issued
+   * before the first store, and none of them is conditional: a lane past the end of the list reads something
+   * all the same (RowsIn), and its store goes past the end of the buffer resource, where the hardware drops
+   * it.  Behind a condition every load and store is a block of its own, and the compiler waits for more
+   * loads than a store needs.
+   * With a step for every key instead of for the found ones, misses cost most of what hits do: 2^20 keys,
+   * none found, rows of 256 bytes 50 -> 34 us, of 1024 128 -> 43; half found, rows of 64 bytes 56 -> 49;
+   * all found, 256 bytes 103 both ways.  (Half found, rows of 1024 bytes and more: up to 5 % the other way,
+   * as wavefronts have unequal numbers of rows to move.) */
+  const unsigned long long hits = __ballot(my_slot >= 0);
+  if (hits == 0) return;
+  uint64_t* const s_found = reinterpret_cast<uint64_t*>(s_slot); /* every lane has read its slot */
+  if (my_slot >= 0)
+    s_found[__popcll(hits & ((1ull << lane) - 1))] = (uint64_t)my_slot | ((i - base) << kFoundShift);
+  wave_sync();
+  const uint32_t count = (uint32_t)__popcll(hits);
   if (v.hbm_slots >= v.capacity && v.capacity <= 0xFFFFFFFFull)
-    copy_found_rows<VEC, R, true>(v, s_slot, a.out_values, base, a.n, lane);
+    copy_found_rows<VEC, R, kRowsHbm>(v, s_found, count, a.out_values, base, a.n, lane);
+  else if (v.hbm_slots != 0)
+    copy_found_rows<VEC, R, kRowsBoth>(v, s_found, count, a.out_values, base, a.n, lane);
   else
-    copy_found_rows<VEC, R, false>(v, s_slot, a.out_values, base, a.n, lane);
+    copy_found_rows<VEC, R, kRowsHost>(v, s_found, count, a.out_values, base, a.n, lane);
 }
 
 }  // namespace hkv

@@ -31,7 +31,17 @@ def test_rows_in_host_memory(row_bytes, shift, hbm_share):
     check(row_bytes, shift, int((1 << 15) * row_bytes * hbm_share), (1, 9, 65, 1000, 16384, 16385))
 
 
-def check(row_bytes, shift, hbm, sizes):
+# no key found, few, half of them, nearly all and all: the copy's list of found keys at its edges, for rows of less
+# than a unit's 16 bytes, of a part of a wavefront's step of 1024 bytes, of one step and of more; the missed-keys
+# form too
+@pytest.mark.parametrize("missed_form", [False, True])
+@pytest.mark.parametrize("row_bytes", [4, 12, 16, 40, 64, 256, 512, 1024, 1040, 4096])
+def test_any_share_of_hits(row_bytes, missed_form):
+    for miss_share in (1.0, 0.97, 0.5, 0.03, 0.0):
+        check(row_bytes, 0, 1 << 34, (1, 8, 17, 65, 1000, 16385), miss_share, missed_form)
+
+
+def check(row_bytes, shift, hbm, sizes, miss_share=0.2, missed_form=False):
     cap, resident = 1 << 15, 20000
     t = HashTable()
     t.init(default_options(init_capacity=cap, max_capacity=cap, max_hbm_for_vectors=hbm, dim=row_bytes,
@@ -47,14 +57,23 @@ def check(row_bytes, shift, hbm, sizes):
         if n > 1000 and row_bytes > 2000:
             continue
         pick = rng.integers(0, resident, n)
-        miss = rng.random(n) < 0.2
+        miss = rng.random(n) < miss_share
         q = np.where(miss, absent[np.arange(n) % len(absent)], keys[pick])
         buf = torch.full((PAD + shift + n * row_bytes + PAD,), 0xA5, dtype=torch.uint8, device=DEV)
         founds = torch.zeros(n, dtype=torch.bool, device=DEV)
         d_q = dev(q)
-        t.find(n, d_q, buf[PAD + shift:], founds)
-        torch.cuda.synchronize()
-        assert (founds.cpu().numpy() == ~miss).all()
+        if missed_form:
+            mk, mi = torch.zeros(n, dtype=torch.int64, device=DEV), torch.zeros(n, dtype=torch.int32, device=DEV)
+            ms = torch.zeros(1, dtype=torch.int32, device=DEV)
+            t.find_missed(n, d_q, buf[PAD + shift:], mk, mi, ms)
+            count = int(ms.item())
+            where = np.sort(mi[:count].cpu().numpy())
+            assert (where == np.flatnonzero(miss)).all()
+            assert (mk[:count] == d_q[mi[:count].long()]).all()
+        else:
+            t.find(n, d_q, buf[PAD + shift:], founds)
+            torch.cuda.synchronize()
+            assert (founds.cpu().numpy() == ~miss).all()
         got = buf.cpu().numpy()
         body = got[PAD + shift:PAD + shift + n * row_bytes].reshape(n, row_bytes)
         assert (body[~miss] == rows[pick[~miss]]).all()

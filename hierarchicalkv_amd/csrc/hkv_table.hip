@@ -670,9 +670,35 @@ uint64_t host_realtime_ns() {
   return (uint64_t)ts.tv_sec * UINT64_C(1000000000) + (uint64_t)ts.tv_nsec;
 }
 
+/* Whether a search through the score bounds is the better one for a batch of n keys.  It reads one or two of
+ * a bucket's eight score lines, one after the other, where the scan reads all eight at once.
+ * LRU, EpochLRU: it loses where many new keys of a bucket take its lowest slots one by one, until every
+ * line's bound is at the limit that the call sets and each search opens line after line.  us per call,
+ * bounds / scan, all keys new, rows of 64 bytes:
+ *   keys per bucket                       4         8         16         32         64          128
+ *   capacity 2^21, insert_or_assign     52/51     87/78    156/213    470/368   1488/667
+ *                  insert_and_evict     73/104   116/165   205/341    549/590   1743/1085
+ *   capacity 2^17, insert_or_assign               47/39     79/63     157/116    632/204     4259/376
+ * (EpochLRU has its line higher: its scores go back with the epoch, and a scan then leaves the bounds to
+ * be made again, a pass over the table.) */
+template <int OP>
+bool bounds_pay(const View& v, int strategy, uint64_t n) {
+  if (strategy == HKV_LRU) return n <= (OP == kOpInsertAndEvict ? 32 : 24) * v.buckets_num;
+  if (strategy == HKV_EPOCH_LRU) return n <= 48 * v.buckets_num;
+  return true;
+}
+/* Slots that a new key of a full bucket tries in one trip (hkv_upsert.hpp).  With more new keys per bucket
+ * most tries find the slot taken again (capacity 2^21, LRU, rows of 64 bytes, four tries / one: 16 keys per
+ * bucket 156/147 us, 32 470/384, 64 1488/1019; insert_and_evict 205/293, 549/663, 1743/1557). */
+template <int OP>
+int victim_tries(const View& v, uint64_t n) {
+  return n <= (OP == kOpInsertAndEvict ? 32 : 16) * v.buckets_num ? 4 : 1;
+}
+
 /* Whether this upsert searches victims through the score bounds, and with which limits (the
  * fields of `a`); launches what has to run first (the batch's lowest score, the rebuild).  The
  * caller holds the inserter role on `s`. */
+template <int OP>
 bool prepare_bounds(hkv_table* t, UpsertArgs& a, hipStream_t s) {
   const int st = t->opts.evict_strategy;
   if (!t->score_bounds || a.strategy != st) return false;
@@ -700,6 +726,8 @@ bool prepare_bounds(hkv_table* t, UpsertArgs& a, hipStream_t s) {
     t->bounds_epoch = t->epoch;
     t->bounds_era = now >> 52;
   }
+  if (!bounds_pay<OP>(t->view, st, a.n)) return false;
+  a.victim_tries = victim_tries<OP>(t->view, a.n);
   BoundsRebuild r{};
   r.clock = t->clock;
   r.strategy = st;
@@ -787,7 +815,7 @@ int run_upsert(hkv_table* t, UpsertArgs a, int vec, bool hybrid_rule, hipStream_
        * the batch is retried instead of skipped) */
       writes_scores_outside_bounds(t, s, own_rule);
       launch_upsert<OP>({true, false, pair, repeats}, vec, t->view, a, s);
-    } else if (prepare_bounds(t, a, s)) {
+    } else if (prepare_bounds<OP>(t, a, s)) {
       launch_upsert<OP>({false, true, pair, repeats}, vec, t->view, a, s);
     } else {
       writes_scores_outside_bounds(t, s, own_rule);

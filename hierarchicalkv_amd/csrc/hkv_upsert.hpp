@@ -78,6 +78,7 @@ struct UpsertArgs {
   uint64_t bound_cap;
   const unsigned long long* bound_cap_in;
   unsigned long long* bound_cap_out;
+  int32_t victim_tries; /* slots a new key of a full bucket tries in one trip (victim_tries in hkv_table.hip) */
   /* strategies whose scores come from the caller (Customized, LFU, EpochLFU): a device word that
    * no bound of the table is above.  A key that writes a score below it lowers the bound of
    * its line itself.  Null where scores only grow (LRU, EpochLRU). */
@@ -550,8 +551,6 @@ __device__ __forceinline__ void bulk_evicted(int kind, const uint8_t* src, uint8
  * 128-bit mask of EMPTY digests.  Every lane of the wavefront must call this.
  */
 constexpr int kMaxLockedWaits = 64;
-/* slots a new key of a full bucket tries in one trip (searches through the score bounds) */
-constexpr int kVictimAttempts = 4;
 template <int R = kTile>
 __device__ __forceinline__ void settle_reprobes(const View& v, uint64_t key, uint32_t bkt,
                                                 uint32_t digest, bool pending, bool& reprobe,
@@ -889,7 +888,7 @@ upsert_kernel(View v, UpsertArgs a) {
       SlotSet lost{0, 0};
       bool again = try_victim && got == kStNone;
 #pragma unroll 1
-      for (int attempt = 1; attempt < kVictimAttempts && __ballot(again); attempt++) {
+      for (int attempt = 1; attempt < a.victim_tries && __ballot(again); attempt++) {
         if (again) lost.add(bpos);
         uint32_t need = tile_ballot(again, tile);
         const int lane_base = lane & ~(kTile - 1);
@@ -907,9 +906,11 @@ upsert_kernel(View v, UpsertArgs a) {
             uint64_t b = bd;
             uint32_t g = (uint32_t)j;
             tile_min_pair(b, g);
-            uint64_t b0, nb0;
-            uint32_t p0;
-            bounded_min(v, bs0, tile, j, bd, g, line_load(v, bs0, g, j), bound_cap, skip, b0, p0, nb0);
+            uint64_t b0 = kMaxScore, nb0 = 0;
+            uint32_t p0 = 0;
+            /* (with no bound below the limit no score is) */
+            if (b < bound_cap)
+              bounded_min(v, bs0, tile, j, bd, g, line_load(v, bs0, g, j), bound_cap, skip, b0, p0, nb0);
             if (j == r0) {
               best = b0;
               bpos = p0;

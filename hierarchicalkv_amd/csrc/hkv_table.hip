@@ -689,9 +689,11 @@ bool bounds_pay(const View& v, int strategy, uint64_t n) {
 }
 /* Slots that a new key of a full bucket tries in one trip (hkv_upsert.hpp).  With more new keys per bucket
  * most tries find the slot taken again (capacity 2^21, LRU, rows of 64 bytes, four tries / one: 16 keys per
- * bucket 156/147 us, 32 470/384, 64 1488/1019; insert_and_evict 205/293, 549/663, 1743/1557). */
+ * bucket 156/147 us, 32 470/384, 64 1488/1019; insert_and_evict 205/293, 549/663, 1743/1557), and under LFU
+ * equal counts leave nothing below the limit to try (2^16 keys 41/30 us, insert_and_evict 55/52). */
 template <int OP>
-int victim_tries(const View& v, uint64_t n) {
+int victim_tries(const View& v, int strategy, uint64_t n) {
+  if (strategy == HKV_LFU || strategy == HKV_EPOCH_LFU) return 1;
   return n <= (OP == kOpInsertAndEvict ? 32 : 16) * v.buckets_num ? 4 : 1;
 }
 
@@ -727,7 +729,7 @@ bool prepare_bounds(hkv_table* t, UpsertArgs& a, hipStream_t s) {
     t->bounds_era = now >> 52;
   }
   if (!bounds_pay<OP>(t->view, st, a.n)) return false;
-  a.victim_tries = victim_tries<OP>(t->view, a.n);
+  a.victim_tries = victim_tries<OP>(t->view, st, a.n);
   BoundsRebuild r{};
   r.clock = t->clock;
   r.strategy = st;

@@ -680,12 +680,17 @@ uint64_t host_realtime_ns() {
  *                  insert_and_evict     73/104   116/165   205/341    549/590   1743/1085
  *   capacity 2^17, insert_or_assign               47/39     79/63     157/116    632/204     4259/376
  * (EpochLRU has its line higher: its scores go back with the epoch, and a scan then leaves the bounds to
- * be made again, a pass over the table.) */
+ * be made again, a pass over the table.)
+ * Customized: every scan does, so a table keeps to one of the two.  Where the scores do not grow, the lowest of
+ * a batch is a limit far below most of the table, and every search opens all lines (2^17 keys, half of
+ * them new, capacity 2^21, insert_or_assign 182/54, insert_and_evict 238/118; with growing scores 77/68 and
+ * 102/135).  Rows of no multiple of 16 bytes take the scan.  The pointer overload moves no rows and is as on
+ * any table. */
 template <int OP>
 bool bounds_pay(const View& v, int strategy, uint64_t n) {
   if (strategy == HKV_LRU) return n <= (OP == kOpInsertAndEvict ? 32 : 24) * v.buckets_num;
   if (strategy == HKV_EPOCH_LRU) return n <= 48 * v.buckets_num;
-  return true;
+  return strategy != HKV_CUSTOMIZED || v.value_bytes % 16 == 0 || OP == kOpFindOrInsertPtr;
 }
 /* Slots that a new key of a full bucket tries in one trip (hkv_upsert.hpp).  With more new keys per bucket
  * most tries find the slot taken again (capacity 2^21, LRU, rows of 64 bytes, four tries / one: 16 keys per

@@ -64,27 +64,32 @@ void launch_upsert_for(bool pair, int vec, const View& v, const UpsertArgs& a, h
   launch_form<OP, R, LOCKED_RULE, BOUNDS, 1>(vec, v, a, s);
 }
 
-/* Keys per tile.  With 8 a wavefront holds 64 keys in 110 to 128 registers and takes them through the
- * victim search and the row copies one or two at a time, so that a batch of a few ten thousand keys
- * is a long chain on part of the chip; with fewer keys per tile the chain is shorter, more wavefronts
- * fit on a SIMD, and every step is issued for fewer keys at once, which is what costs once the chip is
- * full anyway.  us for the whole step, R = 8 / 2 / 1 (with one try for a victim per trip; the tries that
- * follow in the same trip now take 3 to 15 % off each):
- *   full table (bounds), insert_or_assign with half of the keys new, and find, rows of 256 bytes
- *     2^12 keys   68 /  36 /  31      2^16   84 /  54 /  51      2^18  127 / 116 / 120
- *     2^14        71 /  41 /  36      2^17   97 /  74 /  73      2^20  393 / 397 / 438
- *   the same with nearly all keys found, 2^19 keys of 64 bytes: 123 / 132 / 151
- *   full table, insert_and_evict, rows of 64 bytes
- *     2^15 keys  128 /  92 /  88      2^17  151 / 122 / 139      2^18  186 / 167 / 207
- *   table with free slots, find_or_insert and insert_or_assign of repeated ids, 512 (2^18: 128) bytes
- *     2^15 keys   88 /  81 /  81      2^17  145 / 136 / 143      2^18  133 / 147 / 156
- * The last line is what `repeats` is for: there is no search for a victim to shorten, and a good part
- * of the keys has been crossed off beforehand. */
+/* Keys per tile.  With 8 a wavefront takes 64 keys through the victim search and the row copies one or two at
+ * a time, so that a batch of a few ten thousand keys is a long chain on part of the chip; with fewer
+ * keys per tile the chain is shorter, and every step is issued for fewer keys at once, which is what
+ * costs once the chip is full anyway.  (Registers hardly come into it: insert_or_assign with bounds is
+ * compiled to 124 with eight, 97 with two, 95 with one, i.e. 4, 4 and 5 wavefronts per SIMD.)  us per call,
+ * eight / two / one, LRU, rows of 64 bytes; the order is the same for 256:
+ *            capacity 2^24, full, half of the keys found          ... 95 % found           a third full, all found
+ *            insert_or_assign    insert_and_evict      insert_or_assign   insert_and_evict   insert_or_assign
+ *   2^12     29 / 15 / 13        38 / 23 / 20          29 / 15 / 13       37 / 23 / 20       14 /  9 /  8
+ *   2^14     30 / 18 / 16        42 / 25 / 24          33 / 20 / 17       42 / 26 / 25       14 / 11 / 10
+ *   2^15     38 / 25 / 22        48 / 31 / 33          40 / 25 / 23       49 / 34 / 33       16 / 12 / 12
+ *   2^16     43 / 29 / 31        63 / 45 / 53          43 / 30 / 31       65 / 45 / 53       19 / 15 / 18
+ *   2^17     71 / 55 / 54        92 / 76 / 88          59 / 49 / 51       89 / 73 / 86       25 / 25 / 31
+ *   2^18    104 / 93 / 96       120 / 117 / 144        74 / 76 / 82       74 / 92 / 130      36 / 44 / 55
+ *   2^20    345 / 333 / 348     431 / 437 / 531       173 / 211 / 238    205 / 267 / 364    142 / 160 / 217
+ * The line at 2^18: with many new keys per bucket two per tile are far ahead there (capacity 2^21, all keys new,
+ * 216 / 145); what they lose where nearly all keys are found, on a table that only has been offered nine
+ * tenths of its slots for instance, is less.  accum_or_assign searches for few victims (a key that is to be
+ * added to and is not there changes nothing): 2^17 keys 25 / 22 / 26, 2^18 35 / 41 / 53; and a batch that came
+ * with repeated ids (`repeats`) has many of its keys crossed off: 2^18 133 / 147 / 156 with the passes over the
+ * ids.  Both take eight above 2^17. */
 template <int OP, bool BOUNDS>
 void launch_by_size(bool pair, bool repeats, int vec, const View& v, const UpsertArgs& a, hipStream_t s) {
   if (a.n <= (UINT64_C(1) << (BOUNDS ? 15 : 14)))
     launch_upsert_for<OP, false, BOUNDS, 1>(pair, vec, v, a, s);
-  else if (a.n <= (UINT64_C(1) << (BOUNDS && !repeats ? 18 : 17)))
+  else if (a.n <= (UINT64_C(1) << (BOUNDS && !repeats && OP != kOpAccumOrAssign ? 18 : 17)))
     launch_upsert_for<OP, false, BOUNDS, 2>(pair, vec, v, a, s);
   else
     launch_upsert_for<OP, false, BOUNDS, kTile>(pair, vec, v, a, s);

@@ -692,14 +692,27 @@ bool bounds_pay(const View& v, int strategy, uint64_t n) {
   if (strategy == HKV_EPOCH_LRU) return n <= 48 * v.buckets_num;
   return strategy != HKV_CUSTOMIZED || v.value_bytes % 16 == 0 || OP == kOpFindOrInsertPtr;
 }
-/* Slots that a new key of a full bucket tries in one trip (hkv_upsert.hpp).  With more new keys per bucket
- * most tries find the slot taken again (capacity 2^21, LRU, rows of 64 bytes, four tries / one: 16 keys per
- * bucket 156/147 us, 32 470/384, 64 1488/1019; insert_and_evict 205/293, 549/663, 1743/1557), and under LFU
- * equal counts leave nothing below the limit to try (2^16 keys 41/30 us, insert_and_evict 55/52). */
+/* Slots that a new key of a full bucket tries in one trip (hkv_upsert.hpp).  The more new keys a bucket gets,
+ * the more tries find the slot taken again; with eight keys per tile (above 2^18 keys) a try is made for one
+ * key after the other.  insert_and_evict, whose trips end at a barrier, gains most.  us per call with one /
+ * two / four tries, LRU, all keys new, rows of 64 bytes:
+ *                          insert_or_assign     insert_and_evict
+ *   2^17 keys,  2 a bucket    57 /   57 /   56    103 /   81 /   76
+ *               8             85 /   83 /   89    165 /  117 /  117
+ *   2^18 keys,  4             97 /   97 /   98    179 /  139 /  132
+ *              16            146 /  145 /  157    293 /  202 /  205
+ *   2^20 keys,  2            290 /  289 /  289    368 /  339 /  332
+ *               8            342 /  355 /  376    483 /  432 /  452
+ *              32            502 /  538 /  605    835 /  641 /  719
+ * (2^15 keys, 2 a bucket: 34 / 31 / 30 and 71 / 54 / 46.)  Under LFU equal counts leave nothing below the limit
+ * to try (2^16 keys, one / four: 30/41, insert_and_evict 52/55). */
 template <int OP>
 int victim_tries(const View& v, int strategy, uint64_t n) {
   if (strategy == HKV_LFU || strategy == HKV_EPOCH_LFU) return 1;
-  return n <= (OP == kOpInsertAndEvict ? 32 : 16) * v.buckets_num ? 4 : 1;
+  const bool many = n > (UINT64_C(1) << 18);
+  if (OP == kOpInsertAndEvict) return many ? 2 : n <= 32 * v.buckets_num ? 4 : 1;
+  if (many) return n <= 2 * v.buckets_num ? 2 : 1;
+  return n <= 4 * v.buckets_num ? 4 : n <= 16 * v.buckets_num ? 2 : 1;
 }
 
 /* Whether this upsert searches victims through the score bounds, and with which limits (the

@@ -80,16 +80,15 @@ void launch_upsert_for(bool pair, int vec, const View& v, const UpsertArgs& a, h
  *   2^18    104 / 93 / 96       120 / 117 / 144        74 / 76 / 82       74 / 92 / 130      36 / 44 / 55
  *   2^20    345 / 333 / 348     431 / 437 / 531       173 / 211 / 238    205 / 267 / 364    142 / 160 / 217
  * The line at 2^18: with many new keys per bucket two per tile are far ahead there (capacity 2^21, all keys new,
- * 216 / 145); what they lose where nearly all keys are found, on a table that only has been offered nine
- * tenths of its slots for instance, is less.  accum_or_assign searches for few victims (a key that is to be
- * added to and is not there changes nothing): 2^17 keys 25 / 22 / 26, 2^18 35 / 41 / 53; and a batch that came
- * with repeated ids (`repeats`) has many of its keys crossed off: 2^18 133 / 147 / 156 with the passes over the
- * ids.  Both take eight above 2^17. */
+ * 216 / 145; accum_or_assign, half of them, 153 / 117); what they lose where nearly all keys are found, on a
+ * table that only has been offered nine tenths of its slots for instance, is less (accum_or_assign of keys
+ * that are all there or change nothing: 35 / 41).  A batch that came with repeated ids (`repeats`) has many of
+ * its keys crossed off and takes eight above 2^17: 2^18 keys 133 / 147 / 156 with the passes over the ids. */
 template <int OP, bool BOUNDS>
 void launch_by_size(bool pair, bool repeats, int vec, const View& v, const UpsertArgs& a, hipStream_t s) {
   if (a.n <= (UINT64_C(1) << (BOUNDS ? 15 : 14)))
     launch_upsert_for<OP, false, BOUNDS, 1>(pair, vec, v, a, s);
-  else if (a.n <= (UINT64_C(1) << (BOUNDS && !repeats && OP != kOpAccumOrAssign ? 18 : 17)))
+  else if (a.n <= (UINT64_C(1) << (BOUNDS && !repeats ? 18 : 17)))
     launch_upsert_for<OP, false, BOUNDS, 2>(pair, vec, v, a, s);
   else
     launch_upsert_for<OP, false, BOUNDS, kTile>(pair, vec, v, a, s);

@@ -16,28 +16,28 @@ template <int OP, int R, bool LOCKED_RULE, bool BOUNDS = false, int WAVES = 1, b
 void launch_form(int vec, const View& v, const UpsertArgs& a, hipStream_t s) {
   constexpr uint64_t kKeys = (uint64_t)kTilesPerWave * R * WAVES;
   const dim3 grid((unsigned)((a.n + kKeys - 1) / kKeys)), block(kWave * WAVES);
-  if constexpr (OP == kOpFindOrInsertPtr) {
+  if constexpr (OP == kOpFindOrInsertPtr) { /* moves no rows */
     launch_main(upsert_kernel<OP, 16, 1, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a);
-    return;
-  }
-  constexpr bool kAdds = OP == kOpAccumOrAssign;
-  constexpr int kWide = kAdds ? 16 : kAny + 16;
-  constexpr int kNarrowUpl = kAdds ? 8 : 1; /* the others' rows have no more than two units of less than 16 bytes */
-  if (vec_bytes(vec) == 16) {
-    switch (pick_upl(v.value_bytes)) {
-      case 1: launch_main(upsert_kernel<OP, kWide, 1, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
-      case 2: launch_main(upsert_kernel<OP, kWide, 2, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
-      case 4: launch_main(upsert_kernel<OP, kWide, 4, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
-      default: launch_main(upsert_kernel<OP, kWide, 8, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+  } else {
+    constexpr bool kAdds = OP == kOpAccumOrAssign;
+    constexpr int kWide = kAdds ? 16 : kAny + 16;
+    if (vec_bytes(vec) == 16) {
+      switch (pick_upl(v.value_bytes)) {
+        case 1: launch_main(upsert_kernel<OP, kWide, 1, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+        case 2: launch_main(upsert_kernel<OP, kWide, 2, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+        case 4: launch_main(upsert_kernel<OP, kWide, 4, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+        default: launch_main(upsert_kernel<OP, kWide, 8, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+      }
+      return;
     }
-    return;
-  }
-  constexpr int kNarrow = kAdds ? 0 : kAny;
-  switch (vec_bytes(vec)) {
-    case 8: launch_main(upsert_kernel<OP, kNarrow + 8, kNarrowUpl, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
-    case 4: launch_main(upsert_kernel<OP, kNarrow + 4, kNarrowUpl, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
-    case 2: launch_main(upsert_kernel<OP, kNarrow + 2, kNarrowUpl, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
-    default: launch_main(upsert_kernel<OP, 1, kNarrowUpl, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+    constexpr int kNarrow = kAdds ? 0 : kAny;
+    constexpr int kUpl = kAdds ? 8 : 1; /* the others' rows have no more than two units of less than 16 bytes */
+    switch (vec_bytes(vec)) {
+      case 8: launch_main(upsert_kernel<OP, kNarrow + 8, kUpl, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+      case 4: launch_main(upsert_kernel<OP, kNarrow + 4, kUpl, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+      case 2: launch_main(upsert_kernel<OP, kNarrow + 2, kUpl, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+      default: launch_main(upsert_kernel<OP, 1, kUpl, LOCKED_RULE, BOUNDS, WAVES, HOLD, R>, grid, block, s, v, a); break;
+    }
   }
 }
 

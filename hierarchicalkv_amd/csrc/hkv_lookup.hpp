@@ -26,8 +26,6 @@
 #ifndef HKV_LOOKUP_HPP_
 #define HKV_LOOKUP_HPP_
 
-#include <type_traits>
-
 #include "hkv_common.hpp"
 
 namespace hkv {

@@ -31,12 +31,26 @@ def body(buf, shift, n, vb):
     (1, 0), (2, 1), (3, 0), (4, 0), (6, 1), (8, 4), (12, 0), (15, 1), (16, 0), (16, 1), (17, 0), (40, 0), (66, 1), (128, 4),
     (132, 0), (200, 0), (256, 0), (260, 4), (512, 1), (516, 0), (1024, 0), (1030, 0), (2100, 1)])
 def test_rows_of_every_size(oracle, row_bytes, shift):
+    check(oracle, row_bytes, shift, 1 << 30)
+
+
+# no row in HBM and half of them: unaligned units to and from host memory, slots held to the end of the launch
+@pytest.mark.parametrize("hbm_share", [0, 0.5])
+@pytest.mark.parametrize("row_bytes,shift", [
+    (1, 0), (2, 1), (3, 0), (6, 1), (12, 0), (15, 1), (16, 0), (17, 4), (40, 0), (66, 1), (200, 0), (260, 4), (516, 1), (1030, 0)])
+def test_rows_in_host_memory(oracle, row_bytes, shift, hbm_share):
+    check(oracle, row_bytes, shift, int((1 << 13) * row_bytes * hbm_share))
+
+
+def check(oracle, row_bytes, shift, hbm):
     cap = 1 << 13
-    o = default_options(init_capacity=cap, max_capacity=cap, max_hbm_for_vectors=1 << 30, dim=row_bytes,
+    hybrid = hbm < cap * row_bytes
+    o = default_options(init_capacity=cap, max_capacity=cap, max_hbm_for_vectors=hbm, dim=row_bytes,
                         value_kind=0, value_size=1)
     t = HashTable()
     t.init(o)
-    ot = oracle.OracleTable(o)
+    assert t.is_pure_hbm() != hybrid
+    ot = oracle.OracleTable(o, hybrid)
     t.set_clock(1, 1 << 44)
     ot.set_clock(1, 1 << 44)
     rng = np.random.default_rng(row_bytes * 8 + shift)
@@ -51,6 +65,8 @@ def test_rows_of_every_size(oracle, row_bytes, shift):
         rows = rng.integers(0, 256, (n, row_bytes), dtype=np.uint8)
         buf, dv = placed(rows, shift)
         op = ("insert_or_assign", "find_or_insert", "insert_and_evict")[step % 3]
+        if hybrid and op == "insert_and_evict":  # (pure HBM only)
+            op = "insert_or_assign"
         if op == "insert_or_assign":
             t.insert_or_assign(n, dev(keys), dv)
             ot.insert_or_assign(keys, rows, None)

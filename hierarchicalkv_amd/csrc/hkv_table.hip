@@ -695,23 +695,28 @@ bool bounds_pay(const View& v, int strategy, uint64_t n) {
 /* Slots that a new key of a full bucket tries in one trip (hkv_upsert.hpp).  The more new keys a bucket gets,
  * the more tries find the slot taken again; with eight keys per tile (above 2^18 keys) a try is made for one
  * key after the other.  insert_and_evict, whose trips end at a barrier, gains most.  us per call with one /
- * two / four tries, LRU, all keys new, rows of 64 bytes:
- *                          insert_or_assign     insert_and_evict
- *   2^17 keys,  2 a bucket    57 /   57 /   56    103 /   81 /   76
- *               8             85 /   83 /   89    165 /  117 /  117
- *   2^18 keys,  4             97 /   97 /   98    179 /  139 /  132
- *              16            146 /  145 /  157    293 /  202 /  205
- *   2^20 keys,  2            290 /  289 /  289    368 /  339 /  332
- *               8            342 /  355 /  376    483 /  432 /  452
- *              32            502 /  538 /  605    835 /  641 /  719
- * (2^15 keys, 2 a bucket: 34 / 31 / 30 and 71 / 54 / 46.)  Under LFU equal counts leave nothing below the limit
- * to try (2^16 keys, one / four: 30/41, insert_and_evict 52/55). */
+ * two / four tries, LRU, rows of 64 bytes:
+ *                        insert_or_assign                        insert_and_evict
+ *                        half of the keys new    all             half                   all
+ *   2^17 keys,  4 a bucket   50 /  49 /  48    64 /  63 /  65    106 /  86 /  80    136 / 105 / 102
+ *              16            73 /  70 /  72   113 / 112 / 122    161 / 118 / 113    238 / 169 / 173
+ *   335 299,    5           107 / 102 / 104   149 / 149 / 157    189 / 149 / 145    251 / 205 / 212
+ *   2^20 keys,  2           225 / 217 / 216   287 / 286 / 288    313 / 285 / 280    371 / 339 / 332
+ *               4           244 / 240 / 239   317 / 325 / 334    334 / 302 / 295    412 / 369 / 372
+ *               8           259 / 256 / 258   343 / 355 / 377    370 / 327 / 322    496 / 449 / 468
+ *              16           270 / 265 / 271   384 / 403 / 437    431 / 349 / 349    613 / 512 / 551
+ *              32           296 / 296 / 296   506 / 507 / 507    553 / 408 / 417    844 / 655 / 732
+ * Rows of 200 bytes, 335 299 keys, 5 a bucket: 155 / 148 / 148 and 191 / 189 / 197; of 256, 2^20 keys, 8 a
+ * bucket: 280 / 269 / 267 and 382 / 387 / 414.  The call does not know how many of its keys are new; above
+ * eight per bucket two tries cost a call of new keys more than they give one with half of them.
+ * (2^15 keys, 2 a bucket, all new: 34 / 31 / 30 and 71 / 54 / 46.)  Under LFU equal counts leave nothing below the
+ * limit to try (2^16 keys, one / four: 30/41, insert_and_evict 52/55). */
 template <int OP>
 int victim_tries(const View& v, int strategy, uint64_t n) {
   if (strategy == HKV_LFU || strategy == HKV_EPOCH_LFU) return 1;
   const bool many = n > (UINT64_C(1) << 18);
   if (OP == kOpInsertAndEvict) return many ? 2 : n <= 32 * v.buckets_num ? 4 : 1;
-  if (many) return n <= 2 * v.buckets_num ? 2 : 1;
+  if (many) return n <= 8 * v.buckets_num ? 2 : 1;
   return n <= 4 * v.buckets_num ? 4 : n <= 16 * v.buckets_num ? 2 : 1;
 }
 

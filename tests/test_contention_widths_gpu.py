@@ -128,10 +128,12 @@ def run(strategy, cap, n, dim, hybrid=False, steps=7):
     t.close()
 
 
-# some nine keys of a call per bucket: the searches through the bounds, with several tries in a trip; rows of
-# 16 bytes and of 36 (whose units overlap)
+# some nine keys of a call per bucket: the searches through the bounds, with two tries in a trip where tiles have
+# two keys and with one where they have eight, which make two with five keys per bucket; rows of 16 bytes and of 36
+# (whose units overlap)
 @pytest.mark.parametrize("strategy,dim", [(LRU, 4), (LRU, 9), (ELRU, 9), (CUSTOM, 4), (CUSTOM, 9), (LFU, 4), (ELFU, 9)])
-@pytest.mark.parametrize("cap,n", [(1 << 19, 40000), (1 << 22, (1 << 18) + 33000)], ids=["two-per-tile", "eight-per-tile"])
+@pytest.mark.parametrize("cap,n", [(1 << 19, 40000), (1 << 22, (1 << 18) + 33000), (1 << 23, (1 << 18) + 33000)],
+                         ids=["two-per-tile", "eight-per-tile", "eight-per-tile-two-tries"])
 def test_bounded_searches(cap, n, strategy, dim):
     run(strategy, cap, n, dim)
 

@@ -709,13 +709,23 @@ bool bounds_pay(const View& v, int strategy, uint64_t n) {
  * Rows of 200 bytes, 335 299 keys, 5 a bucket: 155 / 148 / 148 and 191 / 189 / 197; of 256, 2^20 keys, 8 a
  * bucket: 280 / 269 / 267 and 382 / 387 / 414.  The call does not know how many of its keys are new; above
  * eight per bucket two tries cost a call of new keys more than they give one with half of them.
- * (2^15 keys, 2 a bucket, all new: 34 / 31 / 30 and 71 / 54 / 46.)  Under LFU equal counts leave nothing below the
- * limit to try (2^16 keys, one / four: 30/41, insert_and_evict 52/55). */
+ * (2^15 keys, 2 a bucket, all new: 34 / 31 / 30 and 71 / 54 / 46.)
+ * Where slots are held to the end of the launch (rows in host memory) another trip costs more, and four tries pay
+ * up to eight keys per bucket at any size; half of the rows in host memory:
+ *                                       insert_or_assign                        find_or_insert
+ *                                       half of the keys new    all             half                   all
+ *    40 000 keys,  5 a bucket, 32 bytes     52 /  51 /  46     60 /  60 /  60     68 /  65 /  60     60 /  60 /  60
+ *   300 000,       5           64          260 / 254 / 251    262 / 260 / 259    306 / 298 / 288    271 / 268 / 266
+ *   300 000,       9           32          207 / 201 / 197    228 / 225 / 241    308 / 303 / 294    213 / 213 / 231
+ *    30 000,      15           64           62 /  60 /  58     81 /  78 /  86     72 /  70 /  66     80 /  78 /  86
+ * Under LFU equal counts leave nothing below the limit to try (2^16 keys, one / four: 30/41, insert_and_evict
+ * 52/55). */
 template <int OP>
-int victim_tries(const View& v, int strategy, uint64_t n) {
+int victim_tries(const View& v, int strategy, uint64_t n, bool held) {
   if (strategy == HKV_LFU || strategy == HKV_EPOCH_LFU) return 1;
   const bool many = n > (UINT64_C(1) << 18);
   if (OP == kOpInsertAndEvict) return many ? 2 : n <= 32 * v.buckets_num ? 4 : 1;
+  if (held) return n <= 8 * v.buckets_num ? 4 : n <= 16 * v.buckets_num ? 2 : 1;
   if (many) return n <= 8 * v.buckets_num ? 2 : 1;
   return n <= 4 * v.buckets_num ? 4 : n <= 16 * v.buckets_num ? 2 : 1;
 }
@@ -752,7 +762,7 @@ bool prepare_bounds(hkv_table* t, UpsertArgs& a, hipStream_t s) {
     t->bounds_era = now >> 52;
   }
   if (!bounds_pay<OP>(t->view, st, a.n)) return false;
-  a.victim_tries = victim_tries<OP>(t->view, st, a.n);
+  a.victim_tries = victim_tries<OP>(t->view, st, a.n, a.held_scores != nullptr);
   BoundsRebuild r{};
   r.clock = t->clock;
   r.strategy = st;

@@ -47,9 +47,9 @@ void launch_lookup_by(int vec, const View& v, const FindArgs& a, hipStream_t s) 
   }
 }
 
-/* Keys per tile.  A wavefront of 64 keys (R = 8) holds 114 registers, four of them fit on a SIMD, and
- * a tile does much of its work on its 8 keys one after the other; with 2 keys per tile it is 48
- * registers, eight wavefronts, and a quarter of the chain.  us per call (hits 7/8, cold):
+/* Keys per tile.  A wavefront of 64 keys (R = 8) was compiled to 114 registers, four of them fit on a SIMD,
+ * and a tile does much of its work on its 8 keys one after the other; with 2 keys per tile it is 48
+ * registers, eight wavefronts, and a quarter of the chain (with 1, 33).  us per call (hits 7/8, cold):
  *   keys     row        R = 8    2      1
  *   2^20    256 bytes    119    112    115
  *   2^20     32           73     68     84
@@ -59,10 +59,15 @@ void launch_lookup_by(int vec, const View& v, const FindArgs& a, hipStream_t s) 
  *   500     256            9.6    4.6    3.8
  *   2^20   no rows (contains)  51  46.5  58
  * One key per tile where that leaves the chip room (a quarter of its 8192 wave slots at 2^14 keys)
- * or where the rows outweigh the probes. */
+ * or where the rows outweigh the probes.  us per call with two / one (7/8 found):
+ *   row         171 667 keys     500 000 keys
+ *   256 bytes   20.6 / 21.8      52.4 / 54.3
+ *   320         27.1 / 27.3      68.9 / 68.9
+ *   400         33.5 / 33.0      86.3 / 84.9
+ *   480         37.2 / 36.0      97.0 / 93.6 */
 template <int MODE>
 void launch_lookup(int vec, const View& v, const FindArgs& a, hipStream_t s) {
-  if (a.n <= (UINT64_C(1) << 14) || (MODE == kLookupValues && v.value_bytes >= 512))
+  if (a.n <= (UINT64_C(1) << 14) || (MODE == kLookupValues && v.value_bytes >= 384))
     launch_lookup_by<MODE, 1>(vec, v, a, s);
   else
     launch_lookup_by<MODE, 2>(vec, v, a, s);

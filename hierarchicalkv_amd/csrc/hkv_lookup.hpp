@@ -279,6 +279,9 @@ enum LookupMode { kLookupValues = 0, kLookupPtr = 1, kLookupContains = 2 };
  * 2^38) and the key's number in its wavefront. */
 constexpr int kFoundShift = 56;
 constexpr uint64_t kFoundSlot = (UINT64_C(1) << kFoundShift) - 1;
+/* a key that was not found: reads slot 0's row, and its place is past the end of any wavefront's rows (a row is at
+ * most 2^20 bytes) */
+constexpr uint64_t kListedMiss = UINT64_C(0xFF) << kFoundShift;
 
 /* Where the rows of the table are; an address is one multiply-add in the first case (slot numbers fit 32 bits
  * there).  A lane past the end of the list reads a row that the caches have: the first key's; slot 0's, in
@@ -414,15 +417,22 @@ lookup_kernel(View v, FindArgs a) {
    * loads than a store needs.
    * With a step for every key instead of for the found ones, misses cost most of what hits do: 2^20 keys,
    * none found, rows of 256 bytes 50 -> 34 us, of 1024 128 -> 43; half found, rows of 64 bytes 56 -> 49;
-   * all found, 256 bytes 103 both ways.  (Half found, rows of 1024 bytes and more: up to 5 % the other way,
-   * as wavefronts have unequal numbers of rows to move.) */
+   * all found, 256 bytes 103 both ways.  Where at least three quarters of a wavefront's keys are found, the others
+   * are listed too: with gaps in the list a store covers parts of lines that the next one completes.  2^19
+   * keys, 7/8 found, rows of 512 bytes 90.5 -> 88.8, of 1024 172 -> 168; 2^20 of 400 174 -> 171; rows of 256 bytes and
+   * less the same both ways; with the line at half, half found, 400 bytes 110 -> 118. */
   const unsigned long long hits = __ballot(my_slot >= 0);
   if (hits == 0) return;
+  constexpr uint32_t kKeys = kTilesPerWave * R;
+  const bool most = v.hbm_slots != 0 && (uint32_t)__popcll(hits) * 4 >= kKeys * 3;
+  const bool listed = most ? i < a.n : my_slot >= 0;
+  const unsigned long long all = __ballot(listed);
   uint64_t* const s_found = reinterpret_cast<uint64_t*>(s_slot); /* every lane has read its slot */
-  if (my_slot >= 0)
-    s_found[__popcll(hits & ((1ull << lane) - 1))] = (uint64_t)my_slot | ((i - base) << kFoundShift);
+  if (listed)
+    s_found[__popcll(all & ((1ull << lane) - 1))] =
+        my_slot >= 0 ? (uint64_t)my_slot | ((i - base) << kFoundShift) : kListedMiss;
   wave_sync();
-  const uint32_t count = (uint32_t)__popcll(hits);
+  const uint32_t count = (uint32_t)__popcll(all);
   if (v.hbm_slots >= v.capacity && v.capacity <= 0xFFFFFFFFull)
     copy_found_rows<VEC, R, kRowsHbm>(v, s_found, count, a.out_values, base, a.n, lane);
   else if (v.hbm_slots != 0)

@@ -25,7 +25,7 @@
  *            tile, reduce inside the lane and then over the tile) and the
  *            value-row copies, issued for several keys before the first result
  *            is awaited.  How much is in flight per wavefront is weighed
- *            against registers: at 118 registers four wavefronts share a SIMD,
+ *            against registers: at 124 registers four wavefronts share a SIMD,
  *            and that is worth more here than deeper batches per wavefront.
  *
  * Lock discipline on a SIMD machine: every lock taken in a trip of the retry
@@ -430,8 +430,8 @@ constexpr int kRowUnits = 8;
  * Bulk row traffic of one trip.  Round q of a tile is the key owned by lane q
  * of the tile: `move` says what to do with it, `tab` is its table row, `usr`
  * the caller's row.  All loads of a group of rounds are issued before the
- * first store; a group holds 16 units per lane (64 VGPRs at 16-byte units),
- * i.e. the whole trip for rows up to 256 bytes.
+ * first store; a group holds 8 units per lane (32 VGPRs at 16-byte units),
+ * i.e. the whole trip for rows up to 128 bytes, or, with two keys per tile, 512.
  * UPL = units per lane and row held in registers (1, 2, 4 or 8).
  * Units may overlap within a row (kAny) where rows are moved as they are, not where they are added to.
  * Every lane of the wavefront must call this.

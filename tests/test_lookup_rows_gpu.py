@@ -33,11 +33,12 @@ def test_rows_in_host_memory(row_bytes, shift, hbm_share):
 
 # no key found, few, half of them, nearly all and all: the copy's list of found keys at its edges, for rows of less
 # than a unit's 16 bytes, of a part of a wavefront's step of 1024 bytes, of one step and of more; the missed-keys
-# form too
+# form too.  A quarter missed: wavefronts on both sides of the line where misses are listed as well; rows of 383 and 384
+# bytes: two keys and one per tile
 @pytest.mark.parametrize("missed_form", [False, True])
-@pytest.mark.parametrize("row_bytes", [4, 12, 16, 40, 64, 256, 512, 1024, 1040, 4096])
+@pytest.mark.parametrize("row_bytes", [4, 12, 16, 40, 64, 256, 383, 384, 512, 1024, 1040, 4096])
 def test_any_share_of_hits(row_bytes, missed_form):
-    for miss_share in (1.0, 0.97, 0.5, 0.03, 0.0):
+    for miss_share in (1.0, 0.97, 0.5, 0.25, 0.03, 0.0):
         check(row_bytes, 0, 1 << 34, (1, 8, 17, 65, 1000, 16385), miss_share, missed_form)
 
 

@@ -184,7 +184,7 @@ struct hkv_table {
   unsigned long long* d_counters; /* scratch words for size / size_if / the count-returning
                                      insert_and_evict: one per call in flight (CounterLease) */
   unsigned long long* h_words; /* pinned: a word per word of d_counters that hands its value to the
-                                  host, then the one fast_load_factor reads */
+                                  host, then the one fast_load_factor reads and the falls of bounds_pay() */
   mutable std::mutex counter_mu;
   mutable std::condition_variable counter_cv;
   mutable std::vector<unsigned> counter_free;
@@ -681,16 +681,20 @@ uint64_t host_realtime_ns() {
  *   capacity 2^17, insert_or_assign               47/39     79/63     157/116    632/204     4259/376
  * (EpochLRU has its line higher: its scores go back with the epoch, and a scan then leaves the bounds to
  * be made again, a pass over the table.)
- * Customized: every scan does, so a table keeps to one of the two.  Where the scores do not grow, the lowest of
- * a batch is a limit far below most of the table, and every search opens all lines (2^17 keys, half of
+ * Customized: every scan does, so a table does not go back and forth.  Where the scores do not grow, the lowest
+ * of a batch is a limit far below most of the table, and every search opens all lines (2^17 keys, half of
  * them new, capacity 2^21, insert_or_assign 182/54, insert_and_evict 238/118; with growing scores 77/68 and
- * 102/135).  Rows of no multiple of 16 bytes take the scan.  The pointer overload moves no rows and is as on
- * any table. */
+ * 102/135).  Rows of no multiple of 16 bytes start with the bounds and take the scan, until the table is
+ * cleared, once a few calls have come with a lower lowest score than a call before: `falls`, which a kernel
+ * counts and nobody waits for, as both searches find the same victims.  The pointer overload moves no rows and is
+ * as on any table. */
+constexpr uint64_t kMostFalls = 3;
 template <int OP>
-bool bounds_pay(const View& v, int strategy, uint64_t n) {
+bool bounds_pay(const View& v, int strategy, uint64_t n, const unsigned long long* falls) {
   if (strategy == HKV_LRU) return n <= (OP == kOpInsertAndEvict ? 32 : 24) * v.buckets_num;
   if (strategy == HKV_EPOCH_LRU) return n <= 48 * v.buckets_num;
-  return strategy != HKV_CUSTOMIZED || v.value_bytes % 16 == 0 || OP == kOpFindOrInsertPtr;
+  if (strategy != HKV_CUSTOMIZED || v.value_bytes % 16 == 0 || OP == kOpFindOrInsertPtr) return true;
+  return __atomic_load_n(falls, __ATOMIC_RELAXED) <= kMostFalls;
 }
 /* Slots that a new key of a full bucket tries in one trip (hkv_upsert.hpp).  The more new keys a bucket gets,
  * the more tries find the slot taken again; with eight keys per tile (above 2^18 keys) a try is made for one
@@ -761,7 +765,9 @@ bool prepare_bounds(hkv_table* t, UpsertArgs& a, hipStream_t s) {
     t->bounds_epoch = t->epoch;
     t->bounds_era = now >> 52;
   }
-  if (!bounds_pay<OP>(t->view, st, a.n)) return false;
+  unsigned long long* const falls = t->h_words + kCounterWords + 1;
+  if (!bounds_pay<OP>(t->view, st, a.n, falls)) return false;
+  if (st == HKV_CUSTOMIZED && t->view.value_bytes % 16) a.falls = falls;
   a.victim_tries = victim_tries<OP>(t->view, st, a.n, a.held_scores != nullptr);
   BoundsRebuild r{};
   r.clock = t->clock;
@@ -1261,10 +1267,11 @@ int create_impl(const hkv_options* o, const hkv_allocator* al, hkv_table** out) 
   }
   t->d_counters = (unsigned long long*)cnt;
   {
-    const hipError_t e = hipHostMalloc((void**)&t->h_words, (kCounterWords + 1) * sizeof(unsigned long long),
+    const hipError_t e = hipHostMalloc((void**)&t->h_words, (kCounterWords + 2) * sizeof(unsigned long long),
                                        hipHostMallocDefault);
     if (e != hipSuccess) return bail(fail(HKV_ERROR_HIP, "hipHostMalloc: %s", hipGetErrorString(e)));
   }
+  t->h_words[kCounterWords + 1] = 0;
   for (unsigned w = 0; w < kCounterWords; w++) t->counter_free.push_back(w);
   t->counter_dirty.assign(kCounterWords, 0);
   t->d_bound_caps = t->d_counters + kCounterWords;
@@ -1868,6 +1875,7 @@ int hkv_clear(hkv_table* t, hkv_stream_t stream) {
   t->keys_may_be_locked = false;
   t->locked_recount = false;
   t->keys_offered = 0;
+  __atomic_store_n(t->h_words + kCounterWords + 1, 0, __ATOMIC_RELAXED);
   t->bounds_stale = true;
   hipLaunchKernelGGL(zero_locked_kernel, dim3(1), dim3(kLockedShards), 0, s, t->d_locked);
   const uint64_t groups = t->view.capacity / 16;

@@ -78,6 +78,7 @@ struct UpsertArgs {
   uint64_t bound_cap;
   const unsigned long long* bound_cap_in;
   unsigned long long* bound_cap_out;
+  unsigned long long* falls; /* Customized, may be null: a word of host memory that counts the calls with a lower limit than one before */
   int32_t victim_tries; /* slots a new key of a full bucket tries in one trip (victim_tries in hkv_table.hip) */
   /* strategies whose scores come from the caller (Customized, LFU, EpochLFU): a device word that
    * no bound of the table is above.  A key that writes a score below it lowers the bound of
@@ -644,7 +645,13 @@ upsert_kernel(View v, UpsertArgs a) {
        * call sets by its limit */
       const uint64_t c = *a.bound_ceil;
       bound_ceil = c > bound_cap ? c : bound_cap;
-      if (blockIdx.x == 0 && threadIdx.x == 0 && bound_cap > c) *a.bound_ceil = bound_cap;
+      if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (bound_cap > c) *a.bound_ceil = bound_cap;
+        /* (one call at a time uses the bounds of a table: nobody else changes the word) */
+        if (bound_cap < c && a.falls)
+          __hip_atomic_store(a.falls, 1 + __hip_atomic_load(a.falls, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM),
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
     }
   }
   const uint64_t key = stage_keys(v, a.keys, a.n, i, s_meta, s_slot, lane);

@@ -390,6 +390,34 @@ def test_customized_calls_without_scores(oracle, row_bytes):
     t.close()
 
 
+@pytest.mark.parametrize("row_bytes", [8, 36])
+def test_customized_scores_that_stop_growing(oracle, row_bytes):
+    """Rows of no multiple of 16 bytes: searches through the bounds while the lowest score of a call is above the ones
+    before, full scans after some calls where it is not, and bounds again once the table has been cleared."""
+    cap, bs, dim = 1 << 13, 2048, row_bytes // 4
+    t, o = make(cap, dim, EvictStrategy.kCustomized)
+    for again in range(2):
+        ot = oracle.OracleTable(o)
+        pos, batch = 0, 10
+        while pos < cap + 4 * bs:
+            k = w.unique_keys(670 + again, pos, bs)
+            upsert(t, ot, k, w.values_from_keys(k, dim), w.monotone_scores(batch, bs, seed=67))
+            pos += bs
+            batch += 1
+        ok, bad, n_tight = bounds_hold(t)
+        assert ok and n_tight > 0, (again, bad)
+        assert_same_table(t, ot, row_bytes)
+        for step in range(12):
+            k = one_per_bucket(oracle, w.unique_keys(680 + again, step * 400, 400), cap // 128)
+            low = batch - step if step % 4 else batch + step  # falling, with a rise now and then
+            upsert(t, ot, k, w.values_from_keys(k, dim), w.monotone_scores(low, len(k), seed=67))
+            torch.cuda.synchronize()
+            assert_same_table(t, ot, row_bytes)
+        t.clear()
+        assert t.size() == 0
+    t.close()
+
+
 @pytest.mark.parametrize("strategy", [EvictStrategy.kLfu, EvictStrategy.kEpochLfu])
 def test_frequency_scores_and_bounds(oracle, strategy):
     """LFU / EpochLFU: a new key comes in with the caller's count, which under LFU may be below

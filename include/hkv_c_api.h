@@ -164,9 +164,9 @@ int hkv_table_create_with_allocator(const hkv_options* opts,
 int hkv_table_destroy(hkv_table* t);
 
 /* unique_key (here and below): 1 = the caller guarantees that no key occurs twice in the
- * batch; 0 = keys may repeat: the batch is first reduced to one occurrence per key (device
- * sort, temporary memory from the stream's pool), as the reference's kernels for such
- * batches leave every key in the table once.  A dual-bucket table needs 1
+ * batch; 0 = keys may repeat: the batch is first reduced to one occurrence per key (a device
+ * index of the batch, temporary memory from the stream's pool), as the reference's kernels
+ * for such batches leave every key in the table once.  A dual-bucket table needs 1
  * (merlin_hashtable.cuh:1167-1169).
  *
  * HashTable::insert_or_assign, merlin_hashtable.cuh:1125-1305.  On a table with rows in host

@@ -5,8 +5,8 @@
  * (merlin_hashtable.cuh:1194-1252, 1737-1790, 1925-1960): every occurrence is applied,
  * in no particular order, and the table ends up holding the key once (tests/
  * find_or_insert_ptr_test.cc.cu:3390-3475: 1024 copies of one key leave one entry).  Here
- * the batch is reduced to one occurrence per key before the ordinary kernels run: the first
- * occurrence stands for the key, and the other occurrences travel as the EMPTY key, which
+ * the batch is reduced to one occurrence per key: the first
+ * occurrence stands for the key, and the upsert takes the others for the EMPTY key, which
  * every kernel skips.  Calls that hand something back per key (find_or_insert) copy it from
  * the representative afterwards.
  *
@@ -14,13 +14,14 @@
  * settles the repetitions among its own keys in LDS and brings one entry per key to the index in
  * device memory, so that a key that makes up a fifteenth of a batch (ids of a recommender are
  * Zipf-distributed) costs one atomic per workgroup and not one per occurrence: atomics on one word
- * are served one at a time, about 15 ns each.  An entry is a word of 32 hash bits and the index of
+ * are served one at a time, about 15 ns each.  An entry is a word of 16 hash bits, the number of the call and the index of
  * the lowest occurrence seen so far: a minimum on the word keeps the lowest one, and keys are only
- * fetched for comparison where the hash bits agree.  It is bound by one 8-byte atomic on a random
+ * fetched for comparison where the hash bits agree.  An entry of another call counts as free, so that the index, which a
+ * table keeps, is cleared once in 65 535 calls, and the upsert looks up for itself whether a key stands for the others
+ * of its kind: a launch of its own takes 4 us however little it does.  What is left is bound by one 8-byte atomic on a random
  * line per distinct key of a workgroup and by the queue at the most frequent keys.
- * 2^18 keys of 32 floats, Zipf(1.05) over 2^21 ids, the whole find_or_insert + insert_or_assign:
- * 0.383 ms with a radix sort of (key, index) and a running maximum (18 launches, 0.125 ms a batch),
- * 0.13 ms as it is here (clear 4, enter 18, mark 5 us).
+ * 2^18 keys of 32 floats, Zipf(1.05) over 2^21 ids, the whole find_or_insert + insert_or_assign: 129 us with a clear
+ * before and a pass over the keys behind every call's index (3.5 and 4.5 us), 116 as it is here.
  */
 #ifndef HKV_DEDUP_HPP_
 #define HKV_DEDUP_HPP_
@@ -29,14 +30,8 @@
 
 namespace hkv {
 
-struct DedupPlan {
-  uint64_t* keys = nullptr; /* [n] the batch with later occurrences replaced by EMPTY */
-  uint32_t* rep = nullptr;  /* [n] index of the occurrence that stands for key i */
-  void* block = nullptr;
-  hipStream_t stream = nullptr;
-};
-
-constexpr uint64_t kDedupFree = UINT64_C(0xFFFFFFFFFFFFFFFF);
+/* entries that no call has made */
+constexpr uint32_t kNoCall = 0xFFFF;
 
 __global__ void __launch_bounds__(256)
 dedup_clear_kernel(uint64_t* index, uint64_t words) {
@@ -45,11 +40,12 @@ dedup_clear_kernel(uint64_t* index, uint64_t words) {
 }
 
 /* Enters every key of the batch; at[i] = the place in the index of key i's entry.  `mask` + 1
- * entries, at least twice as many as keys, so that a free one always ends the search.  One key per
+ * entries, at least twice as many as keys, so that a free one always ends the search; two neighbours, which one load brings,
+ * are tried before the next pair.  One key per
  * thread: two or four of them meant fewer, longer workgroups and were slower at every size. */
 template <int THREADS>
 __global__ void __launch_bounds__(THREADS)
-dedup_enter_kernel(const uint64_t* keys, uint64_t n, uint64_t* index, uint64_t mask, uint32_t* at) {
+dedup_enter_kernel(const uint64_t* keys, uint64_t n, uint64_t* index, uint64_t mask, uint32_t call, uint32_t* at) {
   constexpr uint32_t kPlaces = 2 * THREADS; /* half of them stay free */
   __shared__ uint64_t s_key[THREADS];
   __shared__ uint32_t s_index[kPlaces]; /* lowest thread with the key, ~0: free */
@@ -59,12 +55,12 @@ dedup_enter_kernel(const uint64_t* keys, uint64_t n, uint64_t* index, uint64_t m
   const bool valid = i < n;
   const uint64_t key = valid ? keys[i] : 0;
   const uint64_t h = fmix64(key);
-  /* the place and the hash bits of the entry have no bit in common below 2^31 keys */
-  uint64_t where = (h >> 32) & mask;
-  const uint64_t mine = (h << 32) | i;
-  /* How the place looks now: an entry stays where it is once it is there, so whatever stands
+  /* the place and the hash bits of the entry have no bit in common below 2^31 keys (2^47 entries) */
+  uint64_t where = (h >> 16) & mask;
+  const uint64_t mine = (h << 48) | ((uint64_t)call << 32) | i;
+  /* How the places look now: an entry of this call stays where it is once it is there, so whatever stands
    * there needs no atomic.  The load is under way while the workgroup sorts out its own keys. */
-  unsigned long long ahead = index[where];
+  uint4 pair = *reinterpret_cast<const uint4*>(index + (where & ~UINT64_C(1)));
   s_key[l] = key;
   s_index[l] = s_index[l + THREADS] = ~0u;
   __syncthreads();
@@ -81,32 +77,27 @@ dedup_enter_kernel(const uint64_t* keys, uint64_t n, uint64_t* index, uint64_t m
   __syncthreads();
   if (valid && s_index[place] == l) {
     unsigned long long* const words = reinterpret_cast<unsigned long long*>(index);
-    for (;;) {
-      const unsigned long long old =
-          ahead != kDedupFree ? ahead : atomicCAS(words + where, (unsigned long long)kDedupFree, (unsigned long long)mine);
-      ahead = kDedupFree;
-      if (old == kDedupFree) break;
-      if ((uint32_t)(old >> 32) == (uint32_t)h && keys[(uint32_t)old] == key) {
+    for (uint32_t tried = 1;; tried++) {
+      unsigned long long old = (where & 1) ? (pair.z | ((unsigned long long)pair.w << 32)) : (pair.x | ((unsigned long long)pair.y << 32));
+      if ((uint32_t)(old >> 32 & 0xFFFF) != call) {
+        const unsigned long long stale = old;
+        old = atomicCAS(words + where, stale, (unsigned long long)mine);
+        if (old == stale) break;
+      }
+      if ((old >> 32) == (mine >> 32) && keys[(uint32_t)old] == key) {
         if (i < (uint32_t)old) atomicMin(words + where, (unsigned long long)mine);
         break;
       }
-      where = (where + 1) & mask;
+      where ^= 1;
+      if ((tried & 1) == 0) {
+        where = ((where | 1) + 1) & mask;
+        pair = *reinterpret_cast<const uint4*>(index + where);
+      }
     }
     s_at[l] = (uint32_t)where;
   }
   __syncthreads();
   if (valid) at[i] = s_at[s_index[place]];
-}
-
-/* `rep` comes in as the place of every key's entry and becomes the occurrence that stands for it */
-__global__ void __launch_bounds__(256)
-dedup_mark_kernel(const uint64_t* keys, uint64_t n, const uint64_t* index, uint64_t empty_key, uint64_t* keys_mod,
-                  uint32_t* rep) {
-  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const uint32_t first = (uint32_t)index[rep[i]];
-  rep[i] = first;
-  keys_mod[i] = first == (uint32_t)i ? keys[i] : empty_key;
 }
 
 /* what a duplicate gets back: the representative's pointer and flag ... */
@@ -154,41 +145,53 @@ inline void dedup_fix_rows(const uint32_t* rep, uint64_t n, uint8_t* rows, uint3
     dedup_fix_rows_by<uint8_t>(rep, n, rows, row_bytes, s);
 }
 
-inline void dedup_free(DedupPlan& d) {
-  if (d.block) (void)hipFreeAsync(d.block, d.stream);
-  d.block = nullptr;
+/* The index of a batch: memory for `keys` keys and the number of the last call that used it. */
+struct RepeatIndex {
+  uint8_t* block = nullptr;
+  uint64_t keys = 0;
+  uint32_t call = 0;
+};
+inline uint64_t repeat_entries(uint64_t keys) {
+  uint64_t entries = 64;
+  while (entries < 2 * keys) entries *= 2;
+  return entries;
+}
+inline hipError_t repeat_index_make(RepeatIndex& x, uint64_t keys, hipStream_t s) {
+  const uint64_t entries = repeat_entries(keys);
+  const hipError_t e = hipMallocAsync((void**)&x.block, entries * 8 + keys * 4, s);
+  if (e != hipSuccess) {
+    x.block = nullptr;
+    return e;
+  }
+  x.keys = keys;
+  x.call = kNoCall; /* to be cleared */
+  return hipSuccess;
+}
+inline void repeat_index_free(RepeatIndex& x, hipStream_t s) {
+  if (x.block) (void)hipFreeAsync(x.block, s);
+  x = RepeatIndex{};
 }
 
-/* Builds d.keys and d.rep for the n keys of a batch on stream s (n < 2^31). */
-inline hipError_t dedup_make(const View& v, uint64_t n, const uint64_t* keys, hipStream_t s,
-                             DedupPlan& d) {
-  d.stream = s;
-  auto up = [](uint64_t x) { return (x + 255) & ~UINT64_C(255); };
-  uint64_t entries = 64;
-  while (entries < 2 * n) entries *= 2;
-  const uint64_t o_rep = up(n * 8);
-  const uint64_t o_index = o_rep + up(n * 4);
-  hipError_t e = hipMallocAsync(&d.block, o_index + entries * 8, s);
-  if (e != hipSuccess) return e;
-  uint8_t* b = (uint8_t*)d.block;
-  d.keys = (uint64_t*)b;
-  d.rep = (uint32_t*)(b + o_rep);
-  uint64_t* index = (uint64_t*)(b + o_index);
-  hipLaunchKernelGGL(dedup_clear_kernel, dim3((unsigned)((entries / 2 + 255) / 256)), dim3(256), 0, s, index, entries);
+/* Enters the n keys of a batch (n < 2^31, at most x.keys) on stream s; the upsert gets `index` and `rep`. */
+inline void repeat_index_enter(RepeatIndex& x, uint64_t n, const uint64_t* keys, hipStream_t s, const uint64_t*& index_out,
+                               uint32_t*& rep) {
+  const uint64_t all = repeat_entries(x.keys), entries = repeat_entries(n);
+  uint64_t* const index = (uint64_t*)x.block;
+  rep = (uint32_t*)(x.block + all * 8);
+  index_out = index;
+  if (++x.call >= kNoCall) {
+    hipLaunchKernelGGL(dedup_clear_kernel, dim3((unsigned)((all / 2 + 255) / 256)), dim3(256), 0, s, index, all);
+    x.call = 0;
+  }
   /* Large workgroups keep the queues at the frequent keys short (2^20 keys: 48 us with 1024 threads,
    * 90 with 256), small ones get more CUs to work on a small batch (2^12 keys: 4 and 7 us; the
    * lines cross between 2^15 and 2^16). */
   if (n >= (UINT64_C(1) << 15))
     hipLaunchKernelGGL(dedup_enter_kernel<1024>, dim3((unsigned)((n + 1023) / 1024)), dim3(1024), 0, s, keys, n, index,
-                       entries - 1, d.rep);
+                       entries - 1, x.call, rep);
   else
     hipLaunchKernelGGL(dedup_enter_kernel<256>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, keys, n, index,
-                       entries - 1, d.rep);
-  hipLaunchKernelGGL(dedup_mark_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, keys, n,
-                     (const uint64_t*)index, v.empty_key, d.keys, d.rep);
-  e = hipGetLastError();
-  if (e != hipSuccess) dedup_free(d);
-  return e;
+                       entries - 1, x.call, rep);
 }
 
 }  // namespace hkv

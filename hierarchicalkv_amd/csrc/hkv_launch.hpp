@@ -53,7 +53,7 @@ struct UpsertForm {
   bool locked_rule; /* LOCKED slots may sit in the table: the victim scan reads key words too */
   bool bounds;      /* victims are searched through the score bounds */
   bool pair;        /* insert_and_evict: the wavefronts of a workgroup share their claims */
-  bool repeats;     /* the batch came with repeated keys, which travel as the EMPTY key */
+  bool repeats;     /* the batch may repeat keys, of which all but the first count as the EMPTY key */
 };
 template <int OP>
 void launch_upsert(const UpsertForm& form, int vec, const View& v, const UpsertArgs& a, hipStream_t s);

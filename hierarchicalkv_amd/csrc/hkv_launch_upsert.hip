@@ -83,7 +83,8 @@ void launch_upsert_for(bool pair, int vec, const View& v, const UpsertArgs& a, h
  * 216 / 145; accum_or_assign, half of them, 153 / 117); what they lose where nearly all keys are found, on a
  * table that only has been offered nine tenths of its slots for instance, is less (accum_or_assign of keys
  * that are all there or change nothing: 35 / 41).  A batch that came with repeated ids (`repeats`) has many of
- * its keys crossed off and takes eight above 2^17: 2^18 keys 133 / 147 / 156 with the passes over the ids. */
+ * its keys crossed off and takes eight above 2^17: 2^18 keys 133 / 147 / 156 with the passes over the ids (three launches
+ * per call then, one now: 116 with eight). */
 template <int OP, bool BOUNDS>
 void launch_by_size(bool pair, bool repeats, int vec, const View& v, const UpsertArgs& a, hipStream_t s) {
   if (a.n <= (UINT64_C(1) << (BOUNDS ? 15 : 14)))

@@ -179,6 +179,7 @@ struct hkv_table {
   uint64_t bounds_epoch = 0; /* EpochLRU: epoch and era (clock >> 52: the low half of such a score */
   uint64_t bounds_era = 0;   /* wraps once per era) of the last call that used the bounds */
   uint64_t meta_bytes;
+  RepeatIndex repeats;   /* of batches that may repeat keys, up to kMostKeptKeys; used under the inserter role */
   void* d_values;        /* value rows in HBM */
   void* h_values;        /* host address of the pinned value rows (hybrid) */
   unsigned long long* d_counters; /* scratch words for size / size_if / the count-returning
@@ -811,11 +812,49 @@ bool prepare_bounds(hkv_table* t, UpsertArgs& a, hipStream_t s) {
   return true;
 }
 
+/* unique_key == false: the keys of the batch are entered into an index (hkv_dedup.hpp), the table's own where the call has the
+ * table to itself and the batch is not too long to keep the memory for (40 MB), else one that goes with the call: `own`
+ * frees it, on the stream.  A call that is being recorded into a graph runs again with the same number, so it takes one
+ * that it clears. */
+constexpr uint64_t kMostKeptKeys = UINT64_C(1) << 21;
+struct CallRepeats {
+  RepeatIndex own;
+  hipStream_t stream = nullptr;
+  ~CallRepeats() { repeat_index_free(own, stream); }
+};
+int check_repeats(uint64_t n, bool repeats) {
+  if (repeats && n >= (UINT64_C(1) << 31))
+    return fail(HKV_ERROR_UNSUPPORTED, "unique_key = false needs a batch below 2^31 keys");
+  return HKV_SUCCESS;
+}
+int enter_repeats(hkv_table* t, UpsertArgs& a, hipStream_t s, bool alone, CallRepeats& call) {
+  if (a.n < 2) return HKV_SUCCESS;
+  RepeatIndex* x = &call.own;
+  hipError_t e = hipSuccess;
+  if (alone && t->opts.api_lock && a.n <= kMostKeptKeys && !capturing(s)) {
+    x = &t->repeats;
+    if (x->keys < a.n) {
+      repeat_index_free(*x, s);
+      uint64_t keys = UINT64_C(1) << 12;
+      while (keys < a.n) keys *= 2;
+      e = repeat_index_make(*x, keys, s);
+    }
+  } else {
+    call.stream = s;
+    e = repeat_index_make(*x, a.n, s);
+  }
+  if (e != hipSuccess) return fail(HKV_ERROR_HIP, "duplicate-key pass: %s", hipGetErrorString(e));
+  repeat_index_enter(*x, a.n, a.keys, s, a.repeat_index, a.repeat_of);
+  HKV_HIP(hipGetLastError());
+  return HKV_SUCCESS;
+}
+
 /* `hybrid_rule`: the operation follows the lock-key kernels of hybrid mode when
  * the table is not pure HBM (insert_or_assign, find_or_insert); the pointer
  * overload always does. */
 template <int OP>
 int run_upsert(hkv_table* t, UpsertArgs a, int vec, bool hybrid_rule, hipStream_t s, bool repeats = false) {
+  HKV_TRY(check_repeats(a.n, repeats));
   HKV_TRY(grow_for(t, a.n, s));
   a.epoch = t->epoch;
   a.clock = t->clock;
@@ -825,9 +864,11 @@ int run_upsert(hkv_table* t, UpsertArgs a, int vec, bool hybrid_rule, hipStream_
   const bool own_rule = a.strategy == t->opts.evict_strategy;
   t->keys_offered += a.n;
   {
+    CallRepeats call;
     LockGuard g(t, StreamGroupLock::kInserter, s);
     HKV_HIP(g.acquire());
     HKV_TRY(settle_locked_count(t, s));
+    if (repeats) HKV_TRY(enter_repeats(t, a, s, true, call));
     if (OP == kOpFindOrInsertPtr && a.locked_key_ptrs) t->keys_may_be_locked = true;
     /* a table that has been offered fewer keys than nine tenths of its slots evicts next to nothing */
     const bool pair = OP == kOpInsertAndEvict && t->keys_offered * 10 >= t->view.capacity * 9;
@@ -872,6 +913,15 @@ int run_upsert(hkv_table* t, UpsertArgs a, int vec, bool hybrid_rule, hipStream_
       (void)hipFreeAsync(held, s);
     }
     HKV_HIP(e);
+    if (a.repeat_of) {
+      /* the other occurrences of a key get what its representative ended up with: the row that it read or inserted (a
+       * refused key keeps its own, like its representative), or the pointer and the flag */
+      if (OP == kOpFindOrInsert) dedup_fix_rows(a.repeat_of, a.n, a.values_io, t->view.value_bytes, s);
+      if (OP == kOpFindOrInsertPtr)
+        hipLaunchKernelGGL(dedup_fix_ptrs_kernel, dim3((unsigned)((a.n + 255) / 256)), dim3(256), 0, s,
+                           (const uint32_t*)a.repeat_of, a.n, a.out_ptrs, a.founds);
+      HKV_HIP(hipGetLastError());
+    }
   }
   if (t->clock.mode == 1) t->clock.base += UINT64_C(1) << 40;
   return HKV_SUCCESS;
@@ -959,7 +1009,8 @@ __global__ void cpu_io_owner_kernel(View v, const uint64_t* keys, uint8_t** ptrs
 }
 
 /* insert_or_assign (reads == false) and find_or_insert (reads == true) */
-int cpu_io_upsert(hkv_table* t, UpsertArgs a, void* values, bool reads, hipStream_t s) {
+int cpu_io_upsert(hkv_table* t, UpsertArgs a, void* values, bool reads, bool repeats, hipStream_t s) {
+  HKV_TRY(check_repeats(a.n, repeats));
   HKV_TRY(grow_for(t, a.n, s));
   const uint64_t n = a.n, vb = t->view.value_bytes;
   std::lock_guard<std::mutex> host_lock(t->io_mutex);
@@ -974,10 +1025,18 @@ int cpu_io_upsert(hkv_table* t, UpsertArgs a, void* values, bool reads, hipStrea
   a.value_kind = t->opts.value_kind;
   a.refuse_equal = 0;
   hipError_t e = hipSuccess;
+  CallRepeats call;
+  if (repeats) {
+    const int rc = enter_repeats(t, a, s, false, call);
+    if (rc) {
+      (void)hipFreeAsync(d_tmp, s);
+      return rc;
+    }
+  }
   {
     LockGuard g(t, StreamGroupLock::kInserter, s);
     e = g.acquire();
-    if (e == hipSuccess) e = hipMemsetAsync(d_tmp, 0, n * 9, s); /* reserved / refused keys: no address */
+    if (e == hipSuccess) e = hipMemsetAsync(d_tmp, 0, n * 9, s); /* reserved, repeated and refused keys: no address */
     if (e == hipSuccess) {
       writes_scores_outside_bounds(t, s, a.strategy == t->opts.evict_strategy);
       launch_upsert<kOpFindOrInsertPtr>({true, false, false}, 16, t->view, a, s);
@@ -1005,6 +1064,10 @@ int cpu_io_upsert(hkv_table* t, UpsertArgs a, void* values, bool reads, hipStrea
   }
   (void)hipFreeAsync(d_tmp, s);
   HKV_HIP(e);
+  if (reads && a.repeat_of) {
+    dedup_fix_rows(a.repeat_of, n, (uint8_t*)values, (uint32_t)vb, s);
+    HKV_HIP(hipGetLastError());
+  }
   if (t->clock.mode == 1) t->clock.base += UINT64_C(1) << 40;
   return HKV_SUCCESS;
 }
@@ -1019,27 +1082,6 @@ int refuse_dual(const hkv_table* t, const char* what, bool guarded) {
   if (!t->dual) return HKV_SUCCESS;
   return fail(guarded ? HKV_ERROR_CHECK : HKV_ERROR_UNSUPPORTED,
               "[MEMORY_MODE] %s is not supported in dual-bucket mode.", what);
-}
-
-/* unique_key == false: the batch is reduced to one occurrence per key first; `keys` then
- * points at the reduced copy, which lives until the guard goes out of scope (stream-ordered). */
-struct DedupGuard {
-  DedupPlan d;
-  bool on = false;
-  ~DedupGuard() {
-    if (on) dedup_free(d);
-  }
-};
-int maybe_dedup(const hkv_table* t, int unique_key, uint64_t n, const uint64_t*& keys,
-                hipStream_t s, DedupGuard& g) {
-  if (unique_key || n < 2) return HKV_SUCCESS;
-  if (n >= (UINT64_C(1) << 31))
-    return fail(HKV_ERROR_UNSUPPORTED, "unique_key = false needs a batch below 2^31 keys");
-  const hipError_t e = dedup_make(t->view, n, keys, s, g.d);
-  if (e != hipSuccess) return fail(HKV_ERROR_HIP, "duplicate-key pass: %s", hipGetErrorString(e));
-  g.on = true;
-  keys = g.d.keys;
-  return HKV_SUCCESS;
 }
 
 /* Where a key lands depends on the bucket sizes the moment it is handled, and the keys in
@@ -1331,6 +1373,7 @@ int hkv_table_destroy(hkv_table* t) {
   if (!t) return HKV_SUCCESS;
   (void)hipSetDevice(t->device);
   (void)hipDeviceSynchronize();
+  if (t->repeats.block) (void)hipFree(t->repeats.block);
   table_free(t, 0, t->d_meta);
   table_free(t, 0, t->d_counters);
   table_free(t, 0, t->d_values);
@@ -1347,8 +1390,6 @@ int hkv_insert_or_assign(hkv_table* t, uint64_t n, const uint64_t* keys,
   if (n == 0) return HKV_SUCCESS;
   const int strategy = ignore ? HKV_CUSTOMIZED : t->opts.evict_strategy;
   if (!ignore) HKV_TRY(check_scores_arg(t, strategy, scores));
-  DedupGuard dg;
-  if (!t->dual) HKV_TRY(maybe_dedup(t, unique_key, n, keys, (hipStream_t)stream, dg));
   UpsertArgs a{};
   a.keys = keys;
   a.values_in = (const uint8_t*)values;
@@ -1373,7 +1414,7 @@ int hkv_insert_or_assign(hkv_table* t, uint64_t n, const uint64_t* keys,
     if (t->clock.mode == 1) t->clock.base += UINT64_C(1) << 40;
     return HKV_SUCCESS;
   }
-  if (t->io_by_cpu) return cpu_io_upsert(t, a, const_cast<void*>(values), false, (hipStream_t)stream);
+  if (t->io_by_cpu) return cpu_io_upsert(t, a, const_cast<void*>(values), false, !unique_key, (hipStream_t)stream);
   /* with unique_key == false the reference leaves its lock-key kernels for the plain one
    * (merlin_hashtable.cuh:1235-1258), whose rule is "refuse when score < min" */
   const int vec = lookup_unit(t->view.value_bytes, values);
@@ -1455,8 +1496,6 @@ int hkv_insert_and_evict(hkv_table* t, uint64_t n, const uint64_t* keys,
     return fail(HKV_ERROR_RUNTIME, "Only support pure HBM mode for insert_and_evict.");
   const int strategy = ignore ? HKV_CUSTOMIZED : t->opts.evict_strategy;
   if (!ignore) HKV_TRY(check_scores_arg(t, strategy, scores));
-  DedupGuard dg;
-  HKV_TRY(maybe_dedup(t, unique_key, n, keys, (hipStream_t)stream, dg));
   UpsertArgs a{};
   a.keys = keys;
   a.values_in = (const uint8_t*)values;
@@ -1517,8 +1556,6 @@ int hkv_find_or_insert(hkv_table* t, uint64_t n, const uint64_t* keys,
   if (n == 0) return HKV_SUCCESS;
   const int strategy = ignore ? HKV_CUSTOMIZED : t->opts.evict_strategy;
   if (!ignore) HKV_TRY(check_scores_arg(t, strategy, scores));
-  DedupGuard dg;
-  HKV_TRY(maybe_dedup(t, unique_key, n, keys, (hipStream_t)stream, dg));
   UpsertArgs a{};
   a.keys = keys;
   a.values_io = (uint8_t*)values;
@@ -1526,17 +1563,9 @@ int hkv_find_or_insert(hkv_table* t, uint64_t n, const uint64_t* keys,
   a.n = n;
   a.strategy = strategy;
   const int vec = lookup_unit(t->view.value_bytes, values);
-  if (t->io_by_cpu)
-    HKV_TRY(cpu_io_upsert(t, a, values, true, (hipStream_t)stream));
-  else /* merlin_hashtable.cuh:1779-1803: lock-key kernels only with unique keys */
-    HKV_TRY(run_upsert<kOpFindOrInsert>(t, a, vec, unique_key != 0, (hipStream_t)stream, !unique_key));
-  if (dg.on) {
-    /* the other occurrences of a key get the row its representative ended up with (what it
-     * read, or what it inserted; a refused key keeps its own row, like its representative) */
-    dedup_fix_rows(dg.d.rep, n, (uint8_t*)values, t->view.value_bytes, (hipStream_t)stream);
-    HKV_HIP(hipGetLastError());
-  }
-  return HKV_SUCCESS;
+  if (t->io_by_cpu) return cpu_io_upsert(t, a, values, true, !unique_key, (hipStream_t)stream);
+  /* merlin_hashtable.cuh:1779-1803: lock-key kernels only with unique keys */
+  return run_upsert<kOpFindOrInsert>(t, a, vec, unique_key != 0, (hipStream_t)stream, !unique_key);
 }
 
 int hkv_find_or_insert_ptr_lock(hkv_table* t, uint64_t n, const uint64_t* keys, void** values,
@@ -1566,8 +1595,6 @@ int hkv_find_or_insert_ptr(hkv_table* t, uint64_t n, const uint64_t* keys,
   if (n == 0) return HKV_SUCCESS;
   const int strategy = ignore ? HKV_CUSTOMIZED : t->opts.evict_strategy;
   if (!ignore) HKV_TRY(check_scores_arg(t, strategy, scores));
-  DedupGuard dg;
-  HKV_TRY(maybe_dedup(t, unique_key, n, keys, (hipStream_t)stream, dg));
   UpsertArgs a{};
   a.keys = keys;
   a.out_ptrs = values;
@@ -1575,13 +1602,7 @@ int hkv_find_or_insert_ptr(hkv_table* t, uint64_t n, const uint64_t* keys,
   a.scores = scores;
   a.n = n;
   a.strategy = strategy;
-  HKV_TRY(run_upsert<kOpFindOrInsertPtr>(t, a, 16, true, (hipStream_t)stream));
-  if (dg.on) {
-    hipLaunchKernelGGL(dedup_fix_ptrs_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                       (hipStream_t)stream, (const uint32_t*)dg.d.rep, n, values, founds);
-    HKV_HIP(hipGetLastError());
-  }
-  return HKV_SUCCESS;
+  return run_upsert<kOpFindOrInsertPtr>(t, a, 16, true, (hipStream_t)stream, !unique_key);
 }
 
 /* The group lock keeps every other writer off the table while an updater runs; with unique

@@ -84,6 +84,10 @@ struct UpsertArgs {
    * no bound of the table is above.  A key that writes a score below it lowers the bound of
    * its line itself.  Null where scores only grow (LRU, EpochLRU). */
   unsigned long long* bound_ceil;
+  /* a batch that may repeat keys (hkv_dedup.hpp): the index of its keys, and per key where in the index its entry is;
+   * the kernel leaves the occurrence that stands for the key there.  Null: keys are unique */
+  const uint64_t* repeat_index;
+  uint32_t* repeat_of;
 };
 
 /* ScoreFunctor<Strategy>::desired_when_missed, kernel_utils.cuh:275-279,
@@ -654,7 +658,13 @@ upsert_kernel(View v, UpsertArgs a) {
       }
     }
   }
-  const uint64_t key = stage_keys(v, a.keys, a.n, i, s_meta, s_slot, lane);
+  uint64_t staged = a.n; /* keys up to this one count */
+  if (OP != kOpAccumOrAssign && a.repeat_of && i < a.n) {
+    const uint32_t first = (uint32_t)a.repeat_index[a.repeat_of[i]];
+    a.repeat_of[i] = first;
+    if (first != (uint32_t)i) staged = 0; /* another occurrence stands for the key */
+  }
+  const uint64_t key = stage_keys(v, a.keys, staged, i, s_meta, s_slot, lane);
   const uint64_t in_score = (a.scores && i < a.n) ? a.scores[i] : 0;
   s_unsure[lane] = 0;
   __syncthreads();

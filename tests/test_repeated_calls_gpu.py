@@ -1,0 +1,137 @@
+"""Batches that repeat keys, call after call on one table: the index of the batch's keys is the
+table's and is not cleared between calls.  Expected values are worked out here with numpy."""
+import numpy as np
+import pytest
+import torch
+
+import workloads as w
+from gpu_util import DEV, dev, export_table, sort_by_key
+from hierarchicalkv_amd import HashTable, default_options
+
+pytestmark = pytest.mark.gpu
+VB = 16
+
+
+def make(cap, **kw):
+    t = HashTable()
+    t.init(default_options(init_capacity=cap, max_capacity=cap, max_hbm_for_vectors=kw.pop("hbm", 1 << 32), dim=4, **kw))
+    return t
+
+
+def check_call(t, model, universe, n, rng, stream=None):
+    """One find_or_insert and one insert_or_assign of n keys drawn with repetitions; every occurrence reads
+    what the first one reads or brings, and the first one's row stays."""
+    pick = rng.integers(0, len(universe), n)
+    seen, first = np.unique(pick, return_index=True)
+    keys, rows = universe[pick], rng.integers(0, 256, (n, VB), dtype=np.uint8)
+    stand = np.empty(len(universe), np.int64)
+    stand[seen] = first
+    present, stored = model
+    want = np.where(present[pick][:, None], stored[pick], rows[stand[pick]])
+    d_keys, d_rows = dev(keys), dev(rows)
+    torch.cuda.synchronize()
+    t.find_or_insert(n, d_keys, d_rows, unique_key=False, stream=stream)
+    torch.cuda.synchronize()
+    assert (d_rows.cpu().numpy() == want).all(), n
+    present[seen] = True
+    rows2 = rng.integers(0, 256, (n, VB), dtype=np.uint8)
+    d_rows2 = dev(rows2)
+    torch.cuda.synchronize()
+    t.insert_or_assign(n, d_keys, d_rows2, unique_key=False, stream=stream)
+    stored[seen] = rows2[first]
+    torch.cuda.synchronize()
+
+
+def check_table(t, model, universe, cap):
+    present, stored = model
+    gk, gv, _ = sort_by_key(*export_table(t, VB, chunk=cap))
+    o = np.argsort(universe[present])
+    assert (gk == universe[present][o]).all() and (gv == stored[present][o]).all()
+
+
+# sizes that make the index grow, that use a part of it, and that are too long for it to be kept (above 2^21); at 2^15
+# the workgroups of the pass change; on two streams the index goes from one to the other
+@pytest.mark.parametrize("streams", [1, 2])
+def test_index_is_used_again(streams):
+    cap = 1 << 18
+    t = make(cap)
+    rng = np.random.default_rng(streams)
+    universe = w.unique_keys(51, 0, 60000)
+    model = np.zeros(len(universe), bool), np.zeros((len(universe), VB), np.uint8)
+    s = [torch.cuda.Stream() for _ in range(streams)]
+    for k, n in enumerate((3, 1 << 12, (1 << 12) + 1, 40, 1 << 15, (1 << 15) - 1, 70000, 5, (1 << 21) + 3, 1 << 15, 300000, 64)):
+        check_call(t, model, universe, n, rng, s[k % streams])
+    check_table(t, model, universe, cap)
+    t.close()
+
+
+def test_more_calls_than_the_index_can_count():
+    cap = 1 << 10
+    t = make(cap)
+    universe = w.unique_keys(52, 0, 7)
+    model = np.zeros(len(universe), bool), np.zeros((len(universe), VB), np.uint8)
+    rng = np.random.default_rng(3)
+    check_call(t, model, universe, 30, rng)
+    keys = dev(universe[[0, 1, 0, 2, 1, 6]])
+    rows = dev(np.arange(6 * VB, dtype=np.uint8).reshape(6, VB))
+    for _ in range((1 << 16) - 4):  # 65 535 numbers; the next calls see the last of them and the first again
+        t.insert_or_assign(6, keys, rows, unique_key=False)
+    h = rows.cpu().numpy()
+    for k, at in ((0, 0), (1, 1), (2, 3), (6, 5)):
+        model[0][k], model[1][k] = True, h[at]
+    for n in (30, 6, 64, 1, 2, 17):
+        check_call(t, model, universe, n, rng)
+    check_table(t, model, universe, cap)
+    t.close()
+
+
+@pytest.mark.parametrize("kw", [{"api_lock": 0}, {"hbm": 0, "io_by_cpu": 1}], ids=["no_group_lock", "io_by_cpu"])
+def test_index_that_goes_with_the_call(kw):
+    cap = 1 << 14
+    t = make(cap, **kw)
+    rng = np.random.default_rng(9)
+    universe = w.unique_keys(53, 0, 3000)
+    model = np.zeros(len(universe), bool), np.zeros((len(universe), VB), np.uint8)
+    for n in (2, 5000, 33, 9000):
+        check_call(t, model, universe, n, rng)
+    check_table(t, model, universe, cap)
+    t.close()
+
+
+def test_recorded_calls_beside_eager_ones():
+    """A recorded call runs again with the number it was recorded with, on an index of its own."""
+    cap, n = 1 << 14, 5000
+    t = make(cap)
+    rng = np.random.default_rng(4)
+    universe = w.unique_keys(54, 0, 2000)
+    model = np.zeros(len(universe), bool), np.zeros((len(universe), VB), np.uint8)
+    s = torch.cuda.Stream()
+    keys = torch.zeros(n, dtype=torch.int64, device=DEV)
+    rows = torch.zeros(n, VB, dtype=torch.uint8, device=DEV)
+
+    def load():
+        pick = rng.integers(0, len(universe), n)
+        given = rng.integers(0, 256, (n, VB), dtype=np.uint8)
+        keys.copy_(dev(universe[pick]))
+        rows.copy_(dev(given))
+        seen, first = np.unique(pick, return_index=True)
+        model[0][seen], model[1][seen] = True, given[first]
+        torch.cuda.synchronize()
+
+    with torch.cuda.stream(s):
+        check_call(t, model, universe, n, rng)
+        load()
+        t.insert_or_assign(n, keys, rows, unique_key=False)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            t.insert_or_assign(n, keys, rows, unique_key=False)
+        for _ in range(4):
+            load()
+            g.replay()
+            torch.cuda.synchronize()
+            check_table(t, model, universe, cap)
+            check_call(t, model, universe, 4000, rng)
+        check_table(t, model, universe, cap)
+    torch.cuda.synchronize()
+    t.close()

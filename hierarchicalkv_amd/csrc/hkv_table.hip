@@ -1170,10 +1170,8 @@ template <class Pred>
 void launch_export(const hkv_table* t, uint64_t pattern, uint64_t threshold,
                    uint64_t n, uint64_t offset, uint64_t* d_counter,
                    uint64_t* keys, void* values, uint64_t* scores, hipStream_t s) {
-  const unsigned blocks = export_grid(n, kExportThreads);
-  hipLaunchKernelGGL((export_if_kernel<Pred>), dim3(blocks), dim3(kExportThreads), 0, s,
-                     t->view, Pred(), pattern, threshold, offset, n,
-                     (unsigned long long*)d_counter, keys, (uint8_t*)values, scores);
+  launch_export(t->view, Pred(), pattern, threshold, offset, n, (unsigned long long*)d_counter, keys, (uint8_t*)values,
+                scores, s);
 }
 
 template <class Pred>

@@ -161,16 +161,15 @@ __device__ __forceinline__ void export_rows_any(const hkv_table_view& v, uint64_
  * reserved and for which pred(key, score, pattern, threshold) holds.  `values` and
  * `scores` may be null.
  */
-constexpr int kExportThreads = 256;
-template <class Pred>
-__global__ void __launch_bounds__(kExportThreads)
+template <class Pred, int THREADS>
+__global__ void __launch_bounds__(THREADS)
 export_if_kernel(hkv_table_view v, Pred pred, uint64_t pattern,
                  uint64_t threshold, uint64_t offset, uint64_t n,
                  unsigned long long* counter, uint64_t* out_keys,
                  uint8_t* out_values, uint64_t* out_scores) {
-  constexpr int kChunk = kExportThreads * kExportPerThread;
+  constexpr int kChunk = THREADS * kExportPerThread;
   __shared__ uint16_t s_src[kChunk];
-  __shared__ uint32_t s_wave[kExportThreads / kWave];
+  __shared__ uint32_t s_wave[THREADS / kWave];
   __shared__ unsigned long long s_base;
   const int tid = threadIdx.x;
   const uint64_t chunks = (n + kChunk - 1) / kChunk;
@@ -179,7 +178,7 @@ export_if_kernel(hkv_table_view v, Pred pred, uint64_t pattern,
     uint64_t key[kExportPerThread], score[kExportPerThread];
 #pragma unroll
     for (int r = 0; r < kExportPerThread; r++) {
-      const uint64_t i = cbase + (uint64_t)r * kExportThreads + tid;
+      const uint64_t i = cbase + (uint64_t)r * THREADS + tid;
       key[r] = v.empty_key;
       score[r] = 0;
       if (i < n) {
@@ -192,14 +191,14 @@ export_if_kernel(hkv_table_view v, Pred pred, uint64_t pattern,
     for (int r = 0; r < kExportPerThread; r++)
       if (!is_reserved_key(v, key[r]) && pred(key[r], score[r], pattern, threshold)) mask |= 1u << r;
     uint32_t total;
-    uint32_t at = block_offsets<kExportThreads>((uint32_t)__popc(mask), s_wave, total);
+    uint32_t at = block_offsets<THREADS>((uint32_t)__popc(mask), s_wave, total);
     if (total == 0) continue; /* the same for the whole workgroup */
     if (tid == 0) s_base = atomicAdd(counter, (unsigned long long)total);
     {
       uint32_t a = at;
 #pragma unroll
       for (int r = 0; r < kExportPerThread; r++)
-        if (mask & (1u << r)) s_src[a++] = (uint16_t)(r * kExportThreads + tid);
+        if (mask & (1u << r)) s_src[a++] = (uint16_t)(r * THREADS + tid);
     }
     __syncthreads();
     const unsigned long long base = s_base;
@@ -211,7 +210,7 @@ export_if_kernel(hkv_table_view v, Pred pred, uint64_t pattern,
         at++;
       }
     }
-    if (out_values) export_rows_any<kExportThreads>(v, offset + cbase, s_src, total, base, out_values);
+    if (out_values) export_rows_any<THREADS>(v, offset + cbase, s_src, total, base, out_values);
     __syncthreads(); /* s_src and s_base are reused by the next chunk */
   }
 }
@@ -432,6 +431,33 @@ erase_if_v2_kernel(hkv_table_view v, uint64_t n, Pred pred, unsigned long long* 
 inline unsigned export_grid(uint64_t n, int threads) {
   const uint64_t chunks = (n + (uint64_t)threads * kExportPerThread - 1) / ((uint64_t)threads * kExportPerThread);
   return (unsigned)(chunks < 4096 ? (chunks ? chunks : 1) : 4096);
+}
+/* Every workgroup that has a match claims its part of the output, and the claims are served one at a time: 2048 of them
+ * (2^22 slots) queue for 30 us where reading the slots takes 13.  512 threads claim for 4096 slots at once; 1024 leave
+ * no more than one workgroup on a CU, whose steps nothing else covers.  Below 2^20 slots they would not reach every CU.
+ * us per call with 256 / 512 / 1024 threads, share of the slots that match:
+ *                          none                 2 %                  18 %                   75 %
+ *   2^18 slots, 256 B      11.3 / 11.6 / 11.5   10.8 / 11.3 / 11.8   12.3 /  13.2 /  17.8   39.5 /  45.9 /  73.0
+ *   2^20 slots, 256 B      10.9 / 11.1 / 11.4   12.7 / 11.3 / 11.4   24.1 /  22.0 /  26.8   93.3 /  93.5 / 105.6
+ *   2^22 slots,  64 B      13.2 / 13.3 / 14.7   33.6 / 22.4 / 20.8   40.0 /  33.2 /  35.7    101 /    98 /   110
+ *   2^24 slots,  64 B      39.4 / 39.5 / 46.1    113 /   67 /   62    128 /   108 /   121    406 /   401 /   428 */
+constexpr uint64_t kExportWide = UINT64_C(1) << 20;
+template <class Pred, int THREADS>
+inline void launch_export_by(const hkv_table_view& v, Pred pred, uint64_t pattern, uint64_t threshold, uint64_t offset,
+                             uint64_t n, unsigned long long* counter, uint64_t* keys, uint8_t* values, uint64_t* scores,
+                             hipStream_t s) {
+  hipLaunchKernelGGL((export_if_kernel<Pred, THREADS>), dim3(export_grid(n, THREADS)), dim3(THREADS), 0, s, v, pred,
+                     pattern, threshold, offset, n, counter, keys, values, scores);
+}
+template <class Pred>
+inline void launch_export(const hkv_table_view& v, Pred pred, uint64_t pattern, uint64_t threshold, uint64_t offset,
+                          uint64_t n, unsigned long long* counter, uint64_t* keys, uint8_t* values, uint64_t* scores,
+                          hipStream_t s) {
+  /* (the units of a chunk's rows are counted in 32 bits: 4096 rows of up to 2^18 bytes) */
+  if (n >= kExportWide && v.value_bytes <= (1u << 18))
+    launch_export_by<Pred, 512>(v, pred, pattern, threshold, offset, n, counter, keys, values, scores, s);
+  else
+    launch_export_by<Pred, 256>(v, pred, pattern, threshold, offset, n, counter, keys, values, scores, s);
 }
 inline unsigned scan_grid(uint64_t slots, int threads) {
   const uint64_t blocks = (slots + threads - 1) / threads;

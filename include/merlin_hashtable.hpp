@@ -893,13 +893,10 @@ class HashTable : public HashTableBase<K, V, S> {
     n = std::min<size_type>(v.capacity - offset, n);
     if (n == 0) return;
     detail::ScoresOut<S> so(scores, n, stream);
-    const unsigned blocks = hkv::export_grid(n, hkv::kExportThreads);
-    hipLaunchKernelGGL((hkv::export_if_kernel<detail::PredAdapter<K, S, PredFunctor>>),
-                       dim3(blocks), dim3(256), 0, stream, v,
-                       detail::PredAdapter<K, S, PredFunctor>(), static_cast<uint64_t>(pattern),
+    hkv::launch_export(v, detail::PredAdapter<K, S, PredFunctor>(), static_cast<uint64_t>(pattern),
                        static_cast<uint64_t>(threshold), static_cast<uint64_t>(offset),
                        static_cast<uint64_t>(n), reinterpret_cast<unsigned long long*>(d_counter),
-                       u64(keys), reinterpret_cast<uint8_t*>(values), so.get());
+                       u64(keys), reinterpret_cast<uint8_t*>(values), so.get(), stream);
     HKV_HIP_CHECK(hipGetLastError());
     so.finish();
   }

@@ -21,7 +21,7 @@
  * of its kind: a launch of its own takes 4 us however little it does.  What is left is bound by one 8-byte atomic on a random
  * line per distinct key of a workgroup and by the queue at the most frequent keys.
  * 2^18 keys of 32 floats, Zipf(1.05) over 2^21 ids, the whole find_or_insert + insert_or_assign: 129 us with a clear
- * before and a pass over the keys behind every call's index (3.5 and 4.5 us), 116 as it is here.
+ * before and a pass over the keys behind every call's index (3.5 and 4.5 us), 116 without, 114 as it is here.
  */
 #ifndef HKV_DEDUP_HPP_
 #define HKV_DEDUP_HPP_
@@ -145,25 +145,31 @@ inline void dedup_fix_rows(const uint32_t* rep, uint64_t n, uint8_t* rows, uint3
     dedup_fix_rows_by<uint8_t>(rep, n, rows, row_bytes, s);
 }
 
-/* The index of a batch: memory for `keys` keys and the number of the last call that used it. */
+/* The index of a batch: memory for `keys` keys, `sparse` entries per key at least, and the number of the last call that
+ * used it.  Four entries per key instead of two shorten the longest search of a workgroup, which all its keys wait for:
+ * find_or_insert + insert_or_assign of Zipf-distributed ids, 70 000 of 128 bytes 60.9 -> 59.4 us, 2^17 of 64 bytes
+ * 73.4 -> 71.0, 2^18 of 128 bytes 111.7 -> 109.9, 500 000 the same.  An index that goes with the call is cleared by
+ * it and takes two. */
 struct RepeatIndex {
   uint8_t* block = nullptr;
   uint64_t keys = 0;
+  uint32_t sparse = 2;
   uint32_t call = 0;
 };
-inline uint64_t repeat_entries(uint64_t keys) {
+inline uint64_t repeat_entries(uint64_t keys, uint32_t sparse) {
   uint64_t entries = 64;
-  while (entries < 2 * keys) entries *= 2;
+  while (entries < sparse * keys) entries *= 2;
   return entries;
 }
-inline hipError_t repeat_index_make(RepeatIndex& x, uint64_t keys, hipStream_t s) {
-  const uint64_t entries = repeat_entries(keys);
+inline hipError_t repeat_index_make(RepeatIndex& x, uint64_t keys, uint32_t sparse, hipStream_t s) {
+  const uint64_t entries = repeat_entries(keys, sparse);
   const hipError_t e = hipMallocAsync((void**)&x.block, entries * 8 + keys * 4, s);
   if (e != hipSuccess) {
     x.block = nullptr;
     return e;
   }
   x.keys = keys;
+  x.sparse = sparse;
   x.call = kNoCall; /* to be cleared */
   return hipSuccess;
 }
@@ -175,7 +181,7 @@ inline void repeat_index_free(RepeatIndex& x, hipStream_t s) {
 /* Enters the n keys of a batch (n < 2^31, at most x.keys) on stream s; the upsert gets `index` and `rep`. */
 inline void repeat_index_enter(RepeatIndex& x, uint64_t n, const uint64_t* keys, hipStream_t s, const uint64_t*& index_out,
                                uint32_t*& rep) {
-  const uint64_t all = repeat_entries(x.keys), entries = repeat_entries(n);
+  const uint64_t all = repeat_entries(x.keys, x.sparse), entries = repeat_entries(n, x.sparse);
   uint64_t* const index = (uint64_t*)x.block;
   rep = (uint32_t*)(x.block + all * 8);
   index_out = index;

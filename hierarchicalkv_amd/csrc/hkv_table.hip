@@ -848,7 +848,7 @@ bool prepare_bounds(hkv_table* t, UpsertArgs& a, hipStream_t s) {
 }
 
 /* unique_key == false: the keys of the batch are entered into an index (hkv_dedup.hpp), the table's own where the call has the
- * table to itself and the batch is not too long to keep the memory for (40 MB), else one that goes with the call: `own`
+ * table to itself and the batch is not too long to keep the memory for (72 MB), else one that goes with the call: `own`
  * frees it, on the stream.  A call that is being recorded into a graph runs again with the same number, so it takes one
  * that it clears. */
 constexpr uint64_t kMostKeptKeys = UINT64_C(1) << 21;
@@ -872,11 +872,11 @@ int enter_repeats(hkv_table* t, UpsertArgs& a, hipStream_t s, bool alone, CallRe
       repeat_index_free(*x, s);
       uint64_t keys = UINT64_C(1) << 12;
       while (keys < a.n) keys *= 2;
-      e = repeat_index_make(*x, keys, s);
+      e = repeat_index_make(*x, keys, 4, s);
     }
   } else {
     call.stream = s;
-    e = repeat_index_make(*x, a.n, s);
+    e = repeat_index_make(*x, a.n, 2, s);
   }
   if (e != hipSuccess) return fail(HKV_ERROR_HIP, "duplicate-key pass: %s", hipGetErrorString(e));
   repeat_index_enter(*x, a.n, a.keys, s, a.repeat_index, a.repeat_of);

@@ -68,7 +68,8 @@ void launch_upsert_for(bool pair, int vec, const View& v, const UpsertArgs& a, h
  * a time, so that a batch of a few ten thousand keys is a long chain on part of the chip; with fewer
  * keys per tile the chain is shorter, and every step is issued for fewer keys at once, which is what
  * costs once the chip is full anyway.  (Registers hardly come into it: insert_or_assign with bounds is
- * compiled to 124 with eight, 97 with two, 95 with one, i.e. 4, 4 and 5 wavefronts per SIMD.)  us per call,
+ * compiled to 124 with eight, 96 with two, 95 with one, i.e. 4, 5 and 5 wavefronts per SIMD; the table was
+ * measured while two still had 97 and four, see upsert_waves.)  us per call,
  * eight / two / one, LRU, rows of 64 bytes; the order is the same for 256:
  *            capacity 2^24, full, half of the keys found          ... 95 % found           a third full, all found
  *            insert_or_assign    insert_and_evict      insert_or_assign   insert_and_evict   insert_or_assign

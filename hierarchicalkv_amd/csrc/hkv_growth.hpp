@@ -1,0 +1,56 @@
+/*
+ * What the host knows about the load of a table that can grow: the last load sample and the keys that have been handed
+ * to upserts since.  No HIP here.
+ */
+#ifndef HKV_GROWTH_HPP_
+#define HKV_GROWTH_HPP_
+
+#include <algorithm>
+#include <atomic>
+#include <cstdint>
+#include <mutex>
+
+namespace hkv {
+
+class LoadKnown {
+ public:
+  /* a call of n keys begins: counted before anything else of it is done */
+  void issue(uint64_t n) { issued_ += n; }
+  /* its kernels are about to be launched; the caller has the table to itself (inserter role of the group lock) */
+  void enqueue(uint64_t n) { enqueued_ += n; }
+  uint64_t enqueued() const { return enqueued_; }
+
+  /* a sample that ran behind the first `at` enqueued keys read `sum` */
+  void sampled(uint64_t sum, uint64_t at) {
+    std::lock_guard<std::mutex> g(mu_);
+    sum_ = sum;
+    at_ = at;
+  }
+  void forget() { sampled(kUnknown, 0); }
+  /* upserts have been recorded into a graph: nobody counts what its replays bring */
+  void recorded() { untracked_ = true; }
+
+  /* The most that a sample of `slots` slots could read now, for a call of n keys that has been issued and not been
+   * enqueued: every key enqueued behind the sample may have come into its slots, and the keys of calls that other
+   * threads are about to enqueue may have as well.  Each enqueued key was issued before and this call's are not
+   * enqueued, so what is issued without them is never below what the sample has seen, whichever thread took it. */
+  bool most(uint64_t n, uint64_t slots, uint64_t& sum) {
+    if (untracked_) return false;
+    std::lock_guard<std::mutex> g(mu_);
+    if (sum_ > slots) return false;
+    sum = std::min(slots, sum_ + (issued_ - n - at_));
+    return true;
+  }
+
+ private:
+  static constexpr uint64_t kUnknown = ~UINT64_C(0);
+  std::atomic<uint64_t> issued_{0};   /* keys handed to upserts since creation */
+  std::atomic<uint64_t> enqueued_{0}; /* the same, of calls that came to their launches */
+  std::mutex mu_;
+  uint64_t sum_ = kUnknown;
+  uint64_t at_ = 0;
+  std::atomic<bool> untracked_{false};
+};
+
+}  // namespace hkv
+#endif

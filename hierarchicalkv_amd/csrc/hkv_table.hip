@@ -30,6 +30,7 @@
 #include "hkv_misc.hpp"
 #include "hkv_dedup.hpp"
 #include "hkv_dual.hpp"
+#include "hkv_growth.hpp"
 #include "hkv_grouped.hpp"
 #include "hkv_keylocks.hpp"
 
@@ -194,13 +195,7 @@ struct hkv_table {
   Clock clock;
   mutable StreamGroupLock lock;
   bool reach_max_capacity; /* merlin_hashtable.cuh:1064: no further growth */
-  /* What the last load sample saw and how many keys can have come since (grow_for) */
-  std::atomic<uint64_t> keys_issued{0}; /* keys handed to upserts since creation, counted before anything else is done */
-  uint64_t keys_enqueued = 0;           /* the same, counted with the group lock when their kernels are launched */
-  std::mutex sample_mu;
-  uint64_t sample_sum = ~UINT64_C(0);   /* keys in the sampled buckets; ~0: not known */
-  uint64_t sample_at = 0;               /* keys_enqueued when that was */
-  std::atomic<bool> untracked{false};   /* upserts have been recorded into a graph, whose replays nobody counts */
+  LoadKnown load;          /* what the last load sample saw and how many keys can have come since (grow_for) */
   bool keys_may_be_locked; /* LOCKED key words may sit in the table (lock_keys, the pointer
                               overload with locked_key_ptrs), until the count below reads 0 */
   bool locked_recount;     /* unlock_keys has run since the count was last read */
@@ -563,10 +558,7 @@ int double_table(hkv_table* t, hipStream_t s) {
   t->view = nv;
   t->pure_hbm = nv.hbm_slots == nv.capacity;
   t->bounds_stale = true; /* the new arenas have none yet */
-  {
-    std::lock_guard<std::mutex> g(t->sample_mu);
-    t->sample_sum = ~UINT64_C(0);
-  }
+  t->load.forget();
   free_arenas(t, old);
   return HKV_SUCCESS;
 }
@@ -618,18 +610,14 @@ int fast_load_factor(hkv_table* t, uint64_t delta, hipStream_t s, float* out) {
   {
     LockGuard g(t, StreamGroupLock::kReader, s);
     HKV_HIP(g.acquire());
-    at = t->keys_enqueued;
+    at = t->load.enqueued();
     hipLaunchKernelGGL(load_sample_kernel, dim3(1), dim3(kSampleThreads), 0, s, t->view, n, h);
     HKV_HIP(hipGetLastError());
   }
   HKV_HIP(hipStreamSynchronize(s));
   const unsigned long long sum = __atomic_load_n(h, __ATOMIC_RELAXED);
-  {
-    /* (with another caller's sample in the word, which may be a later one: its keys are counted from here on as well) */
-    std::lock_guard<std::mutex> g(t->sample_mu);
-    t->sample_sum = sum;
-    t->sample_at = at;
-  }
+  /* (with another caller's sample in the word, which may be a later one: its keys are counted from here on as well) */
+  t->load.sampled(sum, at);
   *out = load_estimate(t, delta, sum);
   return HKV_SUCCESS;
 }
@@ -640,14 +628,12 @@ int fast_load_factor(hkv_table* t, uint64_t delta, hipStream_t s, float* out) {
  * in the sampled buckets, leaves the estimate at or below the limit, a new one would too: the call goes on without.
  * erase, insert_or_assign and find of 30 000 keys, capacity 2^21, half full (every second call can tell): 37.5 -> 31.1 us. */
 int grow_for(hkv_table* t, uint64_t n, hipStream_t s) {
-  const uint64_t before = t->keys_issued.fetch_add(n);
-  if (!t->reach_max_capacity && t->opts.api_lock && !t->untracked && !capturing(s)) {
-    const uint64_t most = (uint64_t)kBucketSize * sampled_buckets(t);
-    std::lock_guard<std::mutex> g(t->sample_mu);
-    if (t->sample_sum <= most) {
-      const uint64_t sum = std::min(most, t->sample_sum + (before - t->sample_at));
-      if (!(load_estimate(t, n, sum) > t->opts.max_load_factor)) return HKV_SUCCESS;
-    }
+  t->load.issue(n);
+  if (!t->reach_max_capacity && t->opts.api_lock && !capturing(s)) {
+    uint64_t sum = 0;
+    if (t->load.most(n, (uint64_t)kBucketSize * sampled_buckets(t), sum) &&
+        !(load_estimate(t, n, sum) > t->opts.max_load_factor))
+      return HKV_SUCCESS;
   }
   while (!t->reach_max_capacity) {
     float lf = 0.f;
@@ -902,8 +888,8 @@ int run_upsert(hkv_table* t, UpsertArgs a, int vec, bool hybrid_rule, hipStream_
     CallRepeats call;
     LockGuard g(t, StreamGroupLock::kInserter, s);
     HKV_HIP(g.acquire());
-    t->keys_enqueued += a.n;
-    if (capturing(s)) t->untracked = true;
+    t->load.enqueue(a.n);
+    if (capturing(s)) t->load.recorded();
     HKV_TRY(settle_locked_count(t, s));
     if (repeats) HKV_TRY(enter_repeats(t, a, s, true, call));
     if (OP == kOpFindOrInsertPtr && a.locked_key_ptrs) t->keys_may_be_locked = true;
@@ -1073,7 +1059,7 @@ int cpu_io_upsert(hkv_table* t, UpsertArgs a, void* values, bool reads, bool rep
   {
     LockGuard g(t, StreamGroupLock::kInserter, s);
     e = g.acquire();
-    t->keys_enqueued += n;
+    t->load.enqueue(n);
     if (e == hipSuccess) e = hipMemsetAsync(d_tmp, 0, n * 9, s); /* reserved, repeated and refused keys: no address */
     if (e == hipSuccess) {
       writes_scores_outside_bounds(t, s, a.strategy == t->opts.evict_strategy);
@@ -1496,9 +1482,9 @@ int hkv_insert_or_assign_noalloc(hkv_table* t, uint64_t n, const uint64_t* keys,
   {
     LockGuard g(t, StreamGroupLock::kInserter, s);
     HKV_HIP(g.acquire());
-    t->keys_issued += n;
-    t->keys_enqueued += n;
-    if (capturing(s)) t->untracked = true;
+    t->load.issue(n);
+    t->load.enqueue(n);
+    if (capturing(s)) t->load.recorded();
     writes_scores_outside_bounds(t, s, a.strategy == t->opts.evict_strategy);
     /* slots left LOCKED by lock_keys are invisible to the second phase; whether any are left
      * after unlock_keys is settled by the next ordinary upsert (it reads a device counter) */

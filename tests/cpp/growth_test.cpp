@@ -1,0 +1,82 @@
+/* The bookkeeping that decides whether an inserting call has to sample the load (hkv_growth.hpp), in the orders that
+ * several host threads can bring it into.  Prints "all checks passed". */
+#include <cstdio>
+#include <cstdlib>
+
+#include "hkv_growth.hpp"
+
+using hkv::LoadKnown;
+
+#define CHECK(x)                                                  \
+  do {                                                            \
+    if (!(x)) {                                                   \
+      std::printf("%s:%d: %s\n", __FILE__, __LINE__, #x);         \
+      std::exit(1);                                               \
+    }                                                             \
+  } while (0)
+
+static const uint64_t kSlots = 4096;
+
+static uint64_t most(LoadKnown& k, uint64_t n) {
+  uint64_t sum = ~UINT64_C(0);
+  CHECK(k.most(n, kSlots, sum));
+  return sum;
+}
+
+static void nothing_known() {
+  LoadKnown k;
+  uint64_t sum = 0;
+  k.issue(5);
+  CHECK(!k.most(5, kSlots, sum));
+  k.sampled(100, 0);
+  CHECK(most(k, 5) == 100);
+  k.forget();
+  CHECK(!k.most(5, kSlots, sum));
+  k.sampled(kSlots + 1, 0); /* of more slots than the table samples now */
+  CHECK(!k.most(5, kSlots, sum));
+  k.sampled(100, 0);
+  k.recorded();
+  CHECK(!k.most(5, kSlots, sum));
+}
+
+static void keys_since_the_sample() {
+  LoadKnown k;
+  for (int call = 0; call < 3; call++) {
+    k.issue(10);
+    k.enqueue(10);
+  }
+  k.sampled(25, k.enqueued());
+  for (uint64_t call = 0; call < 4; call++) {
+    k.issue(7);
+    CHECK(most(k, 7) == 25 + 7 * call);
+    k.enqueue(7);
+  }
+  k.issue(1);
+  k.issue(6000); /* of another thread */
+  CHECK(most(k, 1) == kSlots);
+}
+
+/* a call is issued; before it asks, another thread issues and enqueues its own and takes a sample that has them */
+static void sample_behind_a_later_call() {
+  for (uint64_t seen : {0, 3, 50, 1000}) {
+    LoadKnown k;
+    k.issue(100);
+    k.enqueue(100);
+    k.issue(10);   /* this call */
+    k.issue(50);   /* the other one */
+    k.enqueue(50);
+    k.sampled(seen, k.enqueued());
+    CHECK(most(k, 10) == seen);
+    k.issue(20); /* a third one, not enqueued: it may come in between */
+    CHECK(most(k, 10) == seen + 20);
+    k.enqueue(20);
+    CHECK(most(k, 10) == seen + 20);
+  }
+}
+
+int main() {
+  nothing_known();
+  keys_since_the_sample();
+  sample_behind_a_later_call();
+  std::puts("all checks passed");
+}

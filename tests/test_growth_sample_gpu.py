@@ -1,6 +1,8 @@
 """When a table grows.  An inserting call takes a sample of the load unless the last one, with all keys that have come
 since, rules growth out; a table without the group lock takes one at every call.  Both must have the
 same capacity after every call."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -98,4 +100,47 @@ def test_replays_of_a_recorded_call_are_not_counted():
         t.insert_or_assign(8, dev(w.unique_keys(63, 8, 8)), rows)
         assert t.capacity() == 2 * cap
     torch.cuda.synchronize()
+    t.close()
+
+
+def test_host_threads_insert_into_one_table_that_grows():
+    """Eight threads, each on a stream and with keys of its own: whatever sample a call goes by, the table has grown
+    whenever it had to, so that no bucket ever was full and every key is there with its row."""
+    threads, rounds, n, dim = 8, 80, 50, 4
+    t = HashTable()
+    t.init(default_options(init_capacity=1 << 13, max_capacity=1 << 18, max_hbm_for_vectors=1 << 30, dim=dim,
+                           max_load_factor=0.5))
+    errors = []
+
+    def worker(tid):
+        try:
+            torch.cuda.set_device(0)
+            s = torch.cuda.Stream()
+            for r in range(rounds):
+                keys = w.unique_keys(6400 + tid, r * n, n)
+                dk, dv = dev(keys), dev(w.values_from_keys(keys, dim))
+                torch.cuda.current_stream().synchronize()
+                if r % 3 == 2:
+                    t.find_or_insert(n, dk, dv, stream=s)
+                else:
+                    t.insert_or_assign(n, dk, dv, stream=s, unique_key=r % 3 == 0)
+                s.synchronize()  # the buffers go away
+        except BaseException as e:  # noqa: BLE001 - reported by the main thread
+            errors.append((tid, repr(e)))
+
+    running = [threading.Thread(target=worker, args=(i,)) for i in range(threads)]
+    for th in running:
+        th.start()
+    for th in running:
+        th.join()
+    assert not errors, errors[:3]
+    torch.cuda.synchronize()
+    assert t.size() == threads * rounds * n and t.capacity() >= 2 * (threads * rounds - threads) * n
+    for tid in range(threads):
+        keys = w.unique_keys(6400 + tid, 0, rounds * n)
+        out = torch.zeros(rounds * n, dim, dtype=torch.float32, device=DEV)
+        founds = torch.zeros(rounds * n, dtype=torch.bool, device=DEV)
+        t.find(rounds * n, dev(keys), out, founds)
+        torch.cuda.synchronize()
+        assert bool(founds.all()) and np.array_equal(out.cpu().numpy(), w.values_from_keys(keys, dim))
     t.close()

@@ -592,12 +592,11 @@ bool capturing(hipStream_t s) {
 
 /* fast_load_factor, merlin_hashtable.cuh:3796-3830: the first min(buckets,
  * 1024) buckets stand for the table; the incoming batch counts as all new */
-uint32_t sampled_buckets(const hkv_table* t) { return (uint32_t)std::min<uint64_t>(t->view.buckets_num, 1024); }
-float load_estimate(const hkv_table* t, uint64_t delta, uint64_t sum) {
-  return (float)((delta * 1.0) / (t->view.capacity * 1.0) + (sum * 1.0) / (kBucketSize * sampled_buckets(t) * 1.0));
+uint64_t sampled_slots(uint64_t capacity) { return std::min<uint64_t>(capacity, 1024 * kBucketSize); }
+float load_estimate(uint64_t capacity, uint64_t delta, uint64_t sum) {
+  return (float)((delta * 1.0) / (capacity * 1.0) + (sum * 1.0) / (sampled_slots(capacity) * 1.0));
 }
 int fast_load_factor(hkv_table* t, uint64_t delta, hipStream_t s, float* out) {
-  const uint32_t n = sampled_buckets(t);
   /* A word of its own, not one of the leased counters: callers that hold a lease come through
    * here (the count-returning insert_and_evict), and with all leases out they would wait for
    * each other.  The kernel stores its whole result in one write, so callers that overlap read
@@ -606,19 +605,21 @@ int fast_load_factor(hkv_table* t, uint64_t delta, hipStream_t s, float* out) {
    * stream is waited for and nothing is copied: erase, insert_or_assign and find of 30 000 keys on a
    * table that can grow, 57 -> 42 us. */
   unsigned long long* h = t->h_words + kCounterWords;
-  uint64_t at = 0;
+  uint64_t at = 0, capacity = 0;
   {
     LockGuard g(t, StreamGroupLock::kReader, s);
     HKV_HIP(g.acquire());
     at = t->load.enqueued();
-    hipLaunchKernelGGL(load_sample_kernel, dim3(1), dim3(kSampleThreads), 0, s, t->view, n, h);
+    capacity = t->view.capacity; /* (of the table that is sampled: without the lock another thread may double it) */
+    hipLaunchKernelGGL(load_sample_kernel, dim3(1), dim3(kSampleThreads), 0, s, t->view,
+                       (uint32_t)(sampled_slots(capacity) / kBucketSize), h);
     HKV_HIP(hipGetLastError());
   }
   HKV_HIP(hipStreamSynchronize(s));
   const unsigned long long sum = __atomic_load_n(h, __ATOMIC_RELAXED);
   /* (with another caller's sample in the word, which may be a later one: its keys are counted from here on as well) */
-  t->load.sampled(sum, at);
-  *out = load_estimate(t, delta, sum);
+  t->load.sampled(sum, sampled_slots(capacity), at);
+  *out = load_estimate(capacity, delta, sum);
   return HKV_SUCCESS;
 }
 
@@ -631,8 +632,8 @@ int grow_for(hkv_table* t, uint64_t n, hipStream_t s) {
   t->load.issue(n);
   if (!t->reach_max_capacity && t->opts.api_lock && !capturing(s)) {
     uint64_t sum = 0;
-    if (t->load.most(n, (uint64_t)kBucketSize * sampled_buckets(t), sum) &&
-        !(load_estimate(t, n, sum) > t->opts.max_load_factor))
+    const uint64_t capacity = t->view.capacity;
+    if (t->load.most(n, sampled_slots(capacity), sum) && !(load_estimate(capacity, n, sum) > t->opts.max_load_factor))
       return HKV_SUCCESS;
   }
   while (!t->reach_max_capacity) {

@@ -28,13 +28,11 @@ static void nothing_known() {
   uint64_t sum = 0;
   k.issue(5);
   CHECK(!k.most(5, kSlots, sum));
-  k.sampled(100, 0);
+  k.sampled(100, kSlots, 0);
   CHECK(most(k, 5) == 100);
   k.forget();
   CHECK(!k.most(5, kSlots, sum));
-  k.sampled(kSlots + 1, 0); /* of more slots than the table samples now */
-  CHECK(!k.most(5, kSlots, sum));
-  k.sampled(100, 0);
+  k.sampled(100, kSlots, 0);
   k.recorded();
   CHECK(!k.most(5, kSlots, sum));
 }
@@ -45,7 +43,7 @@ static void keys_since_the_sample() {
     k.issue(10);
     k.enqueue(10);
   }
-  k.sampled(25, k.enqueued());
+  k.sampled(25, kSlots, k.enqueued());
   for (uint64_t call = 0; call < 4; call++) {
     k.issue(7);
     CHECK(most(k, 7) == 25 + 7 * call);
@@ -65,7 +63,7 @@ static void sample_behind_a_later_call() {
     k.issue(10);   /* this call */
     k.issue(50);   /* the other one */
     k.enqueue(50);
-    k.sampled(seen, k.enqueued());
+    k.sampled(seen, kSlots, k.enqueued());
     CHECK(most(k, 10) == seen);
     k.issue(20); /* a third one, not enqueued: it may come in between */
     CHECK(most(k, 10) == seen + 20);
@@ -74,9 +72,25 @@ static void sample_behind_a_later_call() {
   }
 }
 
+/* a sample of another number of slots than the next one would read, which a thread that doubles the table can bring
+ * in at any time: half of the slots hold half of the keys */
+static void sample_of_other_slots() {
+  LoadKnown k;
+  uint64_t sum = 0;
+  k.issue(2000);
+  k.enqueue(2000);
+  k.sampled(1000, kSlots / 2, k.enqueued());
+  k.issue(5);
+  CHECK(!k.most(5, kSlots, sum));
+  CHECK(k.most(5, kSlots / 2, sum) && sum == 1000);
+  k.sampled(2000, kSlots * 2, k.enqueued());
+  CHECK(!k.most(5, kSlots, sum));
+}
+
 int main() {
   nothing_known();
   keys_since_the_sample();
   sample_behind_a_later_call();
+  sample_of_other_slots();
   std::puts("all checks passed");
 }

@@ -14,10 +14,27 @@ namespace hkv {
 
 class LoadKnown {
  public:
-  /* a call of n keys begins: counted before anything else of it is done */
-  void issue(uint64_t n) { issued_ += n; }
-  /* its kernels are about to be launched; the caller has the table to itself (inserter role of the group lock) */
-  void enqueue(uint64_t n) { enqueued_ += n; }
+  /* The keys of one call: issued when it begins, before anything else of it is done, enqueued when its kernels are
+   * about to be launched and the call has the table to itself (inserter role of the group lock).  A call that returns
+   * before that, with an error, brings none: they are taken back. */
+  class Call {
+   public:
+    Call(LoadKnown& k, uint64_t n) : k_(k), n_(n), open_(true) { k_.issued_ += n_; }
+    Call(const Call&) = delete;
+    Call& operator=(const Call&) = delete;
+    ~Call() {
+      if (open_) k_.issued_ -= n_;
+    }
+    void enqueue() {
+      k_.enqueued_ += n_;
+      open_ = false;
+    }
+
+   private:
+    LoadKnown& k_;
+    const uint64_t n_;
+    bool open_;
+  };
   uint64_t enqueued() const { return enqueued_; }
 
   /* a sample of `slots` slots that ran behind the first `at` enqueued keys read `sum` */

@@ -627,9 +627,9 @@ int fast_load_factor(hkv_table* t, uint64_t delta, hipStream_t s, float* out) {
  * (merlin_hashtable.cuh:1151-1154, 1369-1372, 1604-1607, 1712-1715, 1898-1901).
  * The sample has to be waited for.  Where the last one, with every key that has been handed to an upsert since
  * in the sampled buckets, leaves the estimate at or below the limit, a new one would too: the call goes on without.
- * erase, insert_or_assign and find of 30 000 keys, capacity 2^21, half full (every second call can tell): 37.5 -> 31.1 us. */
+ * erase, insert_or_assign and find of 30 000 keys, capacity 2^21, half full (every second call can tell): 37.5 -> 31.1 us.
+ * (The caller has issued its keys, LoadKnown::Call.) */
 int grow_for(hkv_table* t, uint64_t n, hipStream_t s) {
-  t->load.issue(n);
   if (!t->reach_max_capacity && t->opts.api_lock && !capturing(s)) {
     uint64_t sum = 0;
     const uint64_t capacity = t->view.capacity;
@@ -877,6 +877,7 @@ int enter_repeats(hkv_table* t, UpsertArgs& a, hipStream_t s, bool alone, CallRe
 template <int OP>
 int run_upsert(hkv_table* t, UpsertArgs a, int vec, bool hybrid_rule, hipStream_t s, bool repeats = false) {
   HKV_TRY(check_repeats(a.n, repeats));
+  LoadKnown::Call keys(t->load, a.n);
   HKV_TRY(grow_for(t, a.n, s));
   a.epoch = t->epoch;
   a.clock = t->clock;
@@ -889,7 +890,7 @@ int run_upsert(hkv_table* t, UpsertArgs a, int vec, bool hybrid_rule, hipStream_
     CallRepeats call;
     LockGuard g(t, StreamGroupLock::kInserter, s);
     HKV_HIP(g.acquire());
-    t->load.enqueue(a.n);
+    keys.enqueue();
     if (capturing(s)) t->load.recorded();
     HKV_TRY(settle_locked_count(t, s));
     if (repeats) HKV_TRY(enter_repeats(t, a, s, true, call));
@@ -1035,6 +1036,7 @@ __global__ void cpu_io_owner_kernel(View v, const uint64_t* keys, uint8_t** ptrs
 /* insert_or_assign (reads == false) and find_or_insert (reads == true) */
 int cpu_io_upsert(hkv_table* t, UpsertArgs a, void* values, bool reads, bool repeats, hipStream_t s) {
   HKV_TRY(check_repeats(a.n, repeats));
+  LoadKnown::Call keys(t->load, a.n);
   HKV_TRY(grow_for(t, a.n, s));
   const uint64_t n = a.n, vb = t->view.value_bytes;
   std::lock_guard<std::mutex> host_lock(t->io_mutex);
@@ -1060,7 +1062,7 @@ int cpu_io_upsert(hkv_table* t, UpsertArgs a, void* values, bool reads, bool rep
   {
     LockGuard g(t, StreamGroupLock::kInserter, s);
     e = g.acquire();
-    t->load.enqueue(n);
+    if (e == hipSuccess) keys.enqueue();
     if (e == hipSuccess) e = hipMemsetAsync(d_tmp, 0, n * 9, s); /* reserved, repeated and refused keys: no address */
     if (e == hipSuccess) {
       writes_scores_outside_bounds(t, s, a.strategy == t->opts.evict_strategy);
@@ -1483,8 +1485,7 @@ int hkv_insert_or_assign_noalloc(hkv_table* t, uint64_t n, const uint64_t* keys,
   {
     LockGuard g(t, StreamGroupLock::kInserter, s);
     HKV_HIP(g.acquire());
-    t->load.issue(n);
-    t->load.enqueue(n);
+    LoadKnown::Call(t->load, n).enqueue();
     if (capturing(s)) t->load.recorded();
     writes_scores_outside_bounds(t, s, a.strategy == t->opts.evict_strategy);
     /* slots left LOCKED by lock_keys are invisible to the second phase; whether any are left

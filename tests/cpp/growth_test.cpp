@@ -23,10 +23,12 @@ static uint64_t most(LoadKnown& k, uint64_t n) {
   return sum;
 }
 
+static void brings(LoadKnown& k, uint64_t n) { LoadKnown::Call(k, n).enqueue(); }
+
 static void nothing_known() {
   LoadKnown k;
   uint64_t sum = 0;
-  k.issue(5);
+  LoadKnown::Call mine(k, 5);
   CHECK(!k.most(5, kSlots, sum));
   k.sampled(100, kSlots, 0);
   CHECK(most(k, 5) == 100);
@@ -39,18 +41,15 @@ static void nothing_known() {
 
 static void keys_since_the_sample() {
   LoadKnown k;
-  for (int call = 0; call < 3; call++) {
-    k.issue(10);
-    k.enqueue(10);
-  }
+  for (int call = 0; call < 3; call++) brings(k, 10);
+  CHECK(k.enqueued() == 30);
   k.sampled(25, kSlots, k.enqueued());
   for (uint64_t call = 0; call < 4; call++) {
-    k.issue(7);
+    LoadKnown::Call mine(k, 7);
     CHECK(most(k, 7) == 25 + 7 * call);
-    k.enqueue(7);
+    mine.enqueue();
   }
-  k.issue(1);
-  k.issue(6000); /* of another thread */
+  LoadKnown::Call mine(k, 1), others(k, 6000);
   CHECK(most(k, 1) == kSlots);
 }
 
@@ -58,18 +57,28 @@ static void keys_since_the_sample() {
 static void sample_behind_a_later_call() {
   for (uint64_t seen : {0, 3, 50, 1000}) {
     LoadKnown k;
-    k.issue(100);
-    k.enqueue(100);
-    k.issue(10);   /* this call */
-    k.issue(50);   /* the other one */
-    k.enqueue(50);
+    brings(k, 100);
+    LoadKnown::Call mine(k, 10);
+    brings(k, 50);
     k.sampled(seen, kSlots, k.enqueued());
     CHECK(most(k, 10) == seen);
-    k.issue(20); /* a third one, not enqueued: it may come in between */
+    LoadKnown::Call third(k, 20); /* not enqueued: it may come in between */
     CHECK(most(k, 10) == seen + 20);
-    k.enqueue(20);
+    third.enqueue();
     CHECK(most(k, 10) == seen + 20);
   }
+}
+
+/* a large call that fails before its launches leaves nothing behind, neither for this sample nor for the next */
+static void calls_that_fail() {
+  LoadKnown k;
+  brings(k, 100);
+  k.sampled(100, kSlots, k.enqueued());
+  for (int call = 0; call < 5; call++) LoadKnown::Call failed(k, 4000);
+  LoadKnown::Call mine(k, 10);
+  CHECK(most(k, 10) == 100);
+  k.sampled(100, kSlots, k.enqueued());
+  CHECK(most(k, 10) == 100);
 }
 
 /* a sample of another number of slots than the next one would read, which a thread that doubles the table can bring
@@ -77,10 +86,9 @@ static void sample_behind_a_later_call() {
 static void sample_of_other_slots() {
   LoadKnown k;
   uint64_t sum = 0;
-  k.issue(2000);
-  k.enqueue(2000);
+  brings(k, 2000);
   k.sampled(1000, kSlots / 2, k.enqueued());
-  k.issue(5);
+  LoadKnown::Call mine(k, 5);
   CHECK(!k.most(5, kSlots, sum));
   CHECK(k.most(5, kSlots / 2, sum) && sum == 1000);
   k.sampled(2000, kSlots * 2, k.enqueued());
@@ -91,6 +99,7 @@ int main() {
   nothing_known();
   keys_since_the_sample();
   sample_behind_a_later_call();
+  calls_that_fail();
   sample_of_other_slots();
   std::puts("all checks passed");
 }

@@ -178,8 +178,9 @@ inline void repeat_index_free(RepeatIndex& x, hipStream_t s) {
   x = RepeatIndex{};
 }
 
-/* Enters the n keys of a batch (n < 2^31, at most x.keys) on stream s; the upsert gets `index` and `rep`. */
-inline void repeat_index_enter(RepeatIndex& x, uint64_t n, const uint64_t* keys, hipStream_t s, const uint64_t*& index_out,
+/* Enters the n keys of a batch (n < 2^31, at most x.keys) on stream s; the upsert gets `index` and `rep`.  Where a launch
+ * fails nobody knows what is in the index: the next call that uses it clears it. */
+inline hipError_t repeat_index_enter(RepeatIndex& x, uint64_t n, const uint64_t* keys, hipStream_t s, const uint64_t*& index_out,
                                uint32_t*& rep) {
   const uint64_t all = repeat_entries(x.keys, x.sparse), entries = repeat_entries(n, x.sparse);
   uint64_t* const index = (uint64_t*)x.block;
@@ -198,6 +199,9 @@ inline void repeat_index_enter(RepeatIndex& x, uint64_t n, const uint64_t* keys,
   else
     hipLaunchKernelGGL(dedup_enter_kernel<256>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, keys, n, index,
                        entries - 1, x.call, rep);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) x.call = kNoCall;
+  return e;
 }
 
 }  // namespace hkv

@@ -865,9 +865,8 @@ int enter_repeats(hkv_table* t, UpsertArgs& a, hipStream_t s, bool alone, CallRe
     call.stream = s;
     e = repeat_index_make(*x, a.n, 2, s);
   }
+  if (e == hipSuccess) e = repeat_index_enter(*x, a.n, a.keys, s, a.repeat_index, a.repeat_of);
   if (e != hipSuccess) return fail(HKV_ERROR_HIP, "duplicate-key pass: %s", hipGetErrorString(e));
-  repeat_index_enter(*x, a.n, a.keys, s, a.repeat_index, a.repeat_of);
-  HKV_HIP(hipGetLastError());
   return HKV_SUCCESS;
 }
 

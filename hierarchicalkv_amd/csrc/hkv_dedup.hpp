@@ -161,9 +161,15 @@ inline uint64_t repeat_entries(uint64_t keys, uint32_t sparse) {
   while (entries < sparse * keys) entries *= 2;
   return entries;
 }
-inline hipError_t repeat_index_make(RepeatIndex& x, uint64_t keys, uint32_t sparse, hipStream_t s) {
+/* Where an index comes from and goes back to, in the order of the stream */
+struct StreamMemory {
+  static hipError_t take(void** p, size_t bytes, hipStream_t s) { return hipMallocAsync(p, bytes, s); }
+  static void give(void* p, hipStream_t s) { (void)hipFreeAsync(p, s); }
+};
+template <class Memory>
+hipError_t repeat_index_make(RepeatIndex& x, uint64_t keys, uint32_t sparse, Memory memory, hipStream_t s) {
   const uint64_t entries = repeat_entries(keys, sparse);
-  const hipError_t e = hipMallocAsync((void**)&x.block, entries * 8 + keys * 4, s);
+  const hipError_t e = memory.take((void**)&x.block, entries * 8 + keys * 4, s);
   if (e != hipSuccess) {
     x.block = nullptr;
     return e;
@@ -173,8 +179,9 @@ inline hipError_t repeat_index_make(RepeatIndex& x, uint64_t keys, uint32_t spar
   x.call = kNoCall; /* to be cleared */
   return hipSuccess;
 }
-inline void repeat_index_free(RepeatIndex& x, hipStream_t s) {
-  if (x.block) (void)hipFreeAsync(x.block, s);
+template <class Memory>
+void repeat_index_free(RepeatIndex& x, Memory memory, hipStream_t s) {
+  if (x.block) memory.give(x.block, s);
   x = RepeatIndex{};
 }
 

@@ -842,7 +842,24 @@ constexpr uint64_t kMostKeptKeys = UINT64_C(1) << 21;
 struct CallRepeats {
   RepeatIndex own;
   hipStream_t stream = nullptr;
-  ~CallRepeats() { repeat_index_free(own, stream); }
+  ~CallRepeats() { repeat_index_free(own, StreamMemory(), stream); }
+};
+/* The table's own index: from the allocator the table was created with, which takes no part in the order of streams, else from
+ * the stream's pool, which costs no synchronisation of the device. */
+struct KeptMemory {
+  hkv_table* t;
+  hipError_t take(void** p, size_t bytes, hipStream_t s) const {
+    if (t->own_alloc) return hipMallocAsync(p, bytes, s);
+    return table_alloc(t, 0, p, bytes) == HKV_SUCCESS ? hipSuccess : hipErrorOutOfMemory;
+  }
+  void give(void* p, hipStream_t s) const {
+    if (t->own_alloc) {
+      (void)hipFreeAsync(p, s);
+    } else {
+      (void)hipStreamSynchronize(s); /* (the inserter role has ordered the calls of other streams before this one) */
+      table_free(t, 0, p);
+    }
+  }
 };
 int check_repeats(uint64_t n, bool repeats) {
   if (repeats && n >= (UINT64_C(1) << 31))
@@ -856,14 +873,14 @@ int enter_repeats(hkv_table* t, UpsertArgs& a, hipStream_t s, bool alone, CallRe
   if (alone && t->opts.api_lock && a.n <= kMostKeptKeys && !capturing(s)) {
     x = &t->repeats;
     if (x->keys < a.n) {
-      repeat_index_free(*x, s);
+      repeat_index_free(*x, KeptMemory{t}, s);
       uint64_t keys = UINT64_C(1) << 12;
       while (keys < a.n) keys *= 2;
-      e = repeat_index_make(*x, keys, 4, s);
+      e = repeat_index_make(*x, keys, 4, KeptMemory{t}, s);
     }
   } else {
     call.stream = s;
-    e = repeat_index_make(*x, a.n, 2, s);
+    e = repeat_index_make(*x, a.n, 2, StreamMemory(), s);
   }
   if (e == hipSuccess) e = repeat_index_enter(*x, a.n, a.keys, s, a.repeat_index, a.repeat_of);
   if (e != hipSuccess) return fail(HKV_ERROR_HIP, "duplicate-key pass: %s", hipGetErrorString(e));
@@ -1397,7 +1414,7 @@ int hkv_table_destroy(hkv_table* t) {
   if (!t) return HKV_SUCCESS;
   (void)hipSetDevice(t->device);
   (void)hipDeviceSynchronize();
-  if (t->repeats.block) (void)hipFree(t->repeats.block);
+  table_free(t, 0, t->repeats.block);
   table_free(t, 0, t->d_meta);
   table_free(t, 0, t->d_counters);
   table_free(t, 0, t->d_values);

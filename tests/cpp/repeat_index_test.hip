@@ -53,7 +53,7 @@ static int enter(RepeatIndex& x, uint64_t n, hipError_t want) {
 static void failed_launches() {
   for (uint64_t n : {100, 40000}) {
     RepeatIndex x;
-    CHECK(repeat_index_make(x, 40000, 4, nullptr) == hipSuccess);
+    CHECK(repeat_index_make(x, 40000, 4, StreamMemory(), nullptr) == hipSuccess);
     fail_launch = 0; /* the clear */
     enter(x, n, hipErrorLaunchFailure);
     CHECK(enter(x, n, hipSuccess) == 2); /* clears again */
@@ -64,18 +64,18 @@ static void failed_launches() {
     CHECK(enter(x, n, hipErrorLaunchFailure) == 2);
     CHECK(enter(x, n, hipSuccess) == 2);
     CHECK(enter(x, n, hipSuccess) == 1);
-    repeat_index_free(x, nullptr);
+    repeat_index_free(x, StreamMemory(), nullptr);
   }
 }
 
 static void numbers_of_calls() {
   RepeatIndex x;
-  CHECK(repeat_index_make(x, 64, 4, nullptr) == hipSuccess);
+  CHECK(repeat_index_make(x, 64, 4, StreamMemory(), nullptr) == hipSuccess);
   for (int round = 0; round < 2; round++) {
     CHECK(enter(x, 64, hipSuccess) == 2 && x.call == 0);
     for (uint32_t call = 1; call < kNoCall; call++) CHECK(enter(x, 64, hipSuccess) == 1 && x.call == call);
   }
-  repeat_index_free(x, nullptr);
+  repeat_index_free(x, StreamMemory(), nullptr);
 }
 
 int main() {

@@ -185,6 +185,24 @@ void repeat_index_free(RepeatIndex& x, Memory memory, hipStream_t s) {
   x = RepeatIndex{};
 }
 
+/* The index for a batch of n keys: the table's own, `kept`, made large enough, for batches of up to `most_kept` keys;
+ * for others, and where that much memory is not to be had, one that goes with the call and takes less, `own`. */
+template <class Memory>
+hipError_t repeat_index_for(uint64_t n, uint64_t most_kept, RepeatIndex& kept, Memory memory, RepeatIndex& own, hipStream_t s,
+                            RepeatIndex*& x) {
+  x = &kept;
+  if (n <= most_kept) {
+    if (kept.keys >= n) return hipSuccess;
+    repeat_index_free(kept, memory, s);
+    uint64_t keys = UINT64_C(1) << 12;
+    while (keys < n) keys *= 2;
+    if (repeat_index_make(kept, keys, 4, memory, s) == hipSuccess) return hipSuccess;
+    (void)hipGetLastError();
+  }
+  x = &own;
+  return repeat_index_make(own, n, 2, StreamMemory(), s);
+}
+
 /* Enters the n keys of a batch (n < 2^31, at most x.keys) on stream s; the upsert gets `index` and `rep`.  Where a launch
  * fails nobody knows what is in the index: the next call that uses it clears it. */
 inline hipError_t repeat_index_enter(RepeatIndex& x, uint64_t n, const uint64_t* keys, hipStream_t s, const uint64_t*& index_out,

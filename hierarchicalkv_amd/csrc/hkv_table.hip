@@ -868,20 +868,10 @@ int check_repeats(uint64_t n, bool repeats) {
 }
 int enter_repeats(hkv_table* t, UpsertArgs& a, hipStream_t s, bool alone, CallRepeats& call) {
   if (a.n < 2) return HKV_SUCCESS;
-  RepeatIndex* x = &call.own;
-  hipError_t e = hipSuccess;
-  if (alone && t->opts.api_lock && a.n <= kMostKeptKeys && !capturing(s)) {
-    x = &t->repeats;
-    if (x->keys < a.n) {
-      repeat_index_free(*x, KeptMemory{t}, s);
-      uint64_t keys = UINT64_C(1) << 12;
-      while (keys < a.n) keys *= 2;
-      e = repeat_index_make(*x, keys, 4, KeptMemory{t}, s);
-    }
-  } else {
-    call.stream = s;
-    e = repeat_index_make(*x, a.n, 2, StreamMemory(), s);
-  }
+  RepeatIndex* x = nullptr;
+  call.stream = s;
+  const uint64_t most_kept = alone && t->opts.api_lock && !capturing(s) ? kMostKeptKeys : 0;
+  hipError_t e = repeat_index_for(a.n, most_kept, t->repeats, KeptMemory{t}, call.own, s, x);
   if (e == hipSuccess) e = repeat_index_enter(*x, a.n, a.keys, s, a.repeat_index, a.repeat_of);
   if (e != hipSuccess) return fail(HKV_ERROR_HIP, "duplicate-key pass: %s", hipGetErrorString(e));
   return HKV_SUCCESS;

@@ -14,16 +14,21 @@
     }                                                     \
   } while (0)
 
+static size_t largest = ~size_t(0), taken = 0; /* block that is to be had; bytes of the last one */
+static int blocks = 0;
 static int launches = 0, fail_launch = -1; /* of the launches from now on, the one that fails */
 static hipError_t last = hipSuccess;
 
 extern "C" {
 hipError_t hipMallocAsync(void** p, size_t bytes, hipStream_t) {
-  *p = std::malloc(bytes);
+  if (bytes > largest) return last = hipErrorOutOfMemory;
+  *p = std::malloc(taken = bytes);
+  blocks++;
   return hipSuccess;
 }
 hipError_t hipFreeAsync(void* p, hipStream_t) {
   std::free(p);
+  blocks--;
   return hipSuccess;
 }
 hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
@@ -78,8 +83,56 @@ static void numbers_of_calls() {
   repeat_index_free(x, StreamMemory(), nullptr);
 }
 
+static RepeatIndex* index_for(uint64_t n, uint64_t most_kept, RepeatIndex& kept, RepeatIndex& own) {
+  RepeatIndex* x = nullptr;
+  CHECK(repeat_index_for(n, most_kept, kept, StreamMemory(), own, nullptr, x) == hipSuccess);
+  CHECK(x->keys >= n && (x == &kept || x == &own));
+  CHECK(enter(*x, n, hipSuccess) >= 1);
+  return x;
+}
+
+static void kept_or_not() {
+  RepeatIndex kept, own;
+  const uint64_t most = 1 << 16;
+  CHECK(index_for(10, most, kept, own) == &kept && blocks == 1 && kept.keys == 4096);
+  CHECK(index_for(4096, most, kept, own) == &kept && blocks == 1 && kept.keys == 4096);
+  CHECK(index_for(4097, most, kept, own) == &kept && blocks == 1 && kept.keys == 8192);
+  CHECK(index_for(most, most, kept, own) == &kept && blocks == 1 && kept.keys == most);
+  CHECK(index_for(5, most, kept, own) == &kept && kept.keys == most && kept.call == 1);
+  CHECK(index_for(most + 1, most, kept, own) == &own && blocks == 2 && own.sparse == 2);
+  repeat_index_free(own, StreamMemory(), nullptr);
+  CHECK(index_for(5, 0, kept, own) == &own && blocks == 2);
+  repeat_index_free(own, StreamMemory(), nullptr);
+  repeat_index_free(kept, StreamMemory(), nullptr);
+  CHECK(blocks == 0);
+}
+
+/* memory for an index of four entries per key is not to be had, for two it is: the call goes on with that, and with an index that is
+ * kept once there is memory again; with none the call fails and says so */
+static void memory_runs_out() {
+  RepeatIndex kept, own;
+  const uint64_t n = 1 << 15, most = 1 << 16;
+  CHECK(index_for(100, most, kept, own) == &kept);
+  largest = n * 28;
+  CHECK(index_for(n, most, kept, own) == &own && own.sparse == 2 && taken <= largest && !kept.block && blocks == 1);
+  CHECK(last == hipSuccess);
+  repeat_index_free(own, StreamMemory(), nullptr);
+  CHECK(index_for(100, most, kept, own) == &kept);
+  largest = 100;
+  RepeatIndex* x = nullptr;
+  CHECK(repeat_index_for(n, most, kept, StreamMemory(), own, nullptr, x) == hipErrorOutOfMemory && !own.block);
+  last = hipSuccess;
+  largest = ~size_t(0);
+  CHECK(index_for(n, most, kept, own) == &kept);
+  repeat_index_free(own, StreamMemory(), nullptr);
+  repeat_index_free(kept, StreamMemory(), nullptr);
+  CHECK(blocks == 0);
+}
+
 int main() {
   failed_launches();
+  kept_or_not();
+  memory_runs_out();
   numbers_of_calls();
   std::puts("all checks passed");
 }

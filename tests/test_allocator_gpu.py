@@ -91,3 +91,22 @@ def test_index_of_repeated_keys_comes_from_the_allocator():
         assert len(c.out) == blocks + 1
     t.close()
     assert not c.out
+
+
+def test_calls_go_on_where_the_allocator_has_no_room_for_the_index():
+    cap = 1 << 18
+    c = Counting()
+    t = c.table(init_capacity=cap, max_capacity=cap, max_hbm_for_vectors=1 << 30, dim=4)
+    blocks = len(c.out)
+    repeated_calls(t, (3000,))
+    assert len(c.out) == blocks + 1
+    c.refuse_from = 4 * 8 * 50000
+    repeated_calls(t, (50000, 50000))
+    assert len(c.out) == blocks
+    repeated_calls(t, (3000,))
+    assert len(c.out) == blocks + 1
+    c.refuse_from = None
+    repeated_calls(t, (50000, 3000))
+    assert len(c.out) == blocks + 1
+    t.close()
+    assert not c.out

@@ -196,6 +196,7 @@ hipError_t repeat_index_for(uint64_t n, uint64_t most_kept, RepeatIndex& kept, M
     repeat_index_free(kept, memory, s);
     uint64_t keys = UINT64_C(1) << 12;
     while (keys < n) keys *= 2;
+    if (keys > most_kept) keys = most_kept;
     if (repeat_index_make(kept, keys, 4, memory, s) == hipSuccess) return hipSuccess;
     (void)hipGetLastError();
   }

@@ -835,8 +835,9 @@ bool prepare_bounds(hkv_table* t, UpsertArgs& a, hipStream_t s) {
 }
 
 /* unique_key == false: the keys of the batch are entered into an index (hkv_dedup.hpp), the table's own where the call has the
- * table to itself and the batch is not too long to keep the memory for (72 MB), else one that goes with the call: `own`
- * frees it, on the stream.  A call that is being recorded into a graph runs again with the same number, so it takes one
+ * table to itself and the batch is not too long to keep the memory for, else one that goes with the call: `own`
+ * frees it, on the stream.  Too long is more keys than the table has slots, so that the index of a small table stays
+ * small (36 bytes per slot, 68 where their number is no power of two), or 2^21 (72 MB).  A call that is being recorded into a graph runs again with the same number, so it takes one
  * that it clears. */
 constexpr uint64_t kMostKeptKeys = UINT64_C(1) << 21;
 struct CallRepeats {
@@ -870,7 +871,8 @@ int enter_repeats(hkv_table* t, UpsertArgs& a, hipStream_t s, bool alone, CallRe
   if (a.n < 2) return HKV_SUCCESS;
   RepeatIndex* x = nullptr;
   call.stream = s;
-  const uint64_t most_kept = alone && t->opts.api_lock && !capturing(s) ? kMostKeptKeys : 0;
+  const bool keep = alone && t->opts.api_lock && !capturing(s);
+  const uint64_t most_kept = keep ? std::min(kMostKeptKeys, t->view.capacity) : 0;
   hipError_t e = repeat_index_for(a.n, most_kept, t->repeats, KeptMemory{t}, call.own, s, x);
   if (e == hipSuccess) e = repeat_index_enter(*x, a.n, a.keys, s, a.repeat_index, a.repeat_of);
   if (e != hipSuccess) return fail(HKV_ERROR_HIP, "duplicate-key pass: %s", hipGetErrorString(e));

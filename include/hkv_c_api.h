@@ -166,10 +166,10 @@ int hkv_table_destroy(hkv_table* t);
 /* unique_key (here and below): 1 = the caller guarantees that no key occurs twice in the
  * batch; 0 = keys may repeat: one occurrence per key is taken (found with a device index of
  * the batch), as the reference's kernels for such batches leave every key in the table once.
- * The index stays with the table for the next call, up to 2^21 keys (72 MB at the most): table
- * memory, given back by hkv_table_destroy.  Longer batches, calls that are being recorded into
- * a graph and tables without api_lock or with io_by_cpu take temporary memory from the
- * stream's pool instead.  A dual-bucket table needs 1 (merlin_hashtable.cuh:1167-1169).
+ * The index stays with the table for the next call, up to 2^21 keys (72 MB at the most) and no
+ * more keys than the table has slots: table memory, given back by hkv_table_destroy.  Longer
+ * batches, calls that are being recorded into a graph and tables without api_lock or with
+ * io_by_cpu take temporary memory from the stream's pool instead.  A dual-bucket table needs 1 (merlin_hashtable.cuh:1167-1169).
  *
  * HashTable::insert_or_assign, merlin_hashtable.cuh:1125-1305.  On a table with rows in host
  * memory and with unique_key = 1 (the reference's lock-key and write kernels, upsert.cuh:1350-1595)

@@ -104,6 +104,10 @@ static void kept_or_not() {
   CHECK(index_for(5, 0, kept, own) == &own && blocks == 2);
   repeat_index_free(own, StreamMemory(), nullptr);
   repeat_index_free(kept, StreamMemory(), nullptr);
+  CHECK(index_for(10, 384, kept, own) == &kept && kept.keys == 384); /* no more than may be kept */
+  CHECK(index_for(385, 384, kept, own) == &own);
+  repeat_index_free(own, StreamMemory(), nullptr);
+  repeat_index_free(kept, StreamMemory(), nullptr);
   CHECK(blocks == 0);
 }
 

@@ -64,8 +64,8 @@ def pool_bytes():
     return used.value
 
 
-def repeated_calls(t, sizes):
-    universe = w.unique_keys(71, 0, 1000)
+def repeated_calls(t, sizes, ids=1000):
+    universe = w.unique_keys(71, 0, ids)
     rng = np.random.default_rng(5)
     for n in sizes:
         keys = universe[rng.integers(0, len(universe), n)]
@@ -110,3 +110,16 @@ def test_calls_go_on_where_the_allocator_has_no_room_for_the_index():
     assert len(c.out) == blocks + 1
     t.close()
     assert not c.out
+
+
+def test_a_small_table_keeps_a_small_index():
+    for slots in (1 << 10, 3 << 9):
+        c = Counting()
+        t = c.table(init_capacity=slots, max_capacity=slots, max_hbm_for_vectors=1 << 30, dim=4)
+        slots, table_bytes, before = t.capacity(), c.device_bytes(), pool_bytes()
+        for n in (60000, 30, slots, 500, slots + 1):
+            repeated_calls(t, (n,), ids=200)  # (far from filling a bucket)
+            assert c.device_bytes() <= table_bytes + 68 * slots and pool_bytes() == before
+        assert c.device_bytes() > table_bytes
+        t.close()
+        assert not c.out

@@ -161,7 +161,8 @@ __device__ __forceinline__ void export_rows_any(const hkv_table_view& v, uint64_
  * reserved and for which pred(key, score, pattern, threshold) holds.  `values` and
  * `scores` may be null.
  */
-template <class Pred, int THREADS>
+constexpr int kExportThreads = 256; /* of a launch that does not say */
+template <class Pred, int THREADS = kExportThreads>
 __global__ void __launch_bounds__(THREADS)
 export_if_kernel(hkv_table_view v, Pred pred, uint64_t pattern,
                  uint64_t threshold, uint64_t offset, uint64_t n,
@@ -457,7 +458,7 @@ inline void launch_export(const hkv_table_view& v, Pred pred, uint64_t pattern, 
   if (n >= kExportWide && v.value_bytes <= (1u << 18))
     launch_export_by<Pred, 512>(v, pred, pattern, threshold, offset, n, counter, keys, values, scores, s);
   else
-    launch_export_by<Pred, 256>(v, pred, pattern, threshold, offset, n, counter, keys, values, scores, s);
+    launch_export_by<Pred, kExportThreads>(v, pred, pattern, threshold, offset, n, counter, keys, values, scores, s);
 }
 inline unsigned scan_grid(uint64_t slots, int threads) {
   const uint64_t blocks = (slots + threads - 1) / threads;

@@ -294,6 +294,8 @@ struct PredAlways {
     return true;
   }
 };
+template <>
+constexpr bool kMatchesAll<PredAlways> = true;
 struct PredScoreLt {
   __device__ __forceinline__ bool operator()(const uint64_t&, uint64_t& s,
                                              const uint64_t&, const uint64_t& th) const {

@@ -436,12 +436,23 @@ inline unsigned export_grid(uint64_t n, int threads) {
 /* Every workgroup that has a match claims its part of the output, and the claims are served one at a time: 2048 of them
  * (2^22 slots) queue for 30 us where reading the slots takes 13.  512 threads claim for 4096 slots at once; 1024 leave
  * no more than one workgroup on a CU, whose steps nothing else covers.  Below 2^20 slots they would not reach every CU.
- * us per call with 256 / 512 / 1024 threads, share of the slots that match:
- *                          none                 2 %                  18 %                   75 %
- *   2^18 slots, 256 B      11.3 / 11.6 / 11.5   10.8 / 11.3 / 11.8   12.3 /  13.2 /  17.8   39.5 /  45.9 /  73.0
- *   2^20 slots, 256 B      10.9 / 11.1 / 11.4   12.7 / 11.3 / 11.4   24.1 /  22.0 /  26.8   93.3 /  93.5 / 105.6
- *   2^22 slots,  64 B      13.2 / 13.3 / 14.7   33.6 / 22.4 / 20.8   40.0 /  33.2 /  35.7    101 /    98 /   110
- *   2^24 slots,  64 B      39.4 / 39.5 / 46.1    113 /   67 /   62    128 /   108 /   121    406 /   401 /   428 */
+ * Where most slots match the claims hide behind the rows, and half as many workgroups with 16 instead of 20
+ * wavefronts on a CU are what counts: so not where everything matches, nor for rows that gain only where next to nothing does.
+ * us per call with 256 / 512 threads, share of the slots that match, with keys and rows, and with scores in the last column:
+ *                          none              2 %             18 %            50 %            75 %            90 %            all + scores
+ *   2^20 slots,  64 B   10.0 / 10.1     12.0 / 11.0     15.9 / 13.5     26.7 / 24.6     34.0 / 32.4     38.1 / 37.0       43.1 /   41.3
+ *   2^20 slots, 256 B    9.6 /  9.7     13.1 / 11.1     29.2 / 27.1     64.7 / 63.4     92.9 / 94.4      108 / 111         119 /    116
+ *   2^20 slots, 512 B    9.9 / 10.2     15.4 / 13.4     49.9 / 47.6      124 / 114       176 / 180       208 / 213         217 /    216
+ *   2^20 slots,  1 KB   10.2 / 10.4     19.4 / 17.3     89.0 / 87.4      229 / 219       346 / 343       411 / 415         411 /    423
+ *   2^22 slots,  64 B   13.4 / 13.3     34.4 / 23.6     43.4 / 38.1     77.4 / 74.4      104 / 102       119 / 119         130 /    135
+ *   2^22 slots, 128 B   14.0 / 14.2     35.2 / 24.7     56.1 / 50.7      119 / 116       171 / 174       202 / 205         230 /    236
+ *   2^22 slots, 256 B   14.2 / 14.5     36.0 / 26.2     92.5 / 87.2      228 / 228       336 / 341       395 / 409         434 /    436
+ *   2^22 slots,  1 KB   14.3 / 14.5     54.6 / 46.3      326 / 325       876 / 873      1311 / 1330     1579 / 1612       1678 /   1720
+ *   2^24 slots,  64 B   42.0 / 41.6      115 / 70        140 / 132       306 / 296       425 / 421       491 / 492         543 /    553
+ * (2^20 slots of 4 KB: 8 % 168 / 170, all 1658 / 1764; export_batch of a full table of 2^22 slots of 128 bytes 248 / 258.) */
+template <class Pred>
+constexpr bool kMatchesAll = false;
+constexpr uint32_t kExportWideRow = 512;
 constexpr uint64_t kExportWide = UINT64_C(1) << 20;
 template <class Pred, int THREADS>
 inline void launch_export_by(const hkv_table_view& v, Pred pred, uint64_t pattern, uint64_t threshold, uint64_t offset,
@@ -454,11 +465,13 @@ template <class Pred>
 inline void launch_export(const hkv_table_view& v, Pred pred, uint64_t pattern, uint64_t threshold, uint64_t offset,
                           uint64_t n, unsigned long long* counter, uint64_t* keys, uint8_t* values, uint64_t* scores,
                           hipStream_t s) {
-  /* (the units of a chunk's rows are counted in 32 bits: 4096 rows of up to 2^18 bytes) */
-  if (n >= kExportWide && v.value_bytes <= (1u << 18))
-    launch_export_by<Pred, 512>(v, pred, pattern, threshold, offset, n, counter, keys, values, scores, s);
-  else
-    launch_export_by<Pred, kExportThreads>(v, pred, pattern, threshold, offset, n, counter, keys, values, scores, s);
+  if constexpr (!kMatchesAll<Pred>) {
+    if (n >= kExportWide && v.value_bytes <= kExportWideRow) {
+      launch_export_by<Pred, 512>(v, pred, pattern, threshold, offset, n, counter, keys, values, scores, s);
+      return;
+    }
+  }
+  launch_export_by<Pred, kExportThreads>(v, pred, pattern, threshold, offset, n, counter, keys, values, scores, s);
 }
 inline unsigned scan_grid(uint64_t slots, int threads) {
   const uint64_t blocks = (slots + threads - 1) / threads;

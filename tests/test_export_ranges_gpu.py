@@ -27,7 +27,8 @@ def export(t, dim, n, offset, threshold=None, scores=True):
     return keys[:m][order], rows[:m][order], out[:m][order] if scores else None
 
 
-@pytest.mark.parametrize("dim", [16, 3, 65])
+# (rows of more than 512 bytes keep the smaller part)
+@pytest.mark.parametrize("dim", [16, 3, 65, 128, 129])
 def test_export_ranges(dim):
     t = HashTable()
     t.init(default_options(init_capacity=CAPACITY, max_capacity=CAPACITY, max_hbm_for_vectors=1 << 34, dim=dim,

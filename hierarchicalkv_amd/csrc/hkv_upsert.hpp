@@ -662,27 +662,34 @@ __device__ __forceinline__ void settle_reprobes(const View& v, uint64_t key, uin
  * the plain scan would pick and wait for without end.  Whether a key is
  * refused at score == min is a separate switch (UpsertArgs::refuse_equal).
  */
+/* Wavefronts per SIMD that the compiler has to leave registers for.  Five (96 registers) where nothing is spilled for it: with
+ * two keys per tile and rows of up to 256 bytes insert_or_assign and find_or_insert come to 97 by themselves, one more
+ * than five wavefronts can have.  insert_or_assign and find, half of the keys new, rows of 128 bytes, 260 000 keys
+ * 102 -> 98 us, 2^17 of 64 bytes 60.6 -> 59.3; find_or_insert, accum_or_assign and find, 260 000 keys of 128 bytes
+ * 149.4 -> 145.5, of 256 bytes 182.0 -> 176.5.  With more rows per trip or held slots, and in accum_or_assign, 2 to 18
+ * registers go to memory: 2^17 keys of 512 bytes 151.8 -> 161.7, accum_or_assign of 256 bytes 104 -> 107.
+ * MANY: the launch has more wavefronts than four per SIMD (launch_by_size); below that the order that the compiler
+ * finds for 97 registers is the better one. */
+template <int OP, int UPL, bool BOUNDS, bool HOLD, int R>
+constexpr bool fits_five_waves() {
+  return BOUNDS && R == 2 && UPL <= 2 && !HOLD && (OP == kOpInsertOrAssign || OP == kOpFindOrInsert);
+}
+template <int OP, int UPL, bool BOUNDS, bool HOLD, int R, bool MANY>
+constexpr int upsert_waves() {
+  if (BOUNDS && R == kTile) return 4;
+  return MANY && fits_five_waves<OP, UPL, BOUNDS, HOLD, R>() ? 5 : 1;
+}
+
 /* WAVES wavefronts per workgroup, each with its own 8 R keys and its own staging area.  One
  * everywhere except insert_and_evict on a table that is about full, where two or four wavefronts
  * claim their part of the evicted-keys output together: updates of one word are served one at a time, about
  * 15 ns each, and one per wavefront and trip (some 24 thousand for 2^20 keys into full buckets)
  * took 0.07 ms of the call's 0.46.  (While buckets have free slots there is nothing to claim,
  * and two wavefronts that wait for each other in every trip are 4 % slower than one.) */
-/* Wavefronts per SIMD that the compiler has to leave registers for.  Five (96 registers) where nothing is spilled for it: with
- * two keys per tile and rows of up to 256 bytes insert_or_assign and find_or_insert come to 97 by themselves, one more
- * than five wavefronts can have.  insert_or_assign and find, half of the keys new, rows of 128 bytes, 260 000 keys
- * 102 -> 98 us, 2^17 of 64 bytes 60.6 -> 59.3; find_or_insert, accum_or_assign and find, 260 000 keys of 128 bytes
- * 149.4 -> 145.5, of 256 bytes 182.0 -> 176.5.  With more rows per trip or held slots, and in accum_or_assign, 2 to 18
- * registers go to memory: 2^17 keys of 512 bytes 151.8 -> 161.7, accum_or_assign of 256 bytes 104 -> 107. */
-template <int OP, int UPL, bool BOUNDS, bool HOLD, int R>
-constexpr int upsert_waves() {
-  if (BOUNDS && R == kTile) return 4;
-  return BOUNDS && R == 2 && UPL <= 2 && !HOLD && (OP == kOpInsertOrAssign || OP == kOpFindOrInsert) ? 5 : 1;
-}
-
-template <int OP, int VEC, int UPL, bool LOCKED_RULE, bool BOUNDS = false, int WAVES = 1, bool HOLD = false, int R = kTile>
+template <int OP, int VEC, int UPL, bool LOCKED_RULE, bool BOUNDS = false, int WAVES = 1, bool HOLD = false, int R = kTile,
+          bool MANY = false>
 __global__ void __launch_bounds__(kWave * WAVES)
-    __attribute__((amdgpu_waves_per_eu(upsert_waves<OP, UPL, BOUNDS, HOLD, R>())))
+    __attribute__((amdgpu_waves_per_eu(upsert_waves<OP, UPL, BOUNDS, HOLD, R, MANY>())))
 upsert_kernel(View v, UpsertArgs a) {
   static_assert(!(BOUNDS && LOCKED_RULE), "the bounded search does not look at key words");
   static_assert(WAVES == 1 || OP == kOpInsertAndEvict, "only insert_and_evict has anything to share");

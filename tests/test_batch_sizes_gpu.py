@@ -23,6 +23,10 @@ def bytes_of(a):
     (True, 14, 10, (1, 9, 65, 1000)),
     (True, 18, 8, (1, 7, 8, 9, 16, 17, 65, 1 << 15, (1 << 15) + 1)),
     (True, 21, 8, (1 << 18, (1 << 18) + 1)),
+    # up to 2^16 keys two per tile are at most four wavefronts per SIMD, above that more; rows of 12 and 256 bytes, and longer ones
+    (True, 19, 3, (1 << 16, (1 << 16) + 1)),
+    (True, 19, 64, (1 << 16, (1 << 16) + 1)),
+    (True, 19, 65, (1 << 16, (1 << 16) + 1)),
     (False, 18, 8, (1, 8, 9, 17, 1 << 14, (1 << 14) + 1)),
     (False, 21, 8, (1 << 17, (1 << 17) + 1)),
 ])

@@ -86,7 +86,9 @@ void launch_upsert_for(bool pair, int vec, const View& v, const UpsertArgs& a, h
  * table that only has been offered nine tenths of its slots for instance, is less (accum_or_assign of keys
  * that are all there or change nothing: 35 / 41).  A batch that came with repeated ids (`repeats`) has many of
  * its keys crossed off and takes eight above 2^17: 2^18 keys 133 / 147 / 156 with the passes over the ids (three launches
- * per call then, one now: 116 with eight).
+ * per call then, one now: 116 with eight).  Not so the pointer overload, which moves no rows: eight are better for it where
+ * most ids repeat or are found (200 000 Zipf ids 36 / 43), and far worse where few do (140 000 uniform ones, most of
+ * them new to a full table, 150 / 107).
  * Two keys per tile in more wavefronts than four per SIMD (256 CUs, 1024 SIMDs: 2^16 keys) take the instance that leaves room
  * for a fifth, others the one that does not have to.  insert_or_assign, half of the keys new, us with four / five:
  *                        34 000         60 000         2^16           68 000         80 000         100 000
@@ -99,7 +101,7 @@ void launch_by_size(bool pair, bool repeats, int vec, const View& v, const Upser
     launch_upsert_for<OP, false, BOUNDS, 1>(pair, vec, v, a, s);
   else if (a.n <= kFourWaves)
     launch_upsert_for<OP, false, BOUNDS, 2>(pair, vec, v, a, s);
-  else if (a.n <= (UINT64_C(1) << (BOUNDS && !repeats ? 18 : 17)))
+  else if (a.n <= (UINT64_C(1) << (BOUNDS && !(repeats && OP != kOpFindOrInsertPtr) ? 18 : 17)))
     launch_upsert_for<OP, false, BOUNDS, 2, true>(pair, vec, v, a, s);
   else
     launch_upsert_for<OP, false, BOUNDS, kTile>(pair, vec, v, a, s);

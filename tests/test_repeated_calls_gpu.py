@@ -135,3 +135,50 @@ def test_recorded_calls_beside_eager_ones():
         check_table(t, model, universe, cap)
     torch.cuda.synchronize()
     t.close()
+
+
+def check_evict(t, model, universe, n, rng):
+    """insert_and_evict where nothing has to leave: the first occurrence's row stays."""
+    pick = rng.integers(0, len(universe), n)
+    seen, first = np.unique(pick, return_index=True)
+    rows = rng.integers(0, 256, (n, VB), dtype=np.uint8)
+    ek = torch.full((n,), -1, dtype=torch.int64, device=DEV)
+    ev = torch.full((n, VB), 0xA5, dtype=torch.uint8, device=DEV)
+    es = torch.full((n,), -1, dtype=torch.int64, device=DEV)
+    assert t.insert_and_evict(n, dev(universe[pick]), dev(rows), None, ek, ev, es, unique_key=False) == 0
+    assert bool((ek == -1).all()) and bool((ev == 0xA5).all()) and bool((es == -1).all())
+    model[0][seen], model[1][seen] = True, rows[first]
+
+
+def check_ptr(t, model, universe, n, rng):
+    """find_or_insert by pointer: every occurrence gets the slot's row address, and whether the key was there before."""
+    pick = rng.integers(0, len(universe), n)
+    keys = dev(universe[pick])
+    ptrs, want = (torch.zeros(n, dtype=torch.int64, device=DEV) for _ in range(2))
+    founds, found_now = (torch.zeros(n, dtype=torch.bool, device=DEV) for _ in range(2))
+    t.find_or_insert_ptr(n, keys, ptrs, founds, unique_key=False)
+    t.find_ptr(n, keys, want, found_now)
+    torch.cuda.synchronize()
+    assert bool(found_now.all()) and torch.equal(ptrs, want)
+    assert (founds.cpu().numpy() == model[0][pick]).all()
+    model[0][pick] = True
+    # the rows of keys that came in this way are the caller's to write
+    rows = rng.integers(0, 256, (len(universe), VB), dtype=np.uint8)
+    t.assign(n, keys, dev(rows[pick]), unique_key=False)
+    model[1][pick] = rows[pick]
+    torch.cuda.synchronize()
+
+
+# sizes on both sides of those where the keys per tile and the workgroups change (2^15, 2^16, 2^17, 2^18)
+@pytest.mark.parametrize("cap", [1 << 17, 1 << 20])
+def test_every_call_that_takes_repeated_keys(cap):
+    t = make(cap)
+    rng = np.random.default_rng(cap)
+    universe = w.unique_keys(55, 0, 40000)
+    model = np.zeros(len(universe), bool), np.zeros((len(universe), VB), np.uint8)
+    for n in (2, 300, (1 << 15) - 1, (1 << 15) + 1, (1 << 16) + 1, (1 << 17) - 1, (1 << 17) + 1, 1 << 18, (1 << 18) + 1, 77):
+        check_ptr(t, model, universe, n, rng)
+        check_evict(t, model, universe, n, rng)
+        check_call(t, model, universe, n, rng)
+        check_table(t, model, universe, cap)
+    t.close()

@@ -1,5 +1,7 @@
 """Batches that repeat keys, call after call on one table: the index of the batch's keys is the
 table's and is not cleared between calls.  Expected values are worked out here with numpy."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -181,4 +183,91 @@ def test_every_call_that_takes_repeated_keys(cap):
         check_evict(t, model, universe, n, rng)
         check_call(t, model, universe, n, rng)
         check_table(t, model, universe, cap)
+    t.close()
+
+
+def planned_calls(universe, model, sizes, rng):
+    """Alternating find_or_insert and insert_or_assign with repeated keys: per call the keys, the rows and what has to be in the
+    rows afterwards, on the device and on the host."""
+    present, stored = model
+    plan = []
+    for k, n in enumerate(sizes):
+        pick = rng.integers(0, len(universe), n)
+        seen, first = np.unique(pick, return_index=True)
+        rows = rng.integers(0, 256, (n, VB), dtype=np.uint8)
+        stand = np.empty(len(universe), np.int64)
+        stand[seen] = first
+        want = rows
+        if k % 2 == 0:
+            want = np.where(present[pick][:, None], stored[pick], rows[stand[pick]])
+            new = ~present[seen]
+            stored[seen[new]] = rows[first[new]]
+        else:
+            stored[seen] = rows[first]
+        present[seen] = True
+        plan.append((n, dev(universe[pick]), dev(rows), want))
+    return plan
+
+
+def issue(t, k, call, stream):
+    n, keys, rows, _ = call
+    (t.find_or_insert if k % 2 == 0 else t.insert_or_assign)(n, keys, rows, unique_key=False, stream=stream)
+
+
+def check_plan(plan):
+    for k, (n, _, rows, want) in enumerate(plan):
+        assert (rows.cpu().numpy() == want).all(), (k, n)
+
+
+# the index grows, and is used by the next stream, while the calls of the one before are under way
+def test_streams_share_the_index_without_waiting():
+    cap = 1 << 19
+    t = make(cap)
+    rng = np.random.default_rng(12)
+    universe = w.unique_keys(56, 0, 50000)
+    model = np.zeros(len(universe), bool), np.zeros((len(universe), VB), np.uint8)
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    sizes = [5000, 300, 70000, 4000, 150000, 2, 1 << 15, 300000, 300, 200000, 90000, 1000, 300000, 65, 40000, 250000] * 2
+    plan = planned_calls(universe, model, sizes, rng)
+    torch.cuda.synchronize()
+    for k, call in enumerate(plan):  # one after the other on the host, so the group lock orders them in this order
+        issue(t, k, call, streams[k % 3])
+    torch.cuda.synchronize()
+    check_plan(plan)
+    check_table(t, model, universe, cap)
+    t.close()
+
+
+def test_host_threads_share_the_index():
+    cap, threads = 1 << 19, 4
+    t = make(cap)
+    errors, work = [], []
+    for tid in range(threads):
+        universe = w.unique_keys(57 + tid, 0, 15000)
+        model = np.zeros(len(universe), bool), np.zeros((len(universe), VB), np.uint8)
+        sizes = [(1 << (6 + (3 * k + tid) % 13)) + k for k in range(40)]
+        work.append((universe, model, planned_calls(universe, model, sizes, np.random.default_rng(tid))))
+    torch.cuda.synchronize()
+
+    def worker(tid):
+        try:
+            torch.cuda.set_device(0)
+            s = torch.cuda.Stream()
+            for k, call in enumerate(work[tid][2]):
+                issue(t, k, call, s)
+            s.synchronize()
+        except BaseException as e:  # noqa: BLE001 - reported by the main thread
+            errors.append((tid, repr(e)))
+
+    running = [threading.Thread(target=worker, args=(i,)) for i in range(threads)]
+    for th in running:
+        th.start()
+    for th in running:
+        th.join()
+    assert not errors, errors
+    torch.cuda.synchronize()
+    for _, _, plan in work:
+        check_plan(plan)
+    universe = np.concatenate([u for u, _, _ in work])
+    check_table(t, (np.concatenate([m[0] for _, m, _ in work]), np.concatenate([m[1] for _, m, _ in work])), universe, cap)
     t.close()

@@ -85,7 +85,7 @@ struct UpsertArgs {
    * its line itself.  Null where scores only grow (LRU, EpochLRU). */
   unsigned long long* bound_ceil;
   /* a batch that may repeat keys (hkv_dedup.hpp): the index of its keys, and per key where in the index its entry is;
-   * the kernel leaves the occurrence that stands for the key there.  Null: keys are unique */
+   * find_or_insert leaves the occurrence that stands for the key there.  Null: keys are unique */
   const uint64_t* repeat_index;
   uint32_t* repeat_of;
 };
@@ -737,7 +737,7 @@ upsert_kernel(View v, UpsertArgs a) {
   uint64_t staged = a.n; /* keys up to this one count */
   if (OP != kOpAccumOrAssign && a.repeat_of && i < a.n) {
     const uint32_t first = (uint32_t)a.repeat_index[a.repeat_of[i]];
-    a.repeat_of[i] = first;
+    if (OP == kOpFindOrInsert || OP == kOpFindOrInsertPtr) a.repeat_of[i] = first; /* (the others hand nothing back per key) */
     if (first != (uint32_t)i) staged = 0; /* another occurrence stands for the key */
   }
   const uint64_t key = stage_keys(v, a.keys, staged, i, s_meta, s_slot, lane);

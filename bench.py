@@ -769,7 +769,7 @@ CONFIG_PROFILES = [
     ("cfg5", "python3 bench.py --config 5", "configuration 5 (capacity 2^25, dim 128, EpochLRU, load factor 1.0)",
      [("upsert_kernel<3, 16, 4, false", "accum_or_assign (70 % existing)", "last3"),
       ("export_if_kernel", "export_batch_if over the whole table (8 windows)", "sum8"),
-      ("erase_kernel<true>", "erase (2^18 keys)", "last3")]),
+      ("erase_kernel<true", "erase (2^18 keys)", "last3")]),
 ]
 CONFIG_GROUPS = ["trace", "fetch", "write", "wr", "tcp"]
 

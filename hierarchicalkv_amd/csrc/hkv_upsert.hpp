@@ -1078,10 +1078,10 @@ upsert_kernel(View v, UpsertArgs a) {
         __hip_atomic_fetch_min(v.bounds + (slot >> 4), stored, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     /* The rows of a trip, where they fit into 32 registers, are on their way while the claim is: the victim's after the
-     * claim and the caller's after the victim's made two round trips more.  insert_and_evict with what a cache does around
-     * it, rows of 128 bytes: 30 000 keys 65.5 -> 64.5 us, 2^17 97.2 -> 95.4; of 256 bytes, 2^17 116.3 -> 113.4; of
-     * 400 bytes, 30 000 keys (one per tile) 92.0 -> 89.6; 400 000 keys, which take the other way, the same.  (Half the
-     * registers: 96, 116.3, 93.) */
+     * claim and the caller's after the victim's made two round trips more.  insert_and_evict and its count, half of the
+     * keys new, rows of 128 bytes: 30 000 keys 51.6 -> 50.4 us, 60 000 61.2 -> 60.6, 2^17 89.4 -> 87.8; of 256 bytes 54.6 ->
+     * 53.2, 67.0 -> 66.1, 100.3 -> 97.8; of 400 bytes 30 000 keys (one per tile) 63.6 -> 63.0; the other way of larger batches and
+     * rows is as it was.  What a trip waits for is mostly the claim.  (With half the registers there was no gain at 256 bytes.) */
     constexpr bool kAhead = OP == kOpInsertAndEvict && R * UPL <= 4;
     if constexpr (kAhead) {
       typename VecType<VEC>::type out[R][UPL], in[R][UPL];
